@@ -407,68 +407,70 @@ struct ValueBlockArgs {
 };
 
 // 64 tokens of one (b, h) per workgroup.  Four threads per token compute the
-// norm in the reference's pairwise order and stage the normalised row in LDS;
-// then the rotation as in the group encode (DPP row broadcasts of register-
-// held row slices, a column of Pi_T per lane).
+// norm in the reference's pairwise order and stage the scaled row as fp16
+// pairs; then every wave estimates the codes of its channels on the matrix
+// cores, the flagged ones are recomputed, and the bit streams written.
 template <int VB, int D>
 __global__ __launch_bounds__(kVbThreads) void tqk_value_block(ValueBlockArgs a) {
-  constexpr int VROW = D * VB / 8;
+  constexpr int VROW = D * VB / 8, NT = D / 16 > kVbThreads / 64 ? 2 : 1;
   const tqk_block_desc& d = a.d;
   const int S = d.tokens, bh = blockIdx.y, t0 = blockIdx.x * kVbTokens, tid = threadIdx.x;
+  const int lane = tid & 63, wv = tid >> 6;
   const int nb = min(kVbTokens, S - t0);
   const size_t tok0 = (size_t)bh * S + t0;  // flat token index of the first token
-  __shared__ __align__(16) float u_s[kVbTokens][D];
-  __shared__ uint8_t vc_s[kVbTokens][D];
+  __shared__ __align__(16) uint16_t uv_s[kVbTokens][2 * D + 8];
+  __shared__ __align__(16) PolarStage<D, kVbTokens> st;
 
+  if (tid == 0) st.nlist = 0;
   {
     const int tt = tid >> 2, q = tid & 3;
     if (tt < nb) {
       const size_t row = (tok0 + tt) * D;
       float x0[D / 8], x1[D / 8];
+      uint32_t any = 0;
 #pragma unroll
       for (int m = 0; m < D / 8; ++m) {  // channels 8m + 2q, 8m + 2q + 1
         x0[m] = load_x(a.x, d.input_f32, row + 8 * m + 2 * q);
         x1[m] = load_x(a.x, d.input_f32, row + 8 * m + 2 * q + 1);
+        any |= __float_as_uint(x0[m]) | __float_as_uint(x1[m]);
       }
+      any |= __shfl_xor(any, 1, 4);
+      any |= __shfl_xor(any, 2, 4);
       const float ss = pairwise_sumsq<D>(x0, x1, q);
       const float nrm = __builtin_sqrtf(ss);  // correctly rounded (-fhip-fp32-correctly-rounded-divide-sqrt)
-      const float safe = fmaxf(nrm, 1e-30f);
-#pragma unroll
-      for (int m = 0; m < D / 8; ++m) {
-        u_s[tt][8 * m + 2 * q] = __fdiv_rn(x0[m], safe);
-        u_s[tt][8 * m + 2 * q + 1] = __fdiv_rn(x1[m], safe);
+      const bool zero = (any & 0x7FFFFFFFu) == 0u;
+      polar_stage_row<D>(&uv_s[tt][0], x0, x1, q, zero ? 0.f : kPiScale * __builtin_amdgcn_rcpf(nrm));
+      if (q == 0) {
+        polar_token(st, tt, ss, nrm, zero, 1.0f / (kPiScale * kPiScale));
+        a.norms[tok0 + tt] = nrm;
       }
-      if (q == 0) a.norms[tok0 + tt] = nrm;
     }
   }
-  // rotation: wave w owns the rotated channels [16w + 128p, +16) of pass p,
-  // lane l column e = 16w + 128p + (l & 15) of Pi_T (row e of Pi) in
-  // registers; each 16-lane row takes one token of a 4-token step, holds
-  // eight channels of its normalised row and broadcasts them to the row by
-  // DPP (rotate_codes, no LDS broadcast reads)
-  const int lane = tid & 63, wv = tid >> 6;
   float bnd[15];
 #pragma unroll
-  for (int k = 0; k < (1 << VB) - 1; ++k) bnd[k] = a.vbnd[k];
+  for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.vbnd[k] : 0.f;
   __syncthreads();
-  for (int e0 = 16 * wv; e0 < D; e0 += 16 * (kVbThreads / 64))
-    rotate_codes<D, VB>(a.pi, u_s, nb, e0 + (lane & 15), lane, bnd, vc_s);
+  const int e0 = 16 * NT * wv;
+  if (e0 < D) {
+    PiFrags<D, NT> pf;
+    load_pi(pf, a.pi, e0, lane, bnd, (1 << VB) - 1);
+    polar_codes<D, NT, VB, true, false>(st, pf, &uv_s[0][0], 2 * D + 8, nb, e0, lane, bnd);
+  }
   __syncthreads();
-  // the reference's little-endian bit stream, one token per thread
-  if (tid < nb) {
-    uint32_t outw[VROW / 4];
+  if (st.nlist > 0) {
+    polar_fix<D, VB, false, kVbThreads>(st, a.pi, nb, tid, bnd, [&](int t, int dd) {
+      const size_t i = (tok0 + t) * D + dd;
+      return make_float4(load_x(a.x, d.input_f32, i), load_x(a.x, d.input_f32, i + 1),
+                         load_x(a.x, d.input_f32, i + 2), load_x(a.x, d.input_f32, i + 3));
+    });
+    __syncthreads();
+  }
+  for (int f8 = tid; f8 < nb * (D / 32); f8 += kVbThreads) {
+    uint32_t w[VB];
+    pack_fields<VB>(st, f8, w);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(a.packed + (tok0 + f8 / (D / 32)) * VROW) + VB * (f8 % (D / 32));
 #pragma unroll
-    for (int k = 0; k < VROW / 4; ++k) outw[k] = 0u;
-#pragma unroll
-    for (int e = 0; e < D; ++e) {
-      const uint32_t code = vc_s[tid][e];
-      const int bitpos = e * VB;
-      outw[bitpos >> 5] |= code << (bitpos & 31);
-      if ((bitpos & 31) + VB > 32) outw[(bitpos >> 5) + 1] |= code >> (32 - (bitpos & 31));
-    }
-    uint32_t* dst = reinterpret_cast<uint32_t*>(a.packed + (tok0 + tid) * VROW);
-#pragma unroll
-    for (int k = 0; k < VROW / 4; ++k) dst[k] = outw[k];
+    for (int k = 0; k < VB; ++k) dst[k] = w[k];
   }
 }
 

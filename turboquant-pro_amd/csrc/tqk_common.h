@@ -113,108 +113,297 @@ __device__ __forceinline__ float dpp_row_bcast(float x) {
   return __builtin_bit_cast(
       float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + I, 0xF, 0xF, true));
 }
-
-// y0 += u_a[d] * pcol[d], y1 += u_b[d] * pcol[d] for d = 8K .. 8K + 7 and on
-// to d = 8 NL - 1, each product and sum separately rounded, in d order; u_a[d]
-// lives in register d % 8 of lane d / 8 of the 16-lane row (NL <= 16 lanes
-// hold a chunk of 8 NL channels).  Plain operators, so that the broadcast
-// folds into the multiply as its DPP source operand: only for units built
-// with -ffp-contract=off (the encode and the block quantizers), where a
-// product and a sum are never fused.
-template <int K, int NL, int N>
-__device__ __forceinline__ void rotate_row_dpp(float& y0, float& y1, const float (&ua)[8],
-                                               const float (&ub)[8], const float (&pcol)[N]) {
-  static_assert(NL <= 16 && 8 * NL <= N, "a chunk spans at most one 16-lane row");
+// y += the eight values of lane K of the 16-lane row, in order, then those of
+// the lanes after it up to NL - 1 (plain operators, so that the broadcast
+// folds into the addition; every lane of the row gets the sum)
+template <int K, int NL>
+__device__ __forceinline__ void add_row_dpp(float& y, const float (&f)[8]) {
 #pragma unroll
-  for (int r = 0; r < 8; ++r) {
-    const float p0 = dpp_row_bcast<K>(ua[r]) * pcol[8 * K + r];
-    const float p1 = dpp_row_bcast<K>(ub[r]) * pcol[8 * K + r];
-    y0 = y0 + p0;
-    y1 = y1 + p1;
-  }
-  if constexpr (K + 1 < NL) rotate_row_dpp<K + 1, NL>(y0, y1, ua, ub, pcol);
+  for (int r = 0; r < 8; ++r) y = y + dpp_row_bcast<K>(f[r]);
+  if constexpr (K + 1 < NL) add_row_dpp<K + 1, NL>(y, f);
 }
 
-// PolarQuant codes of nb <= 64 normalised rows u_s[0..nb) for the rotated
-// channel ecol this lane owns: y_e = sum_d u_d * pi[e][d] (sequential in d,
-// separately rounded, as the reference's einsum), code = #{ boundaries < y_e }
-// (a NaN y_e takes the last code, as searchsorted does), written to
-// vc[j][ecol].  Lane layout: the lane's 16-lane row (rt = lane >> 4) takes
-// tokens j0 + rt and j0 + 4 + rt of each 8-token step; lane li = lane & 15
-// holds eight channels of the row and broadcasts them to its row by DPP.
-// Rows longer than 128 channels go in 128-channel chunks, the column chunk in
-// registers and every step's sums carried from chunk to chunk.  The 64 lanes
-// of the wave must all run it (the broadcasts read other lanes).
-template <int D, int VB>
-__device__ __forceinline__ void rotate_codes(const float* __restrict__ pi, const float (*u_s)[D],
-                                             int nb, int ecol, int lane, const float (&bnd)[15],
-                                             uint8_t (*vc)[D]) {
-  constexpr int CH = D < 128 ? D : 128;  // channels per chunk
-  const int rt = lane >> 4, lc = (lane & 15) % (CH / 8);
-  auto load_u = [&](int ja, int jb, int c, float (&ua)[8], float (&ub)[8]) {
-    const float4* ra = reinterpret_cast<const float4*>(&u_s[min(ja, nb - 1)][CH * c + 8 * lc]);
-    const float4* rb = reinterpret_cast<const float4*>(&u_s[min(jb, nb - 1)][CH * c + 8 * lc]);
-    const float4 a0 = ra[0], a1 = ra[1], b0 = rb[0], b1 = rb[1];
-    ua[0] = a0.x; ua[1] = a0.y; ua[2] = a0.z; ua[3] = a0.w;
-    ua[4] = a1.x; ua[5] = a1.y; ua[6] = a1.z; ua[7] = a1.w;
-    ub[0] = b0.x; ub[1] = b0.y; ub[2] = b0.z; ub[3] = b0.w;
-    ub[4] = b1.x; ub[5] = b1.y; ub[6] = b1.z; ub[7] = b1.w;
-  };
-  auto store = [&](int ja, int jb, float y0, float y1) {
-    uint32_t c0 = 0, c1 = 0;
+// ---------------------------------------------------------------------------
+// PolarQuant codes.  The code of a rotated channel is #{ boundaries < y_e } for
+// the reference's y_e: the sum over d, in order, of u_d * pi[e][d], every
+// product and sum separately rounded (a NaN y_e takes the last code, as
+// searchsorted does).  Only the code is stored, so y_e itself is needed only
+// where it lies close to a boundary: the matrix cores give an estimate with a
+// proven error bound, every estimate further than the bound from all
+// boundaries has the reference's code, and the others (about 1 in 700 at 3
+// bits and head_dim 128) are listed and recomputed in the reference's order.
+// (Evaluating the ordered sum everywhere took 256 VALU instructions per channel
+// and bounded the whole encode: 16 sequences x 8192 tokens x 8 heads appended
+// in 1584 us, with the estimate, about 20 instructions, in 868 us.)
+//
+// The estimate: x (fp16 as it is, or the fp32 row scaled to |u| <= 256 and
+// split into an fp16 pair) times 256 * pi split into an fp16 pair, summed in
+// fp32 by MFMA, scaled back by 1 / norm.  Against the real sum
+// sum_d u_d pi[e][d], with |u| <= 1 and N = |pi[e]|:
+//   the ordered sum errs by at most D 2^-24 N            (D roundings)
+//   the MFMA sums by at most (D / 32) 33 2^-23 N         (every one of a step's
+//                            32 products and its sum truncated at full scale)
+//   the dropped low x low products and the pairs' own rounding 3 2^-22 N, the
+//   scaling by 1 / norm 2^-22 N
+// which stays below D 2^-22 N for D = 64, 128 and 256.
+// ---------------------------------------------------------------------------
+typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef float f4_t __attribute__((ext_vector_type(4)));
+
+constexpr float kPiScale = 256.0f;  // fp16 pairs of pi (and of u): far from fp16's subnormals
+
+// The 16 * NT rows of pi from e0 on as MFMA operands (lane: row e0 + 16 nt +
+// lane % 16, channels 32 ks + 8 (lane / 16) .. + 7), and the bound on an
+// estimate's distance from the ordered sum: infinite (every code recomputed)
+// for rows that are not finite or longer than 50, and for boundaries that do
+// not ascend (the code's search needs them to).
+template <int D, int NT>
+struct PiFrags {
+  h8_t hi[D / 32][NT], lo[D / 32][NT];
+  float delta;
+};
+template <int D, int NT, int NB>
+__device__ __forceinline__ void load_pi(PiFrags<D, NT>& f, const float* __restrict__ pi, int e0, int lane,
+                                        const float (&bnd)[NB], int nbnd) {
+  float most = 0.f;
+  bool bad = false;
 #pragma unroll
-    for (int k = 0; k < (1 << VB) - 1; ++k) {
-      c0 += (bnd[k] < y0) ? 1u : 0u;
-      c1 += (bnd[k] < y1) ? 1u : 0u;
-    }
-    if (y0 != y0) c0 = (1u << VB) - 1u;
-    if (y1 != y1) c1 = (1u << VB) - 1u;
-    if (ja < nb) vc[ja][ecol] = (uint8_t)c0;
-    if (jb < nb) vc[jb][ecol] = (uint8_t)c1;
-  };
-  auto load_col = [&](int c, float (&pcol)[CH]) {
+  for (int nt = 0; nt < NT; ++nt) {
+    const float* row = pi + (size_t)(e0 + 16 * nt + (lane & 15)) * D + 8 * (lane >> 4);
+    float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < CH / 4; ++k) {
-      const float4 p4 = reinterpret_cast<const float4*>(pi + (size_t)ecol * D + CH * c)[k];
-      pcol[4 * k] = p4.x;
-      pcol[4 * k + 1] = p4.y;
-      pcol[4 * k + 2] = p4.z;
-      pcol[4 * k + 3] = p4.w;
+    for (int ks = 0; ks < D / 32; ++ks) {
+      const float4 a = *reinterpret_cast<const float4*>(row + 32 * ks);
+      const float4 b = *reinterpret_cast<const float4*>(row + 32 * ks + 4);
+      const float p[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float s = p[i] * kPiScale;
+        const _Float16 h = (_Float16)s;
+        f.hi[ks][nt][i] = h;
+        f.lo[ks][nt][i] = (_Float16)(s - (float)h);
+        ss += p[i] * p[i];
+      }
     }
-  };
-  if constexpr (D <= 128) {
-    float pcol[CH];
-    load_col(0, pcol);
-    for (int j0 = 0; j0 < nb; j0 += 8) {
-      const int ja = j0 + rt, jb = j0 + 4 + rt;
-      float ua[8], ub[8];
-      load_u(ja, jb, 0, ua, ub);
-      float y0 = 0.f, y1 = 0.f;
-      rotate_row_dpp<0, CH / 8>(y0, y1, ua, ub, pcol);
-      // keeps the sums out of the conditional stores: sunk into them, the
-      // multiplies would leave their broadcasts behind as separate moves
-      asm volatile("" : "+v"(y0), "+v"(y1));
-      store(ja, jb, y0, y1);
-    }
+    ss += __shfl_xor(ss, 16, 64);
+    ss += __shfl_xor(ss, 32, 64);
+    bad |= !(ss <= 2500.0f);
+    most = fmaxf(most, ss);
+  }
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) most = fmaxf(most, __shfl_xor(most, o, 64));
+  for (int k = 1; k < nbnd; ++k) bad |= !(bnd[k - 1] < bnd[k]);
+  f.delta = __any(bad) ? __builtin_inff() : 1.01f * (float)D * 0x1p-22f * __builtin_sqrtf(most);
+}
+
+// #{ b < y } by binary search, and the distance m to the nearest boundary:
+// both neighbours of the final interval are on the search's path
+template <int VB>
+__device__ __forceinline__ uint32_t code_margin(float y, const float (&b)[15], float& m) {
+  if constexpr (VB == 2) {
+    const bool c1 = b[1] < y;
+    const float q = c1 ? b[2] : b[0];
+    m = fminf(fabsf(y - b[1]), fabsf(y - q));
+    return (c1 ? 2u : 0u) + (q < y ? 1u : 0u);
+  } else if constexpr (VB == 3) {
+    const bool c1 = b[3] < y;
+    const float p = c1 ? b[5] : b[1], r0 = c1 ? b[4] : b[0], r1 = c1 ? b[6] : b[2];
+    const bool c2 = p < y;
+    const float r = c2 ? r1 : r0;
+    m = fminf(fminf(fabsf(y - b[3]), fabsf(y - p)), fabsf(y - r));
+    return (c1 ? 4u : 0u) + (c2 ? 2u : 0u) + (r < y ? 1u : 0u);
   } else {
-    float ya[8], yb[8];
+    const bool c1 = b[7] < y;
+    float t[7];
 #pragma unroll
-    for (int st = 0; st < 8; ++st) ya[st] = yb[st] = 0.f;
-    for (int c = 0; c < D / CH; ++c) {
-      float pcol[CH];
-      load_col(c, pcol);
+    for (int i = 0; i < 7; ++i) t[i] = c1 ? b[8 + i] : b[i];
+    const bool c2 = t[3] < y;
+    const float p = c2 ? t[5] : t[1], r0 = c2 ? t[4] : t[0], r1 = c2 ? t[6] : t[2];
+    const bool c3 = p < y;
+    const float r = c3 ? r1 : r0;
+    m = fminf(fminf(fabsf(y - b[7]), fabsf(y - t[3])), fminf(fabsf(y - p), fabsf(y - r)));
+    return (c1 ? 8u : 0u) + (c2 ? 4u : 0u) + (c3 ? 2u : 0u) + (r < y ? 1u : 0u);
+  }
+}
+template <int VB>
+__device__ __forceinline__ uint32_t code_exact(float y, const float (&b)[15]) {
+  uint32_t c = 0;
 #pragma unroll
-      for (int st = 0; st < 8; ++st) {
-        if (8 * st < nb) {
-          float ua[8], ub[8];
-          load_u(8 * st + rt, 8 * st + 4 + rt, c, ua, ub);
-          rotate_row_dpp<0, CH / 8>(ya[st], yb[st], ua, ub, pcol);
-          asm volatile("" : "+v"(ya[st]), "+v"(yb[st]));
+  for (int k = 0; k < (1 << VB) - 1; ++k) c += (b[k] < y) ? 1u : 0u;
+  return y != y ? (1u << VB) - 1u : c;
+}
+
+// A batch's staging in LDS.  Codes sit in 16-bit fields of four codes: four
+// tokens of one channel (TROWS, the MFMA-tiled value order: field (t / 4) * D +
+// e) or four channels of one token (field t * (D / 4) + e / 4), in either case
+// the order in which eight consecutive fields' bits make up VB whole dwords of
+// the stored row.
+template <int D, int NTOK>
+struct PolarStage {
+  uint16_t fld[NTOK * D / 4];
+  float2 tk[NTOK];   // (estimate scale, factor of the bound)
+  float nrm[NTOK];
+  uint16_t list[1024];  // flagged codes, t * D + e
+  int nlist;
+};
+
+// The token's entry of the stage from its sum of squares.  Zero rows need no
+// bound (their y is exactly 0, as the estimate); rows whose sum of squares is
+// not finite or so small that u may be longer than 1 get a NaN scale, which
+// flags every code of theirs.
+template <int D, int NTOK>
+__device__ __forceinline__ void polar_token(PolarStage<D, NTOK>& st, int t, float ss, float nrm, bool zero,
+                                            float scale) {
+  st.nrm[t] = nrm;
+  const bool plain = ss >= 0x1p-60f && ss <= 0x1p100f;
+  st.tk[t] = zero ? make_float2(0.f, -1.f)
+                  : make_float2(plain ? scale : __builtin_nanf(""), 1.f);
+}
+
+// Estimated codes of the stage's nb tokens for the wave's 16 * NT channels from
+// e0 on; xs: the tokens' rows, fp16 (hi, and at column D the low halves when
+// LO), `stride` halves apart.  All 64 lanes run it.
+template <int D, int NT, int VB, bool LO, bool TROWS, int NTOK>
+__device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFrags<D, NT>& pf,
+                                            const uint16_t* xs, int stride, int nb, int e0, int lane,
+                                            const float (&bnd)[15]) {
+  const int c16 = lane & 15, lg = lane >> 4;
+  for (int t0 = 0; t0 < nb; t0 += 16) {
+    const uint16_t* row = xs + (size_t)min(t0 + c16, nb - 1) * stride + 8 * lg;
+    f4_t acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) {
+      const h8_t xh = *reinterpret_cast<const h8_t*>(row + 32 * ks);
+      h8_t xl = {};
+      if constexpr (LO) xl = *reinterpret_cast<const h8_t*>(row + D + 32 * ks);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        if constexpr (TROWS) {
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.hi[ks][nt], acc[nt], 0, 0, 0);
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.lo[ks][nt], acc[nt], 0, 0, 0);
+          if constexpr (LO) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, pf.hi[ks][nt], acc[nt], 0, 0, 0);
+        } else {
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xh, acc[nt], 0, 0, 0);
+          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.lo[ks][nt], xh, acc[nt], 0, 0, 0);
+          if constexpr (LO) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xl, acc[nt], 0, 0, 0);
         }
       }
     }
+    // the lane's four results of a tile: tokens t0 + 4 lg + r of channel e0 +
+    // 16 nt + c16 (TROWS), else channels e0 + 16 nt + 4 lg + r of token t0 + c16
+    float2 tk[4];
 #pragma unroll
-    for (int st = 0; st < 8; ++st) store(8 * st + rt, 8 * st + 4 + rt, ya[st], yb[st]);
+    for (int r = 0; r < 4; ++r) tk[r] = st.tk[min(TROWS ? t0 + 4 * lg + r : t0 + c16, nb - 1)];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      uint32_t f = 0;
+      uint32_t near = 0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float y = acc[nt][r] * tk[r].x;
+        float m;
+        f |= code_margin<VB>(y, bnd, m) << (VB * r);
+        near |= (m > tk[r].y * pf.delta) ? 0u : (1u << r);
+      }
+      const int t = TROWS ? t0 + 4 * lg : t0 + c16, e = e0 + 16 * nt + (TROWS ? c16 : 4 * lg);
+      if (t < nb) st.fld[TROWS ? (t >> 2) * D + e : t * (D / 4) + (e >> 2)] = (uint16_t)f;
+      while (near) {
+        const int r = __builtin_ctz(near);
+        near &= near - 1u;
+        const int tt = TROWS ? t + r : t, ee = TROWS ? e : e + r;
+        if (tt < nb) {
+          const int at = atomicAdd(&st.nlist, 1);
+          if (at < 1024) st.list[at] = (uint16_t)(tt * D + ee);
+        }
+      }
+    }
+  }
+}
+
+// code of (token t, channel e) in the stage (other codes of the word may
+// change at the same time)
+template <int D, int VB, bool TROWS, int NTOK>
+__device__ __forceinline__ void set_code(PolarStage<D, NTOK>& st, int t, int e, uint32_t code) {
+  const int idx = TROWS ? (t >> 2) * D + e : t * (D / 4) + (e >> 2);
+  const int sh = 16 * (idx & 1) + VB * (TROWS ? t & 3 : e & 3);
+  uint32_t* w = reinterpret_cast<uint32_t*>(st.fld) + (idx >> 1);
+  const uint32_t old = (*reinterpret_cast<volatile uint32_t*>(w) >> sh) & ((1u << VB) - 1u);
+  if (old != code) atomicXor(w, (old ^ code) << sh);
+}
+
+// The flagged codes in the reference's order; x4(t, d) gives channels d .. d + 3
+// of token t as they came.  A list that overflowed (rows of NaN, infinities or
+// vanishing norms, a rotation that puts whole channels on a boundary) has
+// every code recomputed, a wave per token and a lane per channel.  All NTH
+// threads run it, between barriers.
+template <int D, int VB, bool TROWS, int NTH, int NTOK, typename X4>
+__device__ __forceinline__ void polar_fix(PolarStage<D, NTOK>& st, const float* __restrict__ pi, int nb, int tid,
+                                          const float (&bnd)[15], X4 x4) {
+  const int n = st.nlist;
+  if (n <= 1024) {
+    // sixteen lanes per code: each holds eight products of a 128-channel chunk,
+    // and all add them up in order, one lane's after another (DPP)
+    constexpr int CH = D < 128 ? D : 128;
+    const int li = tid & 15;
+    for (int i0 = 0; i0 < n; i0 += NTH / 16) {
+      const int i = i0 + (tid >> 4), at = st.list[min(i, n - 1)], t = at / D, e = at % D;
+      const float safe = fmaxf(st.nrm[t], 1e-30f);
+      float y = 0.f;
+#pragma unroll
+      for (int c = 0; c < D / CH; ++c) {
+        const int d = CH * c + 8 * (li % (CH / 8));
+        const float4 xa = x4(t, d), xb = x4(t, d + 4);
+        const float4* pr = reinterpret_cast<const float4*>(pi + (size_t)e * D + d);
+        const float4 pa = pr[0], pb = pr[1];
+        const float f[8] = {__fmul_rn(__fdiv_rn(xa.x, safe), pa.x), __fmul_rn(__fdiv_rn(xa.y, safe), pa.y),
+                            __fmul_rn(__fdiv_rn(xa.z, safe), pa.z), __fmul_rn(__fdiv_rn(xa.w, safe), pa.w),
+                            __fmul_rn(__fdiv_rn(xb.x, safe), pb.x), __fmul_rn(__fdiv_rn(xb.y, safe), pb.y),
+                            __fmul_rn(__fdiv_rn(xb.z, safe), pb.z), __fmul_rn(__fdiv_rn(xb.w, safe), pb.w)};
+        add_row_dpp<0, CH / 8>(y, f);
+      }
+      if (i < n && li == 0)  // (a NaN norm makes u, and so y, NaN)
+        set_code<D, VB, TROWS>(st, t, e, code_exact<VB>(st.nrm[t] != st.nrm[t] ? st.nrm[t] : y, bnd));
+    }
+    return;
+  }
+  const int lane = tid & 63;
+  for (int t = tid >> 6; t < nb; t += NTH / 64) {
+    const float safe = fmaxf(st.nrm[t], 1e-30f);
+    float y[D / 64];
+#pragma unroll
+    for (int k = 0; k < D / 64; ++k) y[k] = st.nrm[t] != st.nrm[t] ? st.nrm[t] : 0.f;
+    for (int d = st.nrm[t] != st.nrm[t] ? D : 0; d < D; d += 4) {
+      const float4 x = x4(t, d);
+      const float u[4] = {__fdiv_rn(x.x, safe), __fdiv_rn(x.y, safe), __fdiv_rn(x.z, safe), __fdiv_rn(x.w, safe)};
+#pragma unroll
+      for (int k = 0; k < D / 64; ++k) {
+        const float4 p = *reinterpret_cast<const float4*>(pi + (size_t)(lane + 64 * k) * D + d);
+        y[k] = __fadd_rn(y[k], __fmul_rn(u[0], p.x));
+        y[k] = __fadd_rn(y[k], __fmul_rn(u[1], p.y));
+        y[k] = __fadd_rn(y[k], __fmul_rn(u[2], p.z));
+        y[k] = __fadd_rn(y[k], __fmul_rn(u[3], p.w));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < D / 64; ++k) set_code<D, VB, TROWS>(st, t, lane + 64 * k, code_exact<VB>(y[k], bnd));
+  }
+}
+
+// Eight fields (field f8 * 8 on) as VB dwords of the stored bits.
+template <int VB, int D, int NTOK>
+__device__ __forceinline__ void pack_fields(const PolarStage<D, NTOK>& st, int f8, uint32_t (&w)[VB]) {
+  const uint4 v = *reinterpret_cast<const uint4*>(&st.fld[8 * f8]);
+  const uint32_t two[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int k = 0; k < VB; ++k) w[k] = 0u;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t f = (i & 1) ? two[i >> 1] >> 16 : two[i >> 1] & 0xFFFFu;
+    const int bit = 4 * VB * i;
+    w[bit >> 5] |= f << (bit & 31);
+    if ((bit & 31) + 4 * VB > 32) w[(bit >> 5) + 1] |= f >> (32 - (bit & 31));
   }
 }
 
@@ -248,6 +437,21 @@ __device__ __forceinline__ float pairwise_sumsq(const float (&x0)[D / 8], const 
     ss = blk == 0 ? bs : __fadd_rn(ss, bs);
   }
   return ss;
+}
+
+// The thread's channels (8m + 2q, 8m + 2q + 1) of a row times `scale`, as fp16
+// pairs: high halves to row[0..D), low ones to row[D..2D).
+template <int D>
+__device__ __forceinline__ void polar_stage_row(uint16_t* row, const float (&x0)[D / 8], const float (&x1)[D / 8],
+                                                int q, float scale) {
+#pragma unroll
+  for (int m = 0; m < D / 8; ++m) {
+    const float s0 = x0[m] * scale, s1 = x1[m] * scale;
+    const uint16_t h0 = f2h(s0), h1 = f2h(s1);
+    const uint16_t l0 = f2h(s0 - h2f(h0)), l1 = f2h(s1 - h2f(h1));
+    *reinterpret_cast<uint32_t*>(row + 8 * m + 2 * q) = (uint32_t)h0 | ((uint32_t)h1 << 16);
+    *reinterpret_cast<uint32_t*>(row + D + 8 * m + 2 * q) = (uint32_t)l0 | ((uint32_t)l1 << 16);
+  }
 }
 
 template <typename T>

@@ -27,6 +27,10 @@ constexpr int kThreads = 256;
 constexpr int kEncThreads = 256;
 constexpr int kEncWaves = kEncThreads / 64;
 
+// the order of stored codes, as PolarStage has it
+struct TokenRows { static constexpr bool value = false; };
+struct TiledRows { static constexpr bool value = true; };
+
 struct EncodeArgs {
   tqk_cache_desc d;
   tqk_cache_ptrs p;
@@ -135,7 +139,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
   // Key tile (fp16 bits, rows padded against bank conflicts).  Its rows also
   // take the key codes: the codes of token t overwrite the first D / 2 bytes of
   // row t once the wave that owns the row has read it (kc_row).  Then the area
-  // holds the value phase's codes (vc_s) and normalised rows (u_s).
+  // holds the value phase's rows and stage.
   __shared__ __align__(16) uint16_t kt_s[TQK_MAX_G][D + 8];
   __shared__ float stat_s[D][2];             // per channel: (mean, amax) or (min, scale)
   // per channel: 0x8000 - the fp16 magnitude threshold T (so m + it has bit 15
@@ -145,8 +149,6 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
   __shared__ uint32_t omask_s[TQK_MAX_G][D / 32];  // channels of each token stored in the side-list
   __shared__ int32_t wsum_s[kEncWaves];
   auto kc_row = [&](int t) { return reinterpret_cast<uint8_t*>(&kt_s[t][0]); };
-  uint8_t (*vc_s)[D] = reinterpret_cast<uint8_t (*)[D]>(&kt_s[0][0]);
-  static_assert(TQK_MAX_G * (D + 8) * 2 >= TQK_MAX_G * D + 64 * D * 4, "value staging overflows the key tile");
 
   if (d.key_grid != 2) {
     // ---- stage the key tile ----------------------------------------------
@@ -435,170 +437,144 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
         }
       }
     }
+    __syncthreads();
+    // key code rows, one 32-channel chunk (16 pair indices) per thread
+    const int KROW = k_row_bytes(d.key_bits, D);
+    for (int idx = tid; idx < G * (D / 32); idx += kEncThreads) {
+      const int t = idx / (D / 32), ch = idx % (D / 32);
+      const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
+      const uint4 f16 = *reinterpret_cast<const uint4*>(kc_row(t) + 16 * ch);
+      if (d.key_bits == 4) {
+        *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
+      } else {
+        // 16 fields of 2*kb bits, little-endian, into kb dwords
+        const int kb = d.key_bits;
+        const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
+        uint32_t o[3] = {0u, 0u, 0u};
+        for (int i = 0; i < 16; ++i) {
+          const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+          const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
+          o[w] |= f << sh;
+          if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
+        }
+        uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
+        for (int w = 0; w < kb; ++w) dst[w] = o[w];
+      }
+    }
+    __syncthreads();
   }
 
-  // ---- values -------------------------------------------------------------
-  constexpr int VROW = D * VB / 8;
-  const bool tiled = v_tiled(G, P, D, d.input_f32);
-  // PolarQuant codes of the group's tokens (the value encode; PolarQuant keys
-  // run it on the keys): norms to nout, codes staged in vc_s[token][channel]
-  // (the first TQK_MAX_G * D bytes of the key tile area)
-  auto polar_phase = [&](const void* ring, const void* chunk, float* nout, bool vcheck) {
-    // Rotation: in pass p, wave w owns the 16 rotated channels [64p + 16w,
-    // +16), lane l column e = 64p + 16w + (l & 15) of Pi_T (pi[e][0..D)) in
-    // registers; the tokens' normalised rows sit in LDS (kVBatch at a time,
-    // after the code staging area) and reach the lanes by DPP row broadcasts
-    // (rotate_codes) -- no LDS broadcast reads, which would cost the LDS a
-    // full wave's bandwidth each.
-    float bnd[15];
+  // ---- values (and PolarQuant keys) ----------------------------------------
+  // kVBatch tokens at a time: their rows staged in the key tile's area, norms
+  // (four threads per token, the reference's pairwise order), estimated codes
+  // (wave w: channels [NC w, NC w + NC)), the flagged ones recomputed, then the
+  // rows: LE bit streams of VB-bit codes per token, or 4-token x 8-channel
+  // units (the same eight fields a thread either way)
+  constexpr int VROW = D * VB / 8, NC = D / kEncWaves, NT = NC >= 32 ? 2 : 1, kVBatch = 128;
+  using Stage = PolarStage<D, kVBatch>;
+  static_assert(kVBatch * (D + 8) * 2 % 16 == 0 &&
+                kVBatch * (D + 8) * 2 + sizeof(Stage) <= sizeof(kt_s), "value staging overflows the key tile");
+  Stage& st = *reinterpret_cast<Stage*>(&kt_s[kVBatch][0]);
+  float bnd[15];
 #pragma unroll
-    for (int k = 0; k < (1 << VB) - 1; ++k) bnd[k] = a.p.vbnd[k];
-    constexpr int kVBatch = 64;  // rows per batch (rotate_codes takes at most 64)
-    float (*u_s)[D] = reinterpret_cast<float (*)[D]>(&kt_s[0][0] + TQK_MAX_G * D / 2);
+  for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
+  auto polar_phase = [&](const void* ring, const void* chunk, float* nout, bool vcheck, auto trows,
+                         auto put) {
+    constexpr bool TROWS = decltype(trows)::value;
     for (int t0 = 0; t0 < G; t0 += kVBatch) {
       const int nb = min(kVBatch, G - t0);
-      // (1) norms and normalised rows, four threads per token: thread q holds
-      // channels 8m + 2q, 8m + 2q + 1 (pairwise_sumsq's partial sums)
-      {
-        const int tt = tid >> 2, q = tid & 3;
-        if (tt < nb) {
-          const int t = g * G + t0 + tt;
-          const uint32_t* src = reinterpret_cast<const uint32_t*>(token_src<D>(a, ring, chunk, b, h, t));
-          float x0[D / 8], x1[D / 8];
+      for (int idx = tid; idx < nb * (D / 8); idx += kEncThreads) {
+        const int t = idx / (D / 8), c = idx % (D / 8);
+        reinterpret_cast<uint4*>(&kt_s[t][0])[c] =
+            reinterpret_cast<const uint4*>(token_src<D>(a, ring, chunk, b, h, g * G + t0 + t))[c];
+      }
+      if (tid == 0) st.nlist = 0;
+      __syncthreads();
+      for (int t4 = tid; t4 < 4 * nb; t4 += kEncThreads) {
+        const int t = t4 >> 2, q = t4 & 3;
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(&kt_s[t][0]);
+        float x0[D / 8], x1[D / 8];
+        uint32_t any = 0;
 #pragma unroll
-          for (int m = 0; m < D / 8; ++m) {
-            const uint32_t w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
-            x0[m] = h2f((uint16_t)(w2 & 0xFFFFu));
-            x1[m] = h2f((uint16_t)(w2 >> 16));
-          }
-          const float ss = pairwise_sumsq<D>(x0, x1, q);
-          const float nrm = __builtin_sqrtf(ss);  // correctly rounded (-fhip-fp32-correctly-rounded-divide-sqrt)
-          const float safe = fmaxf(nrm, 1e-30f);
-#pragma unroll
-          for (int m = 0; m < D / 8; ++m) {
-            u_s[tt][8 * m + 2 * q] = __fdiv_rn(x0[m], safe);
-            u_s[tt][8 * m + 2 * q + 1] = __fdiv_rn(x1[m], safe);
-          }
-          if (q == 0) {
-            nout[page_row(a.p.block_table, d.max_pages_per_seq, b, t, P, d.n_pages, h)] = nrm;
-            if (vcheck && nrm > TQK_MAX_VNORM && a.overflow) atomicOr(a.overflow, TQK_OVF_VNORM);
-          }
+        for (int m = 0; m < D / 8; ++m) {
+          const uint32_t w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
+          any |= w2;
+          x0[m] = h2f((uint16_t)(w2 & 0xFFFFu));
+          x1[m] = h2f((uint16_t)(w2 >> 16));
+        }
+        any |= __shfl_xor(any, 1, 4);
+        any |= __shfl_xor(any, 2, 4);
+        const float ss = pairwise_sumsq<D>(x0, x1, q);
+        const float nrm = __builtin_sqrtf(ss);  // correctly rounded (-fhip-fp32-correctly-rounded-divide-sqrt)
+        if (q == 0) {
+          polar_token(st, t, ss, nrm, (any & 0x7FFF7FFFu) == 0u, __builtin_amdgcn_rcpf(nrm) * (1.0f / kPiScale));
+          nout[page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + t, P, d.n_pages, h)] = nrm;
+          if (vcheck && nrm > TQK_MAX_VNORM && a.overflow) atomicOr(a.overflow, TQK_OVF_VNORM);
         }
       }
       __syncthreads();
-      // (2) rotation and codes, D / (16 * kEncWaves) passes over the channels
-      for (int pass = 0; pass < D / (16 * kEncWaves); ++pass)
-        rotate_codes<D, VB>(a.p.pi, u_s, nb, 16 * kEncWaves * pass + 16 * wv + (lane & 15), lane, bnd,
-                            vc_s + t0);
-      __syncthreads();
-    }
-  };
-  // code row of token t for the key write-out
-  const uint8_t* kc_base = kc_row(0);
-  int kc_stride = (D + 8) * 2;
-  if (d.key_grid == 2) {
-    // PolarQuant keys (turboquant_pro/core.py:542-617 with kind="key"): the
-    // value encode on the key tokens, norms to knorm, then each row's codes
-    // turned in place (one wave per row) into one table index per channel
-    // pair; the per-channel stats are the identity (scale 1, mean 0) and
-    // there is no side-list
-    polar_phase(a.p.hot_k, a.chunk_k, a.p.knorm, false);
-    for (int t = wv; t < G; t += kEncWaves) {
-      // every pair of the row read before any index is written over it
-      constexpr int NPL = (D / 2 + 63) / 64;  // channel pairs per lane
-      uint32_t f[NPL];
-#pragma unroll
-      for (int k = 0; k < NPL; ++k) {
-        const int pr = lane + 64 * k;
-        const uint32_t cc = pr < D / 2 ? *reinterpret_cast<const uint16_t*>(&vc_s[t][2 * pr]) : 0u;
-        const uint32_t c0 = cc & 0xFFu, c1 = cc >> 8;
-        f[k] = d.key_bits == 4 ? ((rev4(c0) << 4) | rev4(c1)) : (c0 | (c1 << d.key_bits));
+      for (int e0 = NC * wv; e0 < NC * wv + NC; e0 += 16 * NT) {
+        PiFrags<D, NT> pf;
+        load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
+        polar_codes<D, NT, VB, false, TROWS>(st, pf, &kt_s[0][0], D + 8, nb, e0, lane, bnd);
       }
-#pragma unroll
-      for (int k = 0; k < NPL; ++k)
-        if (lane + 64 * k < D / 2) vc_s[t][lane + 64 * k] = (uint8_t)f[k];
+      __syncthreads();
+      if (st.nlist > 0) {
+        polar_fix<D, VB, TROWS, kEncThreads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
+          const uint2 w = *reinterpret_cast<const uint2*>(&kt_s[t][dd]);
+          return make_float4(h2f((uint16_t)w.x), h2f((uint16_t)(w.x >> 16)), h2f((uint16_t)w.y),
+                             h2f((uint16_t)(w.y >> 16)));
+        });
+        __syncthreads();
+      }
+      for (int f8 = tid; f8 < nb * (D / 32); f8 += kEncThreads) {
+        uint32_t w[VB];
+        pack_fields<VB>(st, f8, w);
+        put(t0, f8, w);
+      }
+      // (the next batch's rows may replace these: the fields are written again
+      // only two barriers later)
     }
-    kc_base = &vc_s[0][0];
-    kc_stride = D;
+    __syncthreads();
+  };
+  auto put_row = [&](uint8_t* base, int t0, int f8, const uint32_t (&w)[VB]) {
+    const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + f8 / (D / 32), P,
+                                d.n_pages, h);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(base + row * VROW) + VB * (f8 % (D / 32));
+#pragma unroll
+    for (int k = 0; k < VB; ++k) dst[k] = w[k];
+  };
+  if (d.key_grid == 2) {
+    // PolarQuant keys (turboquant_pro/core.py:542-617 with kind="key"; key_bits
+    // == value_bits): the value encode on the key tokens, norms to knorm; 2-
+    // and 3-bit key rows are the same bit stream, 4-bit ones its bytes with
+    // their bits reversed.  The per-channel stats are the identity (scale 1,
+    // mean 0) and there is no side-list.
+    polar_phase(a.p.hot_k, a.chunk_k, a.p.knorm, false, TokenRows{}, [&](int t0, int f8, uint32_t (&w)[VB]) {
+      if constexpr (VB == 4) {
+#pragma unroll
+        for (int k = 0; k < VB; ++k) w[k] = __builtin_bswap32(__builtin_bitreverse32(w[k]));
+      }
+      put_row(a.p.kcodes, t0, f8, w);
+    });
     if (tid < D) {
       a.p.gscale[mbase + tid] = 1.0f;
       a.p.gmean[mbase + tid] = 0.0f;
     }
     if (tid < TQK_NOB) a.p.ocount[obase * TQK_NOB + tid] = 0;
   }
-  __syncthreads();
-  // key code rows, one 32-channel chunk (16 pair indices) per thread
-  const int KROW = k_row_bytes(d.key_bits, D);
-  for (int idx = tid; idx < G * (D / 32); idx += kEncThreads) {
-    const int t = idx / (D / 32), ch = idx % (D / 32);
-    const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
-    const uint4 f16 = *reinterpret_cast<const uint4*>(kc_base + (size_t)t * kc_stride + 16 * ch);
-    if (d.key_bits == 4) {
-      *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
-    } else {
-      // 16 fields of 2*kb bits, little-endian, into kb dwords
-      const int kb = d.key_bits;
-      const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
-      uint32_t o[3] = {0u, 0u, 0u};
-      for (int i = 0; i < 16; ++i) {
-        const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
-        const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
-        o[w] |= f << sh;
-        if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
-      }
-      uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
-      for (int w = 0; w < kb; ++w) dst[w] = o[w];
-    }
-  }
-  __syncthreads();
-  polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, true);
-  // (3) the code rows: 4-token x 8-channel units of 16-token tiles, or the
-  // reference's little-endian bit stream per token
-  if (D == TQK_D && tiled) {
-    // one unit = tokens [16T + 4lg, +4) x channels [8c, +8) of 16-token tile T
-    for (int un = tid; un < (G / 16) * 64; un += kEncThreads) {
-      const int T = un >> 6, lg = (un >> 4) & 3, c = un & 15;
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int uu = 0; uu < 4; ++uu) {
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-          const uint32_t code = vc_s[16 * T + 4 * lg + uu][8 * c + nt];
-          const int bit = v_unit_bit(uu, nt, VB);
-          w[bit >> 5] |= code << (bit & 31);
-          if ((bit & 31) + VB > 32) w[(bit >> 5) + 1] |= code >> (32 - (bit & 31));
-        }
-      }
-      const int t0 = g * G + 16 * T;  // tile start (absolute token), never straddles a page
-      const size_t row0 = page_row(a.p.block_table, d.max_pages_per_seq, b, t0, P, d.n_pages, h);
+  if (D == TQK_D && v_tiled(G, P, D, d.input_f32)) {
+    polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, true, TiledRows{}, [&](int t0, int f8, uint32_t (&w)[VB]) {
+      // unit (lg, c): tokens [4 lg, +4) of tile T, channels [8c, +8)
+      const int T = f8 >> 6, lg = (f8 >> 4) & 3, c = f8 & 15;
+      const size_t row0 = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + 16 * T, P, d.n_pages, h);
       uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.vcodes + row0 * VROW + v_unit_offset(lg, c, VROW));
 #pragma unroll
-      for (int k = 0; k < VROW / 16; ++k) dst[k] = w[k];
-    }
-  } else if (tid < G) {
-    uint32_t outw[VROW / 4];
-#pragma unroll
-    for (int k = 0; k < VROW / 4; ++k) outw[k] = 0u;
-#pragma unroll
-    for (int e = 0; e < D; ++e) {
-      const uint32_t code = vc_s[tid][e];
-      const int bitpos = e * VB;  // little-endian bit stream (3-bit: 8 codes per 24 bits)
-      outw[bitpos >> 5] |= code << (bitpos & 31);
-      if ((bitpos & 31) + VB > 32) outw[(bitpos >> 5) + 1] |= code >> (32 - (bitpos & 31));
-    }
-    const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + tid, P, d.n_pages, h);
-    // 16-byte stores where the row is whole 16-byte pieces (3-bit rows at
-    // head_dim 64 are 24 bytes: dword stores)
-    if constexpr (VROW % 16 == 0) {
-      uint4* dst = reinterpret_cast<uint4*>(a.p.vcodes + row * VROW);
-#pragma unroll
-      for (int k = 0; k < VROW / 16; ++k)
-        dst[k] = make_uint4(outw[4 * k], outw[4 * k + 1], outw[4 * k + 2], outw[4 * k + 3]);
-    } else {
-      uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.vcodes + row * VROW);
-#pragma unroll
-      for (int k = 0; k < VROW / 4; ++k) dst[k] = outw[k];
-    }
+      for (int k = 0; k < VB; ++k) dst[k] = w[k];
+    });
+  } else {
+    polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, true, TokenRows{},
+                [&](int t0, int f8, uint32_t (&w)[VB]) { put_row(a.p.vcodes, t0, f8, w); });
   }
 }
 
@@ -621,51 +597,84 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
   const int kout = d.outliers_per_channel;
   const size_t mbase = ((size_t)slot * Hkv + h) * D;
   const size_t obase = (size_t)slot * Hkv + h;
-  constexpr int kVBatch = 64;  // rows per value batch (rotate_codes takes at most 64)
+  constexpr int kVBatch = 64;  // tokens per value batch: four threads each
   constexpr int VROW = D * VB / 8;
 
   __shared__ const float* krow_s[TQK_MAX_G];                // source row of each key token
   __shared__ float stat_s[D][2];                             // (mean, amax) or (min, scale)
   __shared__ float thr_s[D];                                 // outlier magnitude threshold
   __shared__ __align__(16) uint8_t kc_s[TQK_MAX_G][D / 2];   // table index per (token, channel pair)
-  __shared__ __align__(16) float u_s[kVBatch][D];
-  __shared__ __align__(16) uint8_t vc_s[kVBatch][D];
+  // scaled rows of a value batch as fp16 pairs (high halves, then low ones)
+  __shared__ __align__(16) uint16_t uv_s[kVBatch][2 * D + 8];
+  __shared__ __align__(16) PolarStage<D, kVBatch> st;
+  __shared__ const float* vrow_s[kVBatch];
   __shared__ int32_t wsum_s[kEncWaves];
 
   for (int t = tid; t < G; t += kEncThreads)
     krow_s[t] = token_src<D, float>(a, a.p.hot_k, a.chunk_k, b, h, g * G + t);
   __syncthreads();
 
-  // norms and normalised rows of tokens [t0, t0 + nb) (four threads per
-  // token, pairwise_sumsq), then their rotated codes into vc_s
   float bnd[15];
 #pragma unroll
-  for (int k = 0; k < (1 << VB) - 1; ++k) bnd[k] = a.p.vbnd[k];
-  auto polar_batch = [&](const void* ring, const void* chunk, int t0, int nb, float* nout) {
-    const int tt = tid >> 2, q = tid & 3;
-    if (tt < nb) {
-      const int t = g * G + t0 + tt;
-      const float2* src = reinterpret_cast<const float2*>(token_src<D, float>(a, ring, chunk, b, h, t));
-      float x0[D / 8], x1[D / 8];
+  for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
+  constexpr int NC = D / kEncWaves, NT = NC >= 32 ? 2 : 1;
+  // PolarQuant of the group's tokens, kVBatch at a time: norms (four threads
+  // per token, pairwise_sumsq) and the scaled rows' fp16 pairs, estimated
+  // codes, the flagged ones recomputed from the fp32 rows, the bit streams
+  auto polar_phase = [&](const void* ring, const void* chunk, float* nout, uint8_t* rows, bool reversed) {
+    for (int t0 = 0; t0 < G; t0 += kVBatch) {
+      const int nb = min(kVBatch, G - t0);
+      if (tid == 0) st.nlist = 0;
+      const int tt = tid >> 2, q = tid & 3;
+      if (tt < nb) {
+        const int t = g * G + t0 + tt;
+        const float* sp = token_src<D, float>(a, ring, chunk, b, h, t);
+        if (q == 0) vrow_s[tt] = sp;
+        const float2* src = reinterpret_cast<const float2*>(sp);
+        float x0[D / 8], x1[D / 8];
+        uint32_t any = 0;
 #pragma unroll
-      for (int m = 0; m < D / 8; ++m) {
-        const float2 w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
-        x0[m] = w2.x;
-        x1[m] = w2.y;
+        for (int m = 0; m < D / 8; ++m) {
+          const float2 w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
+          x0[m] = w2.x;
+          x1[m] = w2.y;
+          any |= __float_as_uint(w2.x) | __float_as_uint(w2.y);
+        }
+        any |= __shfl_xor(any, 1, 4);
+        any |= __shfl_xor(any, 2, 4);
+        const float ss = pairwise_sumsq<D>(x0, x1, q);
+        const float nrm = __builtin_sqrtf(ss);
+        const bool zero = (any & 0x7FFFFFFFu) == 0u;
+        polar_stage_row<D>(&uv_s[tt][0], x0, x1, q, zero ? 0.f : kPiScale * __builtin_amdgcn_rcpf(nrm));
+        if (q == 0) {
+          polar_token(st, tt, ss, nrm, zero, 1.0f / (kPiScale * kPiScale));
+          nout[page_row(a.p.block_table, d.max_pages_per_seq, b, t, P, d.n_pages, h)] = nrm;
+        }
       }
-      const float nrm = __builtin_sqrtf(pairwise_sumsq<D>(x0, x1, q));
-      const float safe = fmaxf(nrm, 1e-30f);
+      __syncthreads();
+      for (int e0 = NC * wv; e0 < NC * wv + NC; e0 += 16 * NT) {
+        PiFrags<D, NT> pf;
+        load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
+        polar_codes<D, NT, VB, true, false>(st, pf, &uv_s[0][0], 2 * D + 8, nb, e0, lane, bnd);
+      }
+      __syncthreads();
+      if (st.nlist > 0) {
+        polar_fix<D, VB, false, kEncThreads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
+          return *reinterpret_cast<const float4*>(vrow_s[t] + dd);
+        });
+        __syncthreads();
+      }
+      for (int f8 = tid; f8 < nb * (D / 32); f8 += kEncThreads) {
+        uint32_t w[VB];
+        pack_fields<VB>(st, f8, w);
+        const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + f8 / (D / 32), P,
+                                    d.n_pages, h);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(rows + row * VROW) + VB * (f8 % (D / 32));
 #pragma unroll
-      for (int m = 0; m < D / 8; ++m) {
-        u_s[tt][8 * m + 2 * q] = __fdiv_rn(x0[m], safe);
-        u_s[tt][8 * m + 2 * q + 1] = __fdiv_rn(x1[m], safe);
+        for (int k = 0; k < VB; ++k) dst[k] = reversed ? __builtin_bswap32(__builtin_bitreverse32(w[k])) : w[k];
       }
-      if (q == 0) nout[page_row(a.p.block_table, d.max_pages_per_seq, b, t, P, d.n_pages, h)] = nrm;
+      __syncthreads();
     }
-    __syncthreads();
-    for (int pass = 0; pass < D / (16 * kEncWaves); ++pass)
-      rotate_codes<D, VB>(a.p.pi, u_s, nb, 16 * kEncWaves * pass + 16 * wv + (lane & 15), lane, bnd, vc_s);
-    __syncthreads();
   };
 
   if (d.key_grid != 2) {
@@ -827,69 +836,41 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
       }
     }
   } else {
-    // PolarQuant keys: the value encode on the key tokens, norms to knorm;
-    // each token's codes become one table index per channel pair
-    for (int t0 = 0; t0 < G; t0 += kVBatch) {
-      const int nb = min(kVBatch, G - t0);
-      polar_batch(a.p.hot_k, a.chunk_k, t0, nb, a.p.knorm);
-      for (int i = tid; i < nb * (D / 2); i += kEncThreads) {
-        const int t = i / (D / 2), pr = i % (D / 2);
-        const uint32_t c0 = vc_s[t][2 * pr], c1 = vc_s[t][2 * pr + 1];
-        kc_s[t0 + t][pr] = (uint8_t)(d.key_bits == 4 ? ((rev4(c0) << 4) | rev4(c1)) : (c0 | (c1 << d.key_bits)));
-      }
-    }
+    // PolarQuant keys: the value encode on the key tokens, norms to knorm; key
+    // rows as the fp16 encode writes them (4-bit bytes bit-reversed)
+    polar_phase(a.p.hot_k, a.chunk_k, a.p.knorm, a.p.kcodes, VB == 4);
     if (tid < D) {
       a.p.gscale[mbase + tid] = 1.0f;
       a.p.gmean[mbase + tid] = 0.0f;
     }
     if (tid < TQK_NOB) a.p.ocount[obase * TQK_NOB + tid] = 0;
   }
-  __syncthreads();
-  // key code rows, one 32-channel chunk (16 table indices) per thread
-  const int KROW = k_row_bytes(d.key_bits, D);
-  for (int idx = tid; idx < G * (D / 32); idx += kEncThreads) {
-    const int t = idx / (D / 32), ch = idx % (D / 32);
-    const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
-    const uint4 f16 = *reinterpret_cast<const uint4*>(&kc_s[t][16 * ch]);
-    if (d.key_bits == 4) {
-      *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
-    } else {
-      const int kb = d.key_bits;
-      const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
-      uint32_t o[3] = {0u, 0u, 0u};
-      for (int i = 0; i < 16; ++i) {
-        const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
-        const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
-        o[w] |= f << sh;
-        if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
+  if (d.key_grid != 2) {
+    __syncthreads();
+    // key code rows, one 32-channel chunk (16 table indices) per thread
+    const int KROW = k_row_bytes(d.key_bits, D);
+    for (int idx = tid; idx < G * (D / 32); idx += kEncThreads) {
+      const int t = idx / (D / 32), ch = idx % (D / 32);
+      const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
+      const uint4 f16 = *reinterpret_cast<const uint4*>(&kc_s[t][16 * ch]);
+      if (d.key_bits == 4) {
+        *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
+      } else {
+        const int kb = d.key_bits;
+        const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
+        uint32_t o[3] = {0u, 0u, 0u};
+        for (int i = 0; i < 16; ++i) {
+          const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+          const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
+          o[w] |= f << sh;
+          if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
+        }
+        uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
+        for (int w = 0; w < kb; ++w) dst[w] = o[w];
       }
-      uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
-      for (int w = 0; w < kb; ++w) dst[w] = o[w];
     }
   }
-  // ---- values, kVBatch tokens at a time: codes, then the reference's
-  // little-endian bit stream per token
-  for (int t0 = 0; t0 < G; t0 += kVBatch) {
-    const int nb = min(kVBatch, G - t0);
-    polar_batch(a.p.hot_v, a.chunk_v, t0, nb, a.p.vnorm);
-    if (tid < nb) {
-      uint32_t outw[VROW / 4];
-#pragma unroll
-      for (int k = 0; k < VROW / 4; ++k) outw[k] = 0u;
-#pragma unroll
-      for (int e = 0; e < D; ++e) {
-        const uint32_t code = vc_s[tid][e];
-        const int bitpos = e * VB;
-        outw[bitpos >> 5] |= code << (bitpos & 31);
-        if ((bitpos & 31) + VB > 32) outw[(bitpos >> 5) + 1] |= code >> (32 - (bitpos & 31));
-      }
-      const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + tid, P, d.n_pages, h);
-      uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.vcodes + row * VROW);
-#pragma unroll
-      for (int k = 0; k < VROW / 4; ++k) dst[k] = outw[k];
-    }
-    __syncthreads();  // vc_s is the next batch's
-  }
+  polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, a.p.vcodes, false);
 }
 
 
