@@ -363,6 +363,9 @@ __device__ __forceinline__ void polar_fix(PolarStage<D, NTOK>& st, const float* 
                             __fmul_rn(__fdiv_rn(xb.z, safe), pb.z), __fmul_rn(__fdiv_rn(xb.w, safe), pb.w)};
         add_row_dpp<0, CH / 8>(y, f);
       }
+      // keeps the sum out of the conditional store: sunk into it, the additions
+      // would leave their broadcasts behind as separate moves
+      asm volatile("" : "+v"(y));
       if (i < n && li == 0)  // (a NaN norm makes u, and so y, NaN)
         set_code<D, VB, TROWS>(st, t, e, code_exact<VB>(st.nrm[t] != st.nrm[t] ? st.nrm[t] : y, bnd));
     }
@@ -374,6 +377,7 @@ __device__ __forceinline__ void polar_fix(PolarStage<D, NTOK>& st, const float* 
     float y[D / 64];
 #pragma unroll
     for (int k = 0; k < D / 64; ++k) y[k] = st.nrm[t] != st.nrm[t] ? st.nrm[t] : 0.f;
+#pragma unroll 1
     for (int d = st.nrm[t] != st.nrm[t] ? D : 0; d < D; d += 4) {
       const float4 x = x4(t, d);
       const float u[4] = {__fdiv_rn(x.x, safe), __fdiv_rn(x.y, safe), __fdiv_rn(x.z, safe), __fdiv_rn(x.w, safe)};

@@ -22,10 +22,12 @@
 namespace {
 
 constexpr int kThreads = 256;
-// the group encode: four waves; its LDS (under 80 KiB) lets two workgroups share
-// a CU, so one's latency-bound key phase runs beside the other's value rotation
-constexpr int kEncThreads = 256;
+// the fp16 group encode: eight waves; its LDS (under 80 KiB at head_dim 128) lets
+// two workgroups share a CU, four waves per SIMD
+constexpr int kEncThreads = 512;
 constexpr int kEncWaves = kEncThreads / 64;
+constexpr int kF32Threads = 256;
+constexpr int kF32Waves = kF32Threads / 64;
 
 // the order of stored codes, as PolarStage has it
 struct TokenRows { static constexpr bool value = false; };
@@ -39,6 +41,7 @@ struct EncodeArgs {
   const void* chunk_k;  // fp16, or fp32 (input_f32)
   const void* chunk_v;
   int chunk_tokens;
+  int n_items;
   int32_t* overflow;
 };
 
@@ -124,9 +127,51 @@ __device__ __forceinline__ int sum_quarters(int x) {
 }
 
 
+// ---- asym-NF4 codes by bucket -----------------------------------------------
+// With the normalised key t = (x - mean) / amax cut into 32 buckets of 1/16 on
+// [-1, 1], every bucket widened by 0.004 on both sides holds at most one
+// midpoint of two NF4 levels (they are at least 0.080 apart), so a bucket's
+// codes are kNf4Pair[bucket] or the next one, and one comparison of x decides:
+// code = pair + (x >= X), X the smallest fp16 number that argmin puts on the
+// pair's upper level.  kNf4From[k] is the first bucket of pair k.
+__constant__ static const int kNf4From[16] = {0, 3, 7, 9, 11, 13, 14, 16, 17, 18, 20, 21, 23, 25, 27, 32};
+
+// the smallest fp16 number x (as bits; 0x7C00 when there is none) with
+// fl|x - c1| < fl|x - c0|, for levels c0 < c1 far enough apart that the two
+// rounded distances order like the real ones away from the midpoint: nearly
+// always next to the rounded midpoint, else searched for
+__device__ __forceinline__ uint16_t nf4_threshold(float c0, float c1) {
+  auto bits = [](int o) { return (uint16_t)(o < 0 ? 0x8000 - o : o); };
+  auto upper = [&](int o) {
+    const float x = h2f(bits(o));
+    return x >= c1 || (x > c0 && fabsf(__fsub_rn(x, c1)) < fabsf(__fsub_rn(x, c0)));
+  };
+  const uint16_t mb = f2h(0.5f * c0 + 0.5f * c1);
+  const int m = (mb & 0x8000) ? -(int)(mb & 0x7FFF) : (int)mb;
+  if (m > -0x7BFF && m < 0x7BFF && !upper(m - 1) && upper(m + 1)) return bits(upper(m) ? m : m + 1);
+  int lo = -0x7C00, hi = 0x7C00;  // not upper, upper (neither is evaluated)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (upper(mid)) hi = mid;
+    else lo = mid;
+  }
+  return bits(hi);
+}
+
+// One workgroup per (group, kv head) and side: eight consecutive key
+// workgroups, then the eight value workgroups of the same groups, so that
+// every XCD and CU gets both kinds and a flush of one group runs them side by
+// side.  What bounds it: the keys' VALU work and LDS traffic (statistics,
+// thresholds, side-list, codes: VALU 62 % busy at four waves per SIMD).  16
+// sequences x 8192 tokens x 8 heads at head_dim 128, appended in 4096-token
+// chunks: 868 us with both sides in one 256-thread workgroup and the argmin
+// over 16 levels, 624 us like this.
 template <int VB, int D>
-__global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
-  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+__global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group(EncodeArgs a) {
+  const int unit = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
+  const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
+  if (unit >= a.n_items * a.d.n_kv_heads) return;
+  const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const tqk_cache_desc& d = a.d;
   const int b = a.items[2 * item], g = a.items[2 * item + 1];
@@ -138,19 +183,31 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
 
   // Key tile (fp16 bits, rows padded against bank conflicts).  Its rows also
   // take the key codes: the codes of token t overwrite the first D / 2 bytes of
-  // row t once the wave that owns the row has read it (kc_row).  Then the area
-  // holds the value phase's rows and stage.
+  // row t once the wave that owns the row has read it (kc_row).  On the value
+  // side the area holds the rows and stage of a value batch.
   __shared__ __align__(16) uint16_t kt_s[TQK_MAX_G][D + 8];
   __shared__ float stat_s[D][2];             // per channel: (mean, amax) or (min, scale)
   // per channel: 0x8000 - the fp16 magnitude threshold T (so m + it has bit 15
   // set exactly when m >= T; 0 for a NaN T), read eight channels at a time by
   // the side-list scan
   __shared__ __align__(16) uint16_t tbias_s[D];
-  __shared__ uint32_t omask_s[TQK_MAX_G][D / 32];  // channels of each token stored in the side-list
+  // channels of each token stored in the side-list: in the tile rows' padding
+  // where it fits
+  __shared__ uint32_t omx_s[D > 128 ? TQK_MAX_G : 1][D / 32];
+  // per bucket and channel (of 64 channels): X | rev4(code) << 16 | rev4(code +
+  // 1) << 20; row 32: the stored outliers' code.  Channel c at column (c >> 1) +
+  // 32 (c & 1): the two half-waves read columns of different halves at a time,
+  // so a wave's reads never share a bank.
+  __shared__ uint32_t nf_s[33][64];
+  __shared__ uint32_t crowded_s;  // bit of every 64 channels with levels too close for the buckets
   __shared__ int32_t wsum_s[kEncWaves];
   auto kc_row = [&](int t) { return reinterpret_cast<uint8_t*>(&kt_s[t][0]); };
+  auto om_row = [&](int t) {
+    if constexpr (D > 128) return &omx_s[t][0];
+    else return reinterpret_cast<uint32_t*>(&kt_s[t][D]);
+  };
 
-  if (d.key_grid != 2) {
+  if (d.key_grid != 2 && key_side) {
     // ---- stage the key tile ----------------------------------------------
     for (int idx = tid; idx < G * (D / 8); idx += kEncThreads) {
       const int t = idx / (D / 8), c = idx % (D / 8);
@@ -158,123 +215,184 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
           reinterpret_cast<const uint4*>(token_src<D>(a, a.p.hot_k, a.chunk_k, b, h, g * G + t));
       reinterpret_cast<uint4*>(&kt_s[t][0])[c] = src[c];
     }
+    if (tid == 0) crowded_s = 0u;
     __syncthreads();
 
-    // ---- per-channel statistics (thread j: channel j) ------------------------
-    if (tid < D && d.key_grid == 1) {
-      // uniform keys (turboquant_pro/per_channel_kv.py:303-306): channel min and
-      // max over the tokens, scale = max(max - min, 1e-8) / (2^bits - 1) (NaN propagates)
+    // ---- the zero point (turboquant_pro/per_channel_kv.py:327-345), thread j:
+    // channel j, a sum in token order
+    if (tid < D && d.key_grid != 1) {
       const int j = tid;
-      float mn = h2f(kt_s[0][j]), mx = mn;
-      bool nan = (mn != mn);
-      for (int s = 1; s < G; ++s) {
-        const float xv = h2f(kt_s[s][j]);
-        nan |= (xv != xv);
-        mn = fminf(mn, xv);
-        mx = fmaxf(mx, xv);
-      }
-      const float rng = __fsub_rn(mx, mn);
-      const float sc = nan ? __builtin_nanf("") : __fdiv_rn(fmaxf(rng, 1e-8f), (float)((1 << d.key_bits) - 1));
-      if (nan) mn = __builtin_nanf("");
-      stat_s[j][0] = mn;
-      stat_s[j][1] = sc;
-      a.p.gscale[mbase + j] = sc;
-      a.p.gmean[mbase + j] = mn;
-    } else if (tid < D) {
-      const int j = tid;
-      // the zero point (turboquant_pro/per_channel_kv.py:327-345)
       float mu;
       if (d.zero_point == 2) {
         // "bias": the RoPE-averaged k_proj bias of the group's positions
         mu = a.p.zp_mean[((size_t)g * Hkv + h) * D + j];
       } else {
         float acc = 0.0f;
-        for (int s = 0; s < G; ++s) acc = __fadd_rn(acc, h2f(kt_s[s][j]));
+        int s = 0;
+        for (; s + 16 <= G; s += 16) {
+          uint16_t x[16];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) x[u] = kt_s[s + u][j];
+#pragma unroll
+          for (int u = 0; u < 16; ++u) acc = __fadd_rn(acc, h2f(x[u]));
+        }
+        for (; s < G; ++s) acc = __fadd_rn(acc, h2f(kt_s[s][j]));
         // np.mean divides the fp32 sum by an intp count: a float64 division, then fp32
         mu = (float)((double)acc / (double)G);
         // "sparse": the mean times the DC-channel mask (a float product, so a
         // non-DC channel gets a signed zero, or NaN from a NaN mean)
         if (d.zero_point == 1) mu = __fmul_rn(mu, ((d.dc_mask[j >> 5] >> (j & 31)) & 1u) ? 1.0f : 0.0f);
       }
-      float amax = 0.0f;
-      bool nan = (mu != mu);
-      for (int s = 0; s < G; ++s) {
-        const float dv = fabsf(__fsub_rn(h2f(kt_s[s][j]), mu));
-        nan |= (dv != dv);
-        amax = fmaxf(amax, dv);
-      }
-      amax = nan ? __builtin_nanf("") : fmaxf(amax, 1e-8f);
       stat_s[j][0] = mu;
-      stat_s[j][1] = amax;
-      a.p.gscale[mbase + j] = amax;
-      a.p.gmean[mbase + j] = mu;
     }
-    // ---- outlier thresholds: the k-th largest |x| of each channel as the
-    // largest fp16 magnitude pattern T with #{ |x_s| >= T } >= k (NaN patterns
-    // order above inf, as np.partition does).  Every thread, 16 channels per
-    // wave and pass: lanes l, l ^ 16, l ^ 32, l ^ 48 take a quarter of the
-    // tokens each, two magnitudes per register.  For k <= 8 the k largest are
-    // kept directly (packed 16-bit max/min insertion); otherwise a bitwise
-    // search, a candidate's count the carry bit of a packed 16-bit add,
-    // summed over the four lanes.
-    if (kout > 0 && kout < G) {
+    __syncthreads();
+    // ---- the other statistics and the outlier thresholds, 16 channels per
+    // wave and pass: lanes l, l ^ 16, l ^ 32, l ^ 48 hold a quarter of the
+    // tokens each, two per register.
+    // Thresholds: the k-th largest |x| of each channel as the largest fp16
+    // magnitude pattern T with #{ |x_s| >= T } >= k (NaN patterns order above
+    // inf, as np.partition does).  For k <= 8 the k largest are kept directly
+    // (packed 16-bit max/min insertion); otherwise a bitwise search, a
+    // candidate's count the carry bit of a packed 16-bit add, summed over the
+    // four lanes.
+    {
       const int part = lane >> 4;
       for (int j = 16 * wv + (lane & 15); j < D; j += 16 * kEncWaves) {
-        u16x2_t m2[TQK_MAX_G / 8];
+        // lane quarter `part` takes token pairs 8i + 2 part (rows 4 apart fall on
+        // LDS banks 8 apart, so the four quarters never conflict); eight pairs
+        // at a time, pairs past G repeat the last token
+        auto for_quarter = [&](auto f) {
+#pragma unroll 1
+          for (int i0 = 0; i0 < TQK_MAX_G / 8; i0 += 8) {
+            uint16_t x[16];
 #pragma unroll
-        for (int i = 0; i < TQK_MAX_G / 8; ++i) {
-          // lane quarter `part` takes token pairs 8i + 2 part (rows 4 apart
-          // fall on LDS banks 8 apart, so the four quarters never conflict);
-          // tokens past G count as magnitude 0
-          const int s = 8 * i + 2 * part;
-          m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
-                          (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
-        }
-        uint32_t T = 0;
-        if (kout <= 5) {
-          T = kth_largest<5>(m2, kout);
-        } else if (kout <= 8) {
-          T = kth_largest<8>(m2, kout);
+            for (int i = 0; i < 8; ++i) {
+              const int s = 8 * (i0 + i) + 2 * part;
+              x[2 * i] = kt_s[min(s, G - 1)][j];
+              x[2 * i + 1] = kt_s[min(s + 1, G - 1)][j];
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f(x[2 * i], x[2 * i + 1]);
+          }
+        };
+        // NaN propagates into scale and zero point
+        uint32_t top = 0;  // the largest magnitude pattern
+        if (d.key_grid == 1) {
+          // uniform (turboquant_pro/per_channel_kv.py:303-306): channel min and
+          // max, scale = max(max - min, 1e-8) / (2^bits - 1)
+          float mn = __builtin_inff(), mx = -__builtin_inff();
+          for_quarter([&](uint16_t ya, uint16_t yb) {
+            top = max(top, max(abs_h(ya), abs_h(yb)));
+            const float x0 = h2f(ya), x1 = h2f(yb);
+            mn = fminf(mn, fminf(x0, x1));
+            mx = fmaxf(mx, fmaxf(x0, x1));
+          });
+#pragma unroll
+          for (int o = 16; o < 64; o <<= 1) {
+            mn = fminf(mn, __shfl_xor(mn, o, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+            top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+          }
+          if (part == 0) {
+            const bool nan = top > 0x7C00u;
+            const float sc = nan ? __builtin_nanf("")
+                                 : __fdiv_rn(fmaxf(__fsub_rn(mx, mn), 1e-8f), (float)((1 << d.key_bits) - 1));
+            if (nan) mn = __builtin_nanf("");
+            stat_s[j][0] = mn;
+            stat_s[j][1] = sc;
+            a.p.gscale[mbase + j] = sc;
+            a.p.gmean[mbase + j] = mn;
+          }
         } else {
-          for (int bit = 14; bit >= 0; --bit) {
-            const uint32_t cand = T | (1u << bit);
-            // m + (0x8000 - cand) has bit 15 set exactly when m >= cand (m, cand < 2^15)
-            const uint16_t bias = (uint16_t)(0x8000u - cand);
-            const u16x2_t bv = {bias, bias};
-            uint32_t acc = 0;  // two 16-bit counts
+          // amax = max |x - mean|, as magnitude patterns (a NaN is the largest)
+          const float mu = stat_s[j][0];
+          for_quarter([&](uint16_t ya, uint16_t yb) {
+            const uint32_t d0 = __float_as_uint(fabsf(__fsub_rn(h2f(ya), mu)));
+            const uint32_t d1 = __float_as_uint(fabsf(__fsub_rn(h2f(yb), mu)));
+            top = max(top, max(d0, d1));
+          });
 #pragma unroll
-            for (int i = 0; i < TQK_MAX_G / 8; ++i)
-              acc += (__builtin_bit_cast(uint32_t, (u16x2_t)(m2[i] + bv)) >> 15) & 0x00010001u;
-            const int cnt = sum_quarters((int)((acc & 0xFFFFu) + (acc >> 16)));
-            if (cnt >= kout) T = cand;
+          for (int o = 16; o < 64; o <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+          if (part == 0) {
+            const float amax = top > 0x7F800000u ? __builtin_nanf("") : fmaxf(__uint_as_float(top), 1e-8f);
+            stat_s[j][1] = amax;
+            a.p.gscale[mbase + j] = amax;
+            a.p.gmean[mbase + j] = mu;
+            // sorted levels far enough apart for the rounded distances to order
+            // as the real ones: every token has |x - mean| <= amax, so a
+            // distance is below R = 2 (|mean| + amax), and gaps of at least
+            // R * 2^-19 (16 ulps of R) cannot round away
+            const float r = __fmul_rn(__fadd_rn(fabsf(mu), amax), 0x1p-18f);
+            bool ok = true;
+            float c = __fadd_rn(mu, __fmul_rn(amax, kNF4[0]));
+#pragma unroll
+            for (int l = 1; l < 16; ++l) {
+              const float n = __fadd_rn(mu, __fmul_rn(amax, kNF4[l]));
+              ok &= __fsub_rn(n, c) >= r;  // (false for any level that is not finite)
+              c = n;
+            }
+            if (!(ok && __builtin_isfinite(c))) atomicOr(&crowded_s, 1u << (j >> 6));
           }
         }
-        // the scan compares magnitudes as floats, as the reference's mask
-        // |x| >= t does: a NaN threshold selects nothing (bias 0)
-        if (part == 0) tbias_s[j] = (uint16_t)(T > 0x7C00u ? 0u : 0x8000u - T);
+        if (kout > 0 && kout < G) {
+          u16x2_t m2[TQK_MAX_G / 8];
+#pragma unroll
+          for (int i = 0; i < TQK_MAX_G / 8; ++i) {
+            const int s = 8 * i + 2 * part;  // tokens past G count as magnitude 0
+            m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
+                            (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
+            if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // (the gathered halves are packed as they come)
+          }
+          uint32_t T = 0;
+          if (kout <= 5) {
+            T = kth_largest<5>(m2, kout);
+          } else if (kout <= 8) {
+            T = kth_largest<8>(m2, kout);
+          } else {
+            for (int bit = 14; bit >= 0; --bit) {
+              const uint32_t cand = T | (1u << bit);
+              // m + (0x8000 - cand) has bit 15 set exactly when m >= cand (m, cand < 2^15)
+              const uint16_t bias = (uint16_t)(0x8000u - cand);
+              const u16x2_t bv = {bias, bias};
+              uint32_t acc = 0;  // two 16-bit counts
+#pragma unroll
+              for (int i = 0; i < TQK_MAX_G / 8; ++i)
+                acc += (__builtin_bit_cast(uint32_t, (u16x2_t)(m2[i] + bv)) >> 15) & 0x00010001u;
+              const int cnt = sum_quarters((int)((acc & 0xFFFFu) + (acc >> 16)));
+              if (cnt >= kout) T = cand;
+            }
+          }
+          // the scan compares magnitudes as floats, as the reference's mask
+          // |x| >= t does: a NaN threshold selects nothing (bias 0)
+          if (part == 0) tbias_s[j] = (uint16_t)(T > 0x7C00u ? 0u : 0x8000u - T);
+        }
       }
     }
     __syncthreads();
 
-    // ---- outlier side-list in flat (token, channel) order, one token per
-    // thread.  ocount holds cumulative counts at every TQK_OBLK-token boundary
-    // of the group (entry TQK_NOB-1 = total), so a decode block finds its
-    // entries without searching; omask_s records the stored (token, channel)
-    // positions, whose codes become the grid's zero level below.
+    // ---- outlier side-list in flat (token, channel) order, two threads per
+    // token, half of the channels each.  ocount holds cumulative counts at
+    // every TQK_OBLK-token boundary of the group (entry TQK_NOB-1 = total), so a
+    // decode block finds its entries without searching; om_row records the
+    // stored (token, channel) positions, whose codes become the grid's zero
+    // level below.
     if (kout > 0) {
+      static_assert(kEncThreads >= 2 * TQK_MAX_G, "two threads per token");
       const bool all = kout >= G;
+      constexpr int NW = D / 64;  // mask words per thread
+      const int tt = tid >> 1, w0 = NW * (tid & 1);
       // the token's outlier channels, eight at a time: magnitudes and biases
       // as packed 16-bit pairs, bit 15 of each half of m + bias is the test
       // m >= T; NaN magnitudes (m > 0x7C00, where m + 0x03FF reaches bit 15)
       // are never selected, as |x| >= t is false for them
-      uint32_t om[D / 32];
+      uint32_t om[NW];
 #pragma unroll
-      for (int k = 0; k < D / 32; ++k) om[k] = 0u;
-      if (tid < G) {
+      for (int k = 0; k < NW; ++k) om[k] = 0u;
+      if (tt < G) {
 #pragma unroll
-        for (int c8 = 0; c8 < D / 8; ++c8) {
-          const uint4 xw = *reinterpret_cast<const uint4*>(&kt_s[tid][8 * c8]);
-          const uint4 bw = *reinterpret_cast<const uint4*>(&tbias_s[8 * c8]);
+        for (int c8 = 0; c8 < D / 16; ++c8) {
+          const uint4 xw = *reinterpret_cast<const uint4*>(&kt_s[tt][32 * w0 + 8 * c8]);
+          const uint4 bw = *reinterpret_cast<const uint4*>(&tbias_s[32 * w0 + 8 * c8]);
           const uint32_t xs[4] = {xw.x, xw.y, xw.z, xw.w}, bs[4] = {bw.x, bw.y, bw.z, bw.w};
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -288,14 +406,12 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
         }
         if (all) {
 #pragma unroll
-          for (int k = 0; k < D / 32; ++k) om[k] = 0xFFFFFFFFu;
+          for (int k = 0; k < NW; ++k) om[k] = 0xFFFFFFFFu;
         }
       }
       int cnt = 0;
-      if (tid < G) {
 #pragma unroll
-        for (int k = 0; k < D / 32; ++k) cnt += __builtin_popcount(om[k]);
-      }
+      for (int k = 0; k < NW; ++k) cnt += __builtin_popcount(om[k]);
       // block exclusive scan of cnt
       int incl = cnt;
 #pragma unroll
@@ -305,33 +421,38 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
       }
       if (lane == 63) wsum_s[wv] = incl;
       __syncthreads();
-      int wofs = 0;
-      for (int w = 0; w < wv; ++w) wofs += wsum_s[w];
-      int total = 0;
-      for (int w = 0; w < kEncWaves; ++w) total += wsum_s[w];
+      int wofs = 0, total = 0;
+#pragma unroll
+      for (int w = 0; w < kEncWaves; ++w) {
+        wofs += w < wv ? wsum_s[w] : 0;
+        total += wsum_s[w];
+      }
       int off = wofs + incl - cnt;
       // token s = TQK_OBLK*k - 1 closes block k-1: its inclusive offset is the bound
-      if (tid < G && ((tid + 1) % TQK_OBLK) == 0 && (tid + 1) / TQK_OBLK <= TQK_NOB)
-        a.p.ocount[obase * TQK_NOB + (tid + 1) / TQK_OBLK - 1] = off + cnt;
+      if (tt < G && (tid & 1) && ((tt + 1) % TQK_OBLK) == 0 && (tt + 1) / TQK_OBLK <= TQK_NOB)
+        a.p.ocount[obase * TQK_NOB + (tt + 1) / TQK_OBLK - 1] = off + cnt;
       if (tid < TQK_NOB && TQK_OBLK * (tid + 1) > G) a.p.ocount[obase * TQK_NOB + tid] = total;
-      if (tid < G) {
+      if (tt < G) {
         // entries in channel order; those past the side-list's capacity are
-        // dropped (and leave their codes alone)
+        // dropped (and leave their codes alone).  A stored position's key gives
+        // way to +inf, the last bucket of the codes below.
 #pragma unroll
-        for (int k = 0; k < D / 32; ++k) {
+        for (int k = 0; k < NW; ++k) {
           uint32_t w = om[k];
           while (w) {
-            const int j = 32 * k + __builtin_ctz(w);
+            const int j = 32 * (w0 + k) + __builtin_ctz(w);
             w &= w - 1u;
-            if (off < d.outlier_cap)
-              a.p.oent[obase * d.outlier_cap + off] = (uint32_t)(tid * D + j) | ((uint32_t)kt_s[tid][j] << 16);
-            else
+            if (off < d.outlier_cap) {
+              a.p.oent[obase * d.outlier_cap + off] = (uint32_t)(tt * D + j) | ((uint32_t)kt_s[tt][j] << 16);
+              kt_s[tt][j] = 0x7C00u;
+            } else {
               om[k] &= ~(1u << (j & 31));
+            }
             ++off;
           }
         }
 #pragma unroll
-        for (int k = 0; k < D / 32; ++k) omask_s[tid][k] = om[k];
+        for (int k = 0; k < NW; ++k) om_row(tt)[w0 + k] = om[k];
       }
       if (tid == 0 && total > d.outlier_cap && a.overflow) atomicOr(a.overflow, TQK_OVF_OUTLIERS);
     } else if (tid < TQK_NOB) {
@@ -339,104 +460,129 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
     }
     __syncthreads();
 
-    // ---- codes: thread = (channel pair jp, token slice = wave); the slice's
-    // rows belong to this wave alone, so a row's code bytes replace its first
-    // D / 2 bytes right after the wave has read it.  A stored outlier takes the
-    // grid level whose value is gmean -- NF4's zero level (code 7), or code 0
-    // of a uniform grid -- so the dense part of a decode contributes gmean
-    // there and the side-list adds val - gmean; export restores the
+    // ---- codes, 64 channels at a time: a wave takes two tokens, a half-wave
+    // the 32 channel pairs of one.  The rows belong to their wave alone and
+    // 64 channels' codes are 32 bytes at or before the channels' own place, so
+    // a row's codes replace keys that have been read.  A stored outlier takes
+    // the grid level whose value is gmean -- NF4's zero level (code 7), or
+    // code 0 of a uniform grid -- so the dense part of a decode contributes
+    // gmean there and the side-list adds val - gmean; export restores the
     // reference's code.
-    for (int jp = lane; jp < D / 2; jp += 64) {
-      const int kb = d.key_bits;
-      const int per_q = (G + kEncWaves - 1) / kEncWaves;
-      const int s0 = wv * per_q, s1 = min(G, s0 + per_q);
-      const uint32_t zc = d.key_grid == 1 ? 0u : 7u;
-      const float st00 = stat_s[2 * jp][0], st01 = stat_s[2 * jp][1];
-      const float st10 = stat_s[2 * jp + 1][0], st11 = stat_s[2 * jp + 1][1];
+    const int kb = d.key_bits, half = lane >> 5, pr = lane & 31;
+    const uint32_t crowded = crowded_s;
+    for (int c0 = 0; c0 < D; c0 += 64) {
+      const int ja = c0 + 2 * pr;  // the lane's channels ja, ja + 1
+      const float st00 = stat_s[ja][0], st01 = stat_s[ja][1];
+      const float st10 = stat_s[ja + 1][0], st11 = stat_s[ja + 1][1];
+      // the wave's token pairs: t and t + 8 of a 16-token stretch (LDS rows 8
+      // apart fall on the other 32 banks)
+      auto for_pairs = [&](auto f) {
+        for (int s = wv; s < (G + 15) / 16 * 8; s += kEncWaves) {
+          const int t = (s >> 3) * 16 + (s & 7) + 8 * half;
+          f(t, t < G);
+        }
+      };
       if (d.key_grid == 1) {
         // uniform: clip(round_half_even((x - min) / scale), 0, 2^bits - 1)
         const float qmax = (float)((1 << kb) - 1);
-        for (int s = s0; s < s1; ++s) {
-          const uint32_t xx = *reinterpret_cast<const uint32_t*>(&kt_s[s][2 * jp]);
+        for_pairs([&](int t, bool in) {
+          if (!in) return;
+          const uint32_t xx = *reinterpret_cast<const uint32_t*>(&kt_s[t][ja]);
           const float r0 = __builtin_rintf(__fdiv_rn(__fsub_rn(h2f((uint16_t)xx), st00), st01));
           const float r1 = __builtin_rintf(__fdiv_rn(__fsub_rn(h2f((uint16_t)(xx >> 16)), st10), st11));
           uint32_t b0 = (uint32_t)fminf(fmaxf(r0, 0.0f), qmax);
           uint32_t b1 = (uint32_t)fminf(fmaxf(r1, 0.0f), qmax);
           if (kout > 0) {
-            const uint32_t om = omask_s[s][jp >> 4] >> (2 * (jp & 15));
-            if (om & 1u) b0 = zc;
-            if (om & 2u) b1 = zc;
+            const uint32_t om = om_row(t)[ja >> 5] >> (ja & 31);
+            if (om & 1u) b0 = 0u;
+            if (om & 2u) b1 = 0u;
           }
           // one table index per channel pair (the key row layout of tqk_common.h)
-          kc_row(s)[jp] = (uint8_t)(kb == 4 ? ((rev4(b0) << 4) | rev4(b1)) : (b0 | (b1 << kb)));
+          kc_row(t)[ja >> 1] = (uint8_t)(kb == 4 ? ((rev4(b0) << 4) | rev4(b1)) : (b0 | (b1 << kb)));
+        });
+      } else if (!((crowded >> (c0 >> 6)) & 1u)) {
+        // asym-NF4 by bucket (above): the 15 thresholds of every channel, then
+        // about 11 VALU and one LDS read a key (the argmin over 16 levels took
+        // 45: the codes were half of the keys' work)
+        __syncthreads();
+        {
+          const int c = tid & 63;
+          const float mu = stat_s[c0 + c][0], amax = stat_s[c0 + c][1];
+          const int col = (c >> 1) + 32 * (c & 1);
+          for (int k = wv; k < 15; k += kEncWaves) {
+            const uint32_t X = nf4_threshold(__fadd_rn(mu, __fmul_rn(amax, kNF4[k])),
+                                             __fadd_rn(mu, __fmul_rn(amax, kNF4[k + 1])));
+            const uint32_t e = X | (rev4((uint32_t)k) << 16) | (rev4((uint32_t)k + 1u) << 20);
+            for (int i = kNf4From[k]; i < kNf4From[k + 1]; ++i) nf_s[i][col] = e;
+          }
+          if (wv == 7) nf_s[32][col] = rev4(7u) << 16 | rev4(7u) << 20;
         }
+        __syncthreads();
+        // (a hair under 16: |x - mean| = amax stays short of bucket 32)
+        const float inv0 = 15.9995f * __builtin_amdgcn_rcpf(st01), inv1 = 15.9995f * __builtin_amdgcn_rcpf(st11);
+        // first read and second read: channel ja + half, then the other one
+        const float muA = half ? st10 : st00, invA = half ? inv1 : inv0;
+        const float muB = half ? st00 : st10, invB = half ? inv0 : inv1;
+        const uint32_t* tabA = &nf_s[0][pr + 32 * half];
+        const uint32_t* tabB = &nf_s[0][pr + 32 * (half ^ 1)];
+        for_pairs([&](int t, bool in) {
+          const uint32_t xx = *reinterpret_cast<const uint32_t*>(&kt_s[min(t, G - 1)][ja]);
+          const float x0 = h2f((uint16_t)xx), x1 = h2f((uint16_t)(xx >> 16));
+          const float xA = half ? x1 : x0, xB = half ? x0 : x1;
+          const uint32_t iA = min((uint32_t)fmaf(__fsub_rn(xA, muA), invA, 16.0f), 32u);
+          const uint32_t iB = min((uint32_t)fmaf(__fsub_rn(xB, muB), invB, 16.0f), 32u);
+          const uint32_t eA = tabA[64 * iA], eB = tabB[64 * iB];
+          const uint32_t nA = (eA >> (xA >= h2f((uint16_t)eA) ? 20 : 16)) & 15u;
+          const uint32_t nB = (eB >> (xB >= h2f((uint16_t)eB) ? 20 : 16)) & 15u;
+          if (in) kc_row(t)[ja >> 1] = (uint8_t)(half ? (nB << 4) | nA : (nA << 4) | nB);
+        });
       } else {
-        // asym-NF4 levels cent_l = mean + amax * NF4[l]
-        float c0[16], c1[16];
+        // levels too close together, or not finite: the argmin over all levels
+        // cent_l = mean + amax * NF4[l]
+        float l0[16], l1[16];
 #pragma unroll
         for (int l = 0; l < 16; ++l) {
-          c0[l] = __fadd_rn(st00, __fmul_rn(st01, kNF4[l]));
-          c1[l] = __fadd_rn(st10, __fmul_rn(st11, kNF4[l]));
+          l0[l] = __fadd_rn(st00, __fmul_rn(st01, kNF4[l]));
+          l1[l] = __fadd_rn(st10, __fmul_rn(st11, kNF4[l]));
         }
-        // With finite levels and a finite x no distance is NaN, and the
-        // argmin needs only the strict comparison.  Sorted levels far enough
-        // apart make it a count: for x >= c_l the distances x - c_l fall
-        // strictly with l (their real gaps exceed the rounding, see below)
-        // and for c_l > x they never fall, so the first argmin is the number
-        // of strict decreases d_l < d_(l-1).  Every token of the group has
-        // |x - mean| <= amax, so a distance is below R = 2 (|mean| + amax);
-        // gaps of at least R * 2^-19 (16 ulps of R) cannot round away.
-        bool lv_finite = true, spread = true;
+        bool lv_finite = true;
 #pragma unroll
-        for (int l = 0; l < 16; ++l) lv_finite &= __builtin_isfinite(c0[l]) && __builtin_isfinite(c1[l]);
-        {
-          const float r0 = __fmul_rn(__fadd_rn(fabsf(st00), st01), 0x1p-18f);
-          const float r1 = __fmul_rn(__fadd_rn(fabsf(st10), st11), 0x1p-18f);
-#pragma unroll
-          for (int l = 1; l < 16; ++l)
-            spread &= __fsub_rn(c0[l], c0[l - 1]) >= r0 && __fsub_rn(c1[l], c1[l - 1]) >= r1;
-          spread &= lv_finite;
-        }
-        for (int s = s0; s < s1; ++s) {
-          const uint32_t xx = *reinterpret_cast<const uint32_t*>(&kt_s[s][2 * jp]);
+        for (int l = 0; l < 16; ++l) lv_finite &= __builtin_isfinite(l0[l]) && __builtin_isfinite(l1[l]);
+        for_pairs([&](int t, bool in) {
+          const uint32_t xx = *reinterpret_cast<const uint32_t*>(&kt_s[min(t, G - 1)][ja]);
           const float x0 = h2f((uint16_t)xx), x1 = h2f((uint16_t)(xx >> 16));
           uint32_t b0 = 0, b1 = 0;
-          float d0 = fabsf(__fsub_rn(x0, c0[0])), d1 = fabsf(__fsub_rn(x1, c1[0]));
+          float d0 = fabsf(__fsub_rn(x0, l0[0])), d1 = fabsf(__fsub_rn(x1, l1[0]));
+          // with finite levels and a finite x no distance is NaN, and the
+          // strict comparison is all that argmin needs
           const bool fin = lv_finite && (xx & 0x7C00u) != 0x7C00u && (xx & 0x7C000000u) != 0x7C000000u;
-          if (__all(fin && spread)) {
+          if (__all(fin)) {
 #pragma unroll
             for (int l = 1; l < 16; ++l) {
-              const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
-              b0 += (e0 < d0) ? 1u : 0u;
-              b1 += (e1 < d1) ? 1u : 0u;
-              d0 = e0;
-              d1 = e1;
-            }
-          } else if (__all(fin)) {
-#pragma unroll
-            for (int l = 1; l < 16; ++l) {
-              const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
+              const float e0 = fabsf(__fsub_rn(x0, l0[l])), e1 = fabsf(__fsub_rn(x1, l1[l]));
               if (e0 < d0) { d0 = e0; b0 = l; }
               if (e1 < d1) { d1 = e1; b1 = l; }
             }
           } else {
 #pragma unroll
             for (int l = 1; l < 16; ++l) {
-              const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
+              const float e0 = fabsf(__fsub_rn(x0, l0[l])), e1 = fabsf(__fsub_rn(x1, l1[l]));
               // np.argmin: strictly smaller wins; the first NaN wins over any number
               if (e0 < d0 || (e0 != e0 && d0 == d0)) { d0 = e0; b0 = l; }
               if (e1 < d1 || (e1 != e1 && d1 == d1)) { d1 = e1; b1 = l; }
             }
           }
+          if (!in) return;
           if (kout > 0) {
-            const uint32_t om = omask_s[s][jp >> 4] >> (2 * (jp & 15));
-            if (om & 1u) b0 = zc;
-            if (om & 2u) b1 = zc;
+            const uint32_t om = om_row(t)[ja >> 5] >> (ja & 31);
+            if (om & 1u) b0 = 7u;
+            if (om & 2u) b1 = 7u;
           }
-          kc_row(s)[jp] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
-        }
+          kc_row(t)[ja >> 1] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
+        });
       }
     }
+
     __syncthreads();
     // key code rows, one 32-channel chunk (16 pair indices) per thread
     const int KROW = k_row_bytes(d.key_bits, D);
@@ -467,10 +613,10 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
   // ---- values (and PolarQuant keys) ----------------------------------------
   // kVBatch tokens at a time: their rows staged in the key tile's area, norms
   // (four threads per token, the reference's pairwise order), estimated codes
-  // (wave w: channels [NC w, NC w + NC)), the flagged ones recomputed, then the
+  // (wave w: channels [16 w, 16 w + 16), then 128 further on), the flagged ones recomputed, then the
   // rows: LE bit streams of VB-bit codes per token, or 4-token x 8-channel
   // units (the same eight fields a thread either way)
-  constexpr int VROW = D * VB / 8, NC = D / kEncWaves, NT = NC >= 32 ? 2 : 1, kVBatch = 128;
+  constexpr int VROW = D * VB / 8, NT = 1, kVBatch = 128;
   using Stage = PolarStage<D, kVBatch>;
   static_assert(kVBatch * (D + 8) * 2 % 16 == 0 &&
                 kVBatch * (D + 8) * 2 + sizeof(Stage) <= sizeof(kt_s), "value staging overflows the key tile");
@@ -513,9 +659,11 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
         }
       }
       __syncthreads();
-      for (int e0 = NC * wv; e0 < NC * wv + NC; e0 += 16 * NT) {
+      for (int e0 = 16 * wv; e0 < D; e0 += 16 * kEncWaves) {
         PiFrags<D, NT> pf;
-        load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
+        const float* pi = a.p.pi;
+        asm volatile("" : "+s"(pi));  // (loaded here, not kept over the norms' registers)
+        load_pi(pf, pi, e0, lane, bnd, (1 << VB) - 1);
         polar_codes<D, NT, VB, false, TROWS>(st, pf, &kt_s[0][0], D + 8, nb, e0, lane, bnd);
       }
       __syncthreads();
@@ -544,7 +692,8 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
 #pragma unroll
     for (int k = 0; k < VB; ++k) dst[k] = w[k];
   };
-  if (d.key_grid == 2) {
+  if (key_side) {
+    if (d.key_grid != 2) return;
     // PolarQuant keys (turboquant_pro/core.py:542-617 with kind="key"; key_bits
     // == value_bits): the value encode on the key tokens, norms to knorm; 2-
     // and 3-bit key rows are the same bit stream, 4-bit ones its bytes with
@@ -562,6 +711,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
       a.p.gmean[mbase + tid] = 0.0f;
     }
     if (tid < TQK_NOB) a.p.ocount[obase * TQK_NOB + tid] = 0;
+    return;
   }
   if (D == TQK_D && v_tiled(G, P, D, d.input_f32)) {
     polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, true, TiledRows{}, [&](int t0, int f8, uint32_t (&w)[VB]) {
@@ -587,7 +737,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group(EncodeArgs a) {
 // value codes are per-token rows.  Value norms are not bounded: the VALU
 // decode, the one that serves fp32 caches, keeps its weights in fp32.
 template <int VB, int D>
-__global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a) {
+__global__ __launch_bounds__(kF32Threads) void tqk_encode_group_f32(EncodeArgs a) {
   const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const tqk_cache_desc& d = a.d;
@@ -608,16 +758,16 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
   __shared__ __align__(16) uint16_t uv_s[kVBatch][2 * D + 8];
   __shared__ __align__(16) PolarStage<D, kVBatch> st;
   __shared__ const float* vrow_s[kVBatch];
-  __shared__ int32_t wsum_s[kEncWaves];
+  __shared__ int32_t wsum_s[kF32Waves];
 
-  for (int t = tid; t < G; t += kEncThreads)
+  for (int t = tid; t < G; t += kF32Threads)
     krow_s[t] = token_src<D, float>(a, a.p.hot_k, a.chunk_k, b, h, g * G + t);
   __syncthreads();
 
   float bnd[15];
 #pragma unroll
   for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
-  constexpr int NC = D / kEncWaves, NT = NC >= 32 ? 2 : 1;
+  constexpr int NC = D / kF32Waves, NT = NC >= 32 ? 2 : 1;
   // PolarQuant of the group's tokens, kVBatch at a time: norms (four threads
   // per token, pairwise_sumsq) and the scaled rows' fp16 pairs, estimated
   // codes, the flagged ones recomputed from the fp32 rows, the bit streams
@@ -659,12 +809,12 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
       }
       __syncthreads();
       if (st.nlist > 0) {
-        polar_fix<D, VB, false, kEncThreads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
+        polar_fix<D, VB, false, kF32Threads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
           return *reinterpret_cast<const float4*>(vrow_s[t] + dd);
         });
         __syncthreads();
       }
-      for (int f8 = tid; f8 < nb * (D / 32); f8 += kEncThreads) {
+      for (int f8 = tid; f8 < nb * (D / 32); f8 += kF32Threads) {
         uint32_t w[VB];
         pack_fields<VB>(st, f8, w);
         const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + f8 / (D / 32), P,
@@ -772,7 +922,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
       if (lane == 63) wsum_s[wv] = incl;
       __syncthreads();
       int wofs = 0, total = 0;
-      for (int w = 0; w < kEncWaves; ++w) {
+      for (int w = 0; w < kF32Waves; ++w) {
         if (w < wv) wofs += wsum_s[w];
         total += wsum_s[w];
       }
@@ -798,7 +948,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
     // ---- codes: thread = (channel pair, token slice = wave), the reference's
     // code everywhere (side-list positions included)
     const int kb = d.key_bits;
-    const int per_q = (G + kEncWaves - 1) / kEncWaves;
+    const int per_q = (G + kF32Waves - 1) / kF32Waves;
     const int s0 = wv * per_q, s1 = min(G, s0 + per_q);
     for (int jp = lane; jp < D / 2; jp += 64) {
       const float st00 = stat_s[2 * jp][0], st01 = stat_s[2 * jp][1];
@@ -849,7 +999,7 @@ __global__ __launch_bounds__(kEncThreads) void tqk_encode_group_f32(EncodeArgs a
     __syncthreads();
     // key code rows, one 32-channel chunk (16 table indices) per thread
     const int KROW = k_row_bytes(d.key_bits, D);
-    for (int idx = tid; idx < G * (D / 32); idx += kEncThreads) {
+    for (int idx = tid; idx < G * (D / 32); idx += kF32Threads) {
       const int t = idx / (D / 32), ch = idx % (D / 32);
       const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
       const uint4 f16 = *reinterpret_cast<const uint4*>(&kc_s[t][16 * ch]);
@@ -1009,18 +1159,21 @@ template <int D>
 void launch_by_vb(int vb, dim3 grid, hipStream_t st, const EncodeArgs& a) {
   if (a.d.input_f32) {
     if (vb == 2)
-      hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), grid, dim3(kF32Threads), 0, st, a);
     else if (vb == 3)
-      hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), grid, dim3(kF32Threads), 0, st, a);
     else
-      hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), grid, dim3(kEncThreads), 0, st, a);
-  } else if (vb == 2) {
-    hipLaunchKernelGGL((tqk_encode_group<2, D>), grid, dim3(kEncThreads), 0, st, a);
-  } else if (vb == 3) {
-    hipLaunchKernelGGL((tqk_encode_group<3, D>), grid, dim3(kEncThreads), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((tqk_encode_group<4, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), grid, dim3(kF32Threads), 0, st, a);
+    return;
   }
+  // a key and a value workgroup per (item, kv head), see tqk_encode_group
+  const dim3 g2(16 * ((grid.x * grid.y + 7) / 8));
+  if (vb == 2)
+    hipLaunchKernelGGL((tqk_encode_group<2, D>), g2, dim3(kEncThreads), 0, st, a);
+  else if (vb == 3)
+    hipLaunchKernelGGL((tqk_encode_group<3, D>), g2, dim3(kEncThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL((tqk_encode_group<4, D>), g2, dim3(kEncThreads), 0, st, a);
 }
 template <int D>
 void launch_by_vb(int vb, dim3 grid, hipStream_t st, const DequantArgs& a) {
@@ -1053,6 +1206,7 @@ int tqk_encode_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t 
   a.chunk_k = chunk_k;
   a.chunk_v = chunk_v;
   a.chunk_tokens = chunk_tokens;
+  a.n_items = n_items;
   a.overflow = overflow;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (d->key_grid == 0 && d->zero_point == 2 && !p->zp_mean) return TQK_EINVAL;
