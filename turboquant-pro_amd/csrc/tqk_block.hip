@@ -108,64 +108,433 @@ struct KeyBlockArgs {
   uint32_t* out_pos;
   uint16_t* out_val;
   int32_t* out_count;
-  int thr_pre;     // the thresholds were left in out_pos by tqk_key_block_thresholds
-  int codes_post;  // the 4-bit codes are written by tqk_key_block_codes4 afterwards
+  int n_chunks;  // kKbChunk-token chunks of a (b, h)
 };
 
-// The outlier thresholds of tqk_key_block ahead of it, spread over the chip:
-// one workgroup per (b, h) and 64 channels, a lane per channel and 16 waves
-// over interleaved token rows (each load one 128-byte row piece).  The same
-// search as tqk_key_block's threshold threads: T is the largest fp32
-// magnitude pattern with #{ |x_s| >= T } >= k, found two bits a pass, each
-// pass's counts exact integer sums of the 16 waves' counts.  T is left in the
-// first D entries of the (b, h)'s side-list row (out_pos), which
-// tqk_key_block reads before it writes that row.
-template <int D>
-__global__ __launch_bounds__(1024) void tqk_key_block_thresholds(KeyBlockArgs a) {
-  constexpr int W = 16;
-  const tqk_block_desc& d = a.d;
-  const int bh = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int j = blockIdx.y * 64 + lane;
-  const int S = d.tokens, f32 = d.input_f32, kout = d.outliers_per_channel;
-  const size_t base = (size_t)bh * S * D + j;
-  // Two bits a pass (bits 30..1 in pairs, then bit 0): the counts of the
-  // three candidates T | d << sh (d = 1, 2, 3) fall with d, so the largest d
-  // whose count reaches k is what two one-bit passes would pick.
-  __shared__ int cnt_s[2][3][W][64];
-  uint32_t T = 0;
-  int par = 0;
-  for (int sh = 29; sh >= -1; sh -= 2, par ^= 1) {
-    const bool two = sh >= 1;
-    const int shift = two ? sh : 0;
-    const uint32_t c1 = T | (1u << shift), c2 = T | (2u << shift), c3 = T | (3u << shift);
-    int n1 = 0, n2 = 0, n3 = 0;
-    for_tokens<D>(a.x, f32, base, w, S, W, [&](int, float xv) {
-      const uint32_t u = __float_as_uint(fabsf(xv));
-      n1 += u >= c1;
-      n2 += u >= c2;
-      n3 += u >= c3;
-    });
-    // (two count buffers: a wave that runs ahead writes the other one; the
-    // next write to this one follows the next pass's barrier)
-    cnt_s[par][0][w][lane] = n1;
-    cnt_s[par][1][w][lane] = n2;
-    cnt_s[par][2][w][lane] = n3;
-    __syncthreads();
-    int t1 = 0, t2 = 0, t3 = 0;
-#pragma unroll
-    for (int v = 0; v < W; ++v) {
-      t1 += cnt_s[par][0][v][lane];
-      t2 += cnt_s[par][1][v][lane];
-      t3 += cnt_s[par][2][v][lane];
-    }
-    const uint32_t dsel = two ? (t3 >= kout ? 3u : t2 >= kout ? 2u : t1 >= kout ? 1u : 0u)
-                              : (t1 >= kout ? 1u : 0u);
-    T |= dsel << shift;
-  }
-  if (w == 0) a.out_pos[(size_t)bh * d.outlier_cap + j] = T;
+// ---- key blocks over the chip -------------------------------------------------
+// Four kernels: tqk_key_block_stats (a workgroup per (b, h) and 16 channels:
+// zero point, scale, outlier threshold), tqk_key_block_masks (a workgroup per
+// (b, h) and 256 tokens: the outlier bits of every token and the chunk's
+// count), tqk_key_block_list (the same grid: the side-list, each chunk at the
+// offset that the counts before it give) and tqk_key_block_codes (the same
+// grid).  Until the codes are written, the (b, h)'s part of the packed output
+// holds what the first kernels hand on: D thresholds, n_chunks counts, and D
+// bits a token (KbScratch).  Bound: the stats kernel's ordered sum, 16000 tokens
+// one after another at about five cycles each, and its passes over the block.
+// One 1 x 8 x 16000 x 128 fp32 block: 3147 us with the thresholds on a workgroup
+// per 64 channels (16 passes) and statistics and side-list on one per (b, h),
+// 251 us like this.
+constexpr int kKbChunk = 256;
+constexpr int kKbTile = 512;           // tokens per LDS tile of the ordered sum
+constexpr int kKbLd = kKbTile + 4;     // tile row stride: 16 channels x 4 tokens on 64 banks
+constexpr int kKbStatThreads = 1024;
+
+struct KbScratch {
+  uint32_t* thr;     // [D]
+  uint32_t* count;   // [n_chunks]
+  uint32_t* mask;    // [S][D / 32]
+};
+__device__ __forceinline__ KbScratch kb_scratch(const KeyBlockArgs& a, int bh) {
+  const int D = a.d.head_dim;
+  uint32_t* base = reinterpret_cast<uint32_t*>(a.packed) + (size_t)bh * ((size_t)a.d.tokens * D * a.d.bits / 32);
+  return {base, base + D, base + D + a.n_chunks};
 }
 
-// one workgroup of 2 * D threads per (b, h)
+template <bool F32>
+__device__ __forceinline__ float kb_load(const void* x, size_t i) {
+  if constexpr (F32) return reinterpret_cast<const float*>(x)[i];
+  else return h2f(reinterpret_cast<const uint16_t*>(x)[i]);
+}
+
+// Statistics and thresholds of 16 channels.  A wave's load is four tokens x 16
+// channels (lane: token lane / 16, channel lane % 16).
+// Pass 1 reads the block tile by tile: minimum, maximum, a histogram of the top
+// eight magnitude bits (LDS columns of the lane's own, so atomics never share a
+// bank), and the tile transposed for wave 0, which sums it in token order (its
+// lane c: channel c) while the others read on.
+// amax = max |x - mu| is taken at the channel's two ends: rounding is monotone.
+// Passes 2 .. 4 refine the threshold by 8, 8 and 7 bits: the largest magnitude
+// pattern T with #{ |x| >= T } >= k is the k-th largest, so each pass picks the
+// bin, counted from the top, in which the k-th falls.
+template <int D, bool F32>
+__global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockArgs a) {
+  constexpr int NW = kKbStatThreads / 64, PER = kKbTile / (4 * NW);  // loads per thread and tile
+  const tqk_block_desc& d = a.d;
+  const int bh = blockIdx.x / (D / 16), c0 = 16 * (blockIdx.x % (D / 16));
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ch = lane & 15, sub = lane >> 4;
+  const int S = d.tokens, kout = d.outliers_per_channel;
+  const bool select = kout > 0 && kout < S, sum = d.key_grid == 0 && d.zero_point != 2;
+  const size_t base = (size_t)bh * S * D + c0 + ch;
+
+  __shared__ __align__(16) float tile_s[2][16][kKbLd];
+  __shared__ uint32_t hist_s[256][64];
+  __shared__ float red_s[3][NW][16];
+  __shared__ float mean_s[16];
+  __shared__ uint32_t pre_s[16];  // the threshold's bits found so far
+  __shared__ int rem_s[16];       // the rank left within them
+
+  auto clear = [&]() {
+    for (int i = tid; i < 256 * 64; i += kKbStatThreads) (&hist_s[0][0])[i] = 0u;
+  };
+  // channel wv: the bin in which the rem-th value from the top falls
+  auto pick = [&](int shift) {
+    int n[4], tot = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t* row = hist_s[255 - (4 * lane + i)];
+      n[i] = (int)(row[wv] + row[16 + wv] + row[32 + wv] + row[48 + wv]);
+      tot += n[i];
+    }
+    int incl = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    int left = rem_s[wv] - (incl - tot);
+    if (left > 0 && left <= tot) {
+      int i = 0;
+      while (left > n[i]) left -= n[i++];
+      pre_s[wv] |= (uint32_t)(255 - (4 * lane + i)) << shift;
+      rem_s[wv] = left;
+    }
+  };
+
+  if (tid < 16) {
+    pre_s[tid] = 0u;
+    rem_s[tid] = kout;
+  }
+  if (select) clear();
+  __syncthreads();
+
+  // ---- pass 1
+  float mn = __builtin_inff(), mx = -__builtin_inff(), acc = 0.0f;
+  uint32_t top = 0;
+  const int n_tiles = (S + kKbTile - 1) / kKbTile;
+  float x[PER], nx[PER];
+  auto load_tile = [&](int t0, float (&v)[PER]) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u)
+      v[u] = kb_load<F32>(a.x, base + (size_t)min(S - 1, t0 + 4 * (PER * wv + u) + sub) * D);
+  };
+  load_tile(0, x);
+  for (int ti = 0; ti < n_tiles; ++ti) {
+    const int t0 = ti * kKbTile;
+    if (ti + 1 < n_tiles) load_tile(t0 + kKbTile, nx);
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int s = 4 * (PER * wv + u) + sub;
+      const uint32_t m = __float_as_uint(fabsf(x[u]));
+      mn = fminf(mn, x[u]);  // (tokens past the end repeat the last one)
+      mx = fmaxf(mx, x[u]);
+      top = max(top, m);
+      if (sum) tile_s[ti & 1][ch][s] = x[u];
+      if (select && t0 + s < S) atomicAdd(&hist_s[m >> 23][lane], 1u);
+    }
+    __syncthreads();
+    // (the other buffer is written next; this one only after the next barrier)
+    if (sum && wv == 0) {
+      const float* row = tile_s[ti & 1][ch];
+      const int n = min(kKbTile, S - t0);
+      int s = 0;
+      for (; s + 32 <= n; s += 32) {
+        float4 v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const float4*>(row + s + 4 * u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          acc = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(acc, v[u].x), v[u].y), v[u].z), v[u].w);
+      }
+      for (; s < n; ++s) acc = __fadd_rn(acc, row[s]);
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) x[u] = nx[u];
+  }
+#pragma unroll
+  for (int o = 16; o < 64; o <<= 1) {
+    mn = fminf(mn, __shfl_xor(mn, o, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+    top = max(top, (uint32_t)__shfl_xor((int)top, o, 64));
+  }
+  if (sub == 0) {
+    red_s[0][wv][ch] = mn;
+    red_s[1][wv][ch] = mx;
+    red_s[2][wv][ch] = __uint_as_float(top);
+  }
+  if (wv == 0 && sub == 0) mean_s[ch] = acc;
+  if (select) pick(23);
+  __syncthreads();
+  if (tid < 16) {
+    for (int w = 0; w < NW; ++w) {
+      mn = fminf(mn, red_s[0][w][tid]);
+      mx = fmaxf(mx, red_s[1][w][tid]);
+      top = max(top, __float_as_uint(red_s[2][w][tid]));
+    }
+    const int j = c0 + tid;
+    const bool xnan = top > 0x7F800000u;
+    float z, sc;
+    if (d.key_grid == 1) {
+      z = xnan ? __builtin_nanf("") : mn;
+      sc = xnan ? __builtin_nanf("") : __fdiv_rn(fmaxf(__fsub_rn(mx, mn), 1e-8f), (float)((1 << d.bits) - 1));
+    } else {
+      if (d.zero_point == 2) {
+        z = a.zp[(size_t)(bh % d.n_heads) * D + j];
+      } else {
+        z = (float)((double)mean_s[tid] / (double)S);
+        if (d.zero_point == 1) z = __fmul_rn(z, dc_channel(d, j) ? 1.0f : 0.0f);
+      }
+      const float lo = fabsf(__fsub_rn(mn, z)), hi = fabsf(__fsub_rn(mx, z));
+      const bool nan = xnan || lo != lo || hi != hi;
+      sc = nan ? __builtin_nanf("") : fmaxf(fmaxf(lo, hi), 1e-8f);
+    }
+    a.scale[(size_t)bh * D + j] = sc;
+    a.zero[(size_t)bh * D + j] = z;
+    if (kout == 0 && j == 0) a.out_count[bh] = 0;
+  }
+  if (!select) return;
+
+  // ---- passes 2 .. 4 (fp16 values have no bits below the third)
+  for (int lv = 1; lv < (F32 ? 4 : 3); ++lv) {
+    const int above = 31 - 8 * lv, shift = lv == 3 ? 0 : above - 8, mask = lv == 3 ? 127 : 255;
+    __syncthreads();
+    clear();
+    const uint32_t pre = pre_s[ch] >> above;
+    __syncthreads();
+    for (int s0 = 0; s0 < S; s0 += kKbTile) {
+      float v[PER];
+      load_tile(s0, v);
+#pragma unroll
+      for (int u = 0; u < PER; ++u) {
+        const uint32_t m = __float_as_uint(fabsf(v[u]));
+        if ((m >> above) == pre && s0 + 4 * (PER * wv + u) + sub < S)
+          atomicAdd(&hist_s[(m >> shift) & mask][lane], 1u);
+      }
+    }
+    __syncthreads();
+    pick(shift);
+  }
+  __syncthreads();
+  if (tid < 16) kb_scratch(a, bh).thr[c0 + tid] = pre_s[tid];
+}
+
+// The outlier bits of 256 tokens: a lane per channel of each 64-channel piece,
+// a ballot a token; a wave takes 64 tokens and lane t keeps token t's bits.
+template <int D, bool F32>
+__global__ __launch_bounds__(kKbChunk) void tqk_key_block_masks(KeyBlockArgs a) {
+  constexpr int NC = D / 64, N = 16;
+  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = a.d.tokens;
+  const KbScratch sc = kb_scratch(a, bh);
+  const int s0 = c * kKbChunk + 64 * wv, n = min(64, S - s0);
+  __shared__ int n_s[kKbChunk / 64];
+  int cnt = 0;
+  if (n > 0) {
+#pragma unroll
+    for (int p = 0; p < NC; ++p) {
+      const float th = __uint_as_float(sc.thr[64 * p + lane]);  // (a NaN threshold selects nothing)
+      const size_t base = ((size_t)bh * S + s0) * D + 64 * p + lane;
+      uint64_t mine = 0;
+      for (int t = 0; t < n; t += N) {
+        float v[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) v[u] = kb_load<F32>(a.x, base + (size_t)min(t + u, n - 1) * D);
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+          const uint64_t m = __ballot(fabsf(v[u]) >= th);
+          mine = lane == t + u ? m : mine;
+        }
+      }
+      if (lane < n) {
+        uint32_t* dst = sc.mask + (size_t)(s0 + lane) * (D / 32) + 2 * p;
+        dst[0] = (uint32_t)mine;
+        dst[1] = (uint32_t)(mine >> 32);
+        cnt += __popcll(mine);
+      }
+    }
+  }
+  cnt = wave_sum(cnt);
+  if (lane == 0) n_s[wv] = cnt;
+  __syncthreads();
+  if (tid == 0) sc.count[c] = (uint32_t)(n_s[0] + n_s[1] + n_s[2] + n_s[3]);
+}
+
+// The side-list entries of 256 tokens in (s, j) order, one token per thread;
+// every element is one when k >= S.
+template <int D, bool F32>
+__global__ __launch_bounds__(kKbChunk) void tqk_key_block_list(KeyBlockArgs a) {
+  const tqk_block_desc& d = a.d;
+  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = d.tokens;
+  const bool all = d.outliers_per_channel >= S;
+  const KbScratch sc = kb_scratch(a, bh);
+  const int s = c * kKbChunk + tid;
+  __shared__ int sum_s[2][kKbChunk / 64];
+  // entries in the chunks before this one, and in all of them
+  int before = 0, total = 0;
+  if (all) {
+    before = c * kKbChunk * D;
+    total = S * D;
+  } else {
+    for (int i = tid; i < a.n_chunks; i += kKbChunk) {
+      const int n = (int)sc.count[i];
+      total += n;
+      before += i < c ? n : 0;
+    }
+    before = wave_sum(before);
+    total = wave_sum(total);
+    if (lane == 0) {
+      sum_s[0][wv] = before;
+      sum_s[1][wv] = total;
+    }
+    __syncthreads();
+    before = sum_s[0][0] + sum_s[0][1] + sum_s[0][2] + sum_s[0][3];
+    total = sum_s[1][0] + sum_s[1][1] + sum_s[1][2] + sum_s[1][3];
+    __syncthreads();
+  }
+  if (c == 0 && tid == 0) a.out_count[bh] = total;
+  uint32_t w[D / 32];
+  int cnt = 0;
+#pragma unroll
+  for (int k = 0; k < D / 32; ++k) {
+    w[k] = s < S ? (all ? 0xFFFFFFFFu : sc.mask[(size_t)s * (D / 32) + k]) : 0u;
+    cnt += __builtin_popcount(w[k]);
+  }
+  int incl = cnt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += v;
+  }
+  if (lane == 63) sum_s[0][wv] = incl;
+  __syncthreads();
+  int off = before + incl - cnt;
+  for (int i = 0; i < wv; ++i) off += sum_s[0][i];
+  const size_t lb = (size_t)bh * d.outlier_cap, row = ((size_t)bh * S + s) * D;
+#pragma unroll
+  for (int k = 0; k < D / 32; ++k) {
+    while (w[k] && off < d.outlier_cap) {
+      const int j = 32 * k + __builtin_ctz(w[k]);
+      w[k] &= w[k] - 1u;
+      a.out_pos[lb + off] = (uint32_t)s * D + (uint32_t)j;
+      a.out_val[lb + off] = f2h(kb_load<F32>(a.x, row + j));  // fp16, round to nearest even
+      ++off;
+    }
+  }
+}
+
+// The codes of 256 tokens.  4-bit: thread = (channel pair, token slice), the
+// levels rebuilt from the stored scale and zero point with the same arithmetic.
+// Levels that are finite and far enough apart for the rounded distances to
+// order as the real ones (gaps of at least 16 ulps of the largest distance, 2
+// (|mean| + amax)) make the first argmin the number of strict decreases from
+// level to level; the others take the comparison that also orders NaN.  2- and
+// 3-bit (uniform): one token row per thread.
+template <int D, bool F32>
+__global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) {
+  constexpr int NPR = D / 2, NS = kKbChunk / NPR, PER = kKbChunk / NS;
+  const tqk_block_desc& d = a.d;
+  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int tid = threadIdx.x, S = d.tokens;
+  const size_t base = (size_t)bh * S * D;
+  const int t0 = c * kKbChunk, t1 = min(S, t0 + kKbChunk);
+  if (d.bits != 4) {
+    const int bits = d.bits, s = t0 + tid;
+    const float qmax = (float)((1 << bits) - 1);
+    if (s >= S) return;
+    uint32_t rw[D / 8] = {0u};
+    for (int j = 0; j < D; ++j) {
+      const float xv = kb_load<F32>(a.x, base + (size_t)s * D + j);
+      const float r = __builtin_rintf(__fdiv_rn(__fsub_rn(xv, a.zero[(size_t)bh * D + j]), a.scale[(size_t)bh * D + j]));
+      put_code_ref(rw, j, bits, (uint32_t)fminf(fmaxf(r, 0.0f), qmax));
+    }
+    uint32_t* dst = reinterpret_cast<uint32_t*>(a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8));
+    for (int w = 0; w < D * bits / 32; ++w) dst[w] = rw[w];
+    return;
+  }
+  const int jp = tid % NPR, sq = tid / NPR;
+  const int s0 = min(t1, t0 + sq * PER), s1 = min(t1, s0 + PER);
+  uint8_t* out = a.packed + base / 2 + jp;
+  const size_t cj = (size_t)bh * D + 2 * jp;
+  const float sc0 = a.scale[cj], z0 = a.zero[cj], sc1 = a.scale[cj + 1], z1 = a.zero[cj + 1];
+  auto for_pairs = [&](auto f) {
+    constexpr int N = 8;
+    for (int s = s0; s < s1; s += N) {
+      float v0[N], v1[N];
+#pragma unroll
+      for (int u = 0; u < N; ++u) {
+        const size_t i = base + (size_t)min(s + u, s1 - 1) * D + 2 * jp;
+        if constexpr (F32) {
+          const float2 p = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(a.x) + i);
+          v0[u] = p.x;
+          v1[u] = p.y;
+        } else {
+          const uint32_t p = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.x) + i);
+          v0[u] = h2f((uint16_t)p);
+          v1[u] = h2f((uint16_t)(p >> 16));
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+        if (s + u < s1) f(s + u, v0[u], v1[u]);
+    }
+  };
+  if (d.key_grid == 1) {
+    for_pairs([&](int s, float x0, float x1) {
+      const float r0 = __builtin_rintf(__fdiv_rn(__fsub_rn(x0, z0), sc0));
+      const float r1 = __builtin_rintf(__fdiv_rn(__fsub_rn(x1, z1), sc1));
+      const uint32_t b0 = (uint32_t)fminf(fmaxf(r0, 0.0f), 15.0f);
+      const uint32_t b1 = (uint32_t)fminf(fmaxf(r1, 0.0f), 15.0f);
+      out[(size_t)s * (D / 2)] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
+    });
+    return;
+  }
+  float c0[16], c1[16];
+#pragma unroll
+  for (int l = 0; l < 16; ++l) {
+    c0[l] = __fadd_rn(z0, __fmul_rn(sc0, kNF4[l]));
+    c1[l] = __fadd_rn(z1, __fmul_rn(sc1, kNF4[l]));
+  }
+  const float r0 = __fmul_rn(__fadd_rn(fabsf(z0), sc0), 0x1p-18f);
+  const float r1 = __fmul_rn(__fadd_rn(fabsf(z1), sc1), 0x1p-18f);
+  // (false for levels that are not finite; every |x - mean| <= amax, so finite
+  // levels mean finite keys)
+  bool spread = __builtin_isfinite(c0[15]) && __builtin_isfinite(c1[15]);
+#pragma unroll
+  for (int l = 1; l < 16; ++l)
+    spread &= __fsub_rn(c0[l], c0[l - 1]) >= r0 && __fsub_rn(c1[l], c1[l - 1]) >= r1;
+  if (__all(spread)) {
+    for_pairs([&](int s, float x0, float x1) {
+      uint32_t b0 = 0, b1 = 0;
+      float d0 = fabsf(__fsub_rn(x0, c0[0])), d1 = fabsf(__fsub_rn(x1, c1[0]));
+#pragma unroll
+      for (int l = 1; l < 16; ++l) {
+        const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
+        b0 += (e0 < d0) ? 1u : 0u;
+        b1 += (e1 < d1) ? 1u : 0u;
+        d0 = e0;
+        d1 = e1;
+      }
+      out[(size_t)s * (D / 2)] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
+    });
+  } else {
+    for_pairs([&](int s, float x0, float x1) {
+      uint32_t b0 = 0, b1 = 0;
+      float d0 = fabsf(__fsub_rn(x0, c0[0])), d1 = fabsf(__fsub_rn(x1, c1[0]));
+#pragma unroll
+      for (int l = 1; l < 16; ++l) {
+        const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
+        // np.argmin: strictly smaller wins; the first NaN wins over any number
+        if (e0 < d0 || (e0 != e0 && d0 == d0)) { d0 = e0; b0 = l; }
+        if (e1 < d1 || (e1 != e1 && d1 == d1)) { d1 = e1; b1 = l; }
+      }
+      out[(size_t)s * (D / 2)] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
+    });
+  }
+}
+
+// The same in one workgroup of 2 * D threads per (b, h): side-list capacities
+// below head_dim, and blocks whose packed output cannot hold KbScratch (a few
+// tokens, or not at a multiple of four bytes).
 template <int D>
 __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
   constexpr int T = 2 * D;  // threads
@@ -225,15 +594,11 @@ __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
     // #{ |x_s| >= T } >= k (NaN patterns order above inf, as np.partition does)
     const int j = tid - D;
     uint32_t T = 0;
-    if (a.thr_pre) {
-      T = a.out_pos[(size_t)bh * d.outlier_cap + j];
-    } else {
-      for (int bit = 30; bit >= 0; --bit) {
-        const uint32_t cand = T | (1u << bit);
-        int cnt = 0;
-        for (int s = 0; s < S; ++s) cnt += (__float_as_uint(fabsf(X(s, j))) >= cand);
-        if (cnt >= kout) T = cand;
-      }
+    for (int bit = 30; bit >= 0; --bit) {
+      const uint32_t cand = T | (1u << bit);
+      int cnt = 0;
+      for (int s = 0; s < S; ++s) cnt += (__float_as_uint(fabsf(X(s, j))) >= cand);
+      if (cnt >= kout) T = cand;
     }
     thr_s[j] = __uint_as_float(T);
   }
@@ -254,7 +619,7 @@ __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
     }
   }
   // ---- 4-bit codes: thread = (channel pair, token slice), one byte per (token, pair)
-  else if (!a.codes_post) {
+  else {
     const int jp = tid % (D / 2), sq = tid / (D / 2);  // four token slices
     const int per = (S + 3) / 4, s0 = sq * per, s1 = min(S, s0 + per);
     uint8_t* out = a.packed + base / 2 + jp;
@@ -348,52 +713,6 @@ __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
     }
   } else if (tid == 0) {
     a.out_count[bh] = 0;
-  }
-}
-
-// The 4-bit codes of tqk_key_block over the chip: a workgroup per (b, h) and
-// 256 tokens, thread = (channel pair, token slice).  The levels are rebuilt
-// from the scale and zero point tqk_key_block stored, with its arithmetic
-// (NF4: mean + amax * level; uniform: min and step), so the codes are its.
-template <int D>
-__global__ __launch_bounds__(256) void tqk_key_block_codes4(KeyBlockArgs a) {
-  constexpr int NPR = D / 2, NS = 256 / NPR, TOK = 256, PER = TOK / NS;
-  const tqk_block_desc& d = a.d;
-  const int bh = blockIdx.x, tid = threadIdx.x, jp = tid % NPR, sq = tid / NPR;
-  const int S = d.tokens, f32 = d.input_f32;
-  const size_t base = (size_t)bh * S * D;
-  const int t0 = blockIdx.y * TOK, t1 = min(S, t0 + TOK);
-  const int s0 = min(t1, t0 + sq * PER), s1 = min(t1, s0 + PER);
-  uint8_t* out = a.packed + base / 2 + jp;
-  const size_t cj = (size_t)bh * D + 2 * jp;
-  const float sc0 = a.scale[cj], z0 = a.zero[cj], sc1 = a.scale[cj + 1], z1 = a.zero[cj + 1];
-  if (d.key_grid == 1) {
-    for_token_pairs<D>(a.x, f32, base + 2 * jp, s0, s1, [&](int s, float x0, float x1) {
-      const float r0 = __builtin_rintf(__fdiv_rn(__fsub_rn(x0, z0), sc0));
-      const float r1 = __builtin_rintf(__fdiv_rn(__fsub_rn(x1, z1), sc1));
-      const uint32_t b0 = (uint32_t)fminf(fmaxf(r0, 0.0f), 15.0f);
-      const uint32_t b1 = (uint32_t)fminf(fmaxf(r1, 0.0f), 15.0f);
-      out[(size_t)s * (D / 2)] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
-    });
-  } else {
-    float c0[16], c1[16];
-#pragma unroll
-    for (int l = 0; l < 16; ++l) {
-      c0[l] = __fadd_rn(z0, __fmul_rn(sc0, kNF4[l]));
-      c1[l] = __fadd_rn(z1, __fmul_rn(sc1, kNF4[l]));
-    }
-    for_token_pairs<D>(a.x, f32, base + 2 * jp, s0, s1, [&](int s, float x0, float x1) {
-      int b0 = 0, b1 = 0;
-      float d0 = fabsf(__fsub_rn(x0, c0[0])), d1 = fabsf(__fsub_rn(x1, c1[0]));
-#pragma unroll
-      for (int l = 1; l < 16; ++l) {
-        const float e0 = fabsf(__fsub_rn(x0, c0[l])), e1 = fabsf(__fsub_rn(x1, c1[l]));
-        // np.argmin: strictly smaller wins; the first NaN wins over any number
-        if (e0 < d0 || (e0 != e0 && d0 == d0)) { d0 = e0; b0 = l; }
-        if (e1 < d1 || (e1 != e1 && d1 == d1)) { d1 = e1; b1 = l; }
-      }
-      out[(size_t)s * (D / 2)] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
-    });
   }
 }
 
@@ -577,6 +896,39 @@ int check_block(const tqk_block_desc* d, bool key) {
   return TQK_OK;
 }
 
+// Key blocks go over the chip where the packed output has room for KbScratch
+// (dwords: 4-byte aligned) and the side-list could hold a row: 61 us at 1 x 8 x
+// 33 x 128 (fp32), 70 at 64 tokens, where one workgroup per (b, h) takes 104
+// and 277.
+template <int D, bool F32>
+void launch_key_chip(hipStream_t st, const KeyBlockArgs& a) {
+  const unsigned bh = (unsigned)(a.d.batch * a.d.n_heads), n = bh * (unsigned)a.n_chunks;
+  hipLaunchKernelGGL((tqk_key_block_stats<D, F32>), dim3(bh * (D / 16)), dim3(kKbStatThreads), 0, st, a);
+  if (a.d.outliers_per_channel > 0) {
+    if (a.d.outliers_per_channel < a.d.tokens)
+      hipLaunchKernelGGL((tqk_key_block_masks<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+    hipLaunchKernelGGL((tqk_key_block_list<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+  }
+  hipLaunchKernelGGL((tqk_key_block_codes<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+}
+template <int D>
+void launch_key(hipStream_t st, const KeyBlockArgs& a) {
+  const long long words = (long long)a.d.tokens * D * a.d.bits / 32;
+  const long long need = D + a.n_chunks + (long long)a.d.tokens * (D / 32);
+  const bool outliers = a.d.outliers_per_channel > 0;
+  const bool chip = (!outliers || (a.d.outlier_cap >= D && need <= words)) &&
+                    (reinterpret_cast<uintptr_t>(a.packed) & 3u) == 0u &&
+                    (reinterpret_cast<uintptr_t>(a.x) & 7u) == 0u &&
+                    (long long)a.d.batch * a.d.n_heads * a.n_chunks < (1LL << 31) &&
+                    (long long)a.d.tokens * D < (1LL << 31);
+  if (!chip)
+    hipLaunchKernelGGL(tqk_key_block<D>, dim3(a.d.batch * a.d.n_heads), dim3(2 * D), 0, st, a);
+  else if (a.d.input_f32)
+    launch_key_chip<D, true>(st, a);
+  else
+    launch_key_chip<D, false>(st, a);
+}
+
 // one kernel instance per (bits, head_dim)
 template <int D>
 void launch_value(int vb, dim3 grid, hipStream_t st, const ValueBlockArgs& a) {
@@ -609,39 +961,15 @@ int tqk_encode_key_block(const tqk_block_desc* d, const void* x, const float* zp
   if (!x || !packed || !scale || !zero || !out_count) return TQK_EINVAL;
   if (d->key_grid == 0 && d->zero_point == 2 && !zp) return TQK_EINVAL;
   if (d->outliers_per_channel > 0 && d->outlier_cap > 0 && (!out_pos || !out_val)) return TQK_EINVAL;
-  KeyBlockArgs a{*d, x, zp, packed, scale, zero, out_pos, out_val, out_count, 0};
-  const dim3 grid(d->batch * d->n_heads);
+  const int n_chunks = (d->tokens + kKbChunk - 1) / kKbChunk;
+  KeyBlockArgs a{*d, x, zp, packed, scale, zero, out_pos, out_val, out_count, n_chunks};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // thresholds ahead, over the chip, where the side-list row can hold them
-  if (d->outliers_per_channel > 0 && d->outliers_per_channel < d->tokens &&
-      d->outlier_cap >= d->head_dim) {
-    a.thr_pre = 1;
-    const dim3 tgrid(d->batch * d->n_heads, d->head_dim / 64);
-    if (d->head_dim == 64)
-      hipLaunchKernelGGL(tqk_key_block_thresholds<64>, tgrid, dim3(1024), 0, st, a);
-    else if (d->head_dim == 128)
-      hipLaunchKernelGGL(tqk_key_block_thresholds<128>, tgrid, dim3(1024), 0, st, a);
-    else
-      hipLaunchKernelGGL(tqk_key_block_thresholds<256>, tgrid, dim3(1024), 0, st, a);
-  }
-  // 4-bit codes afterwards, over the chip (a workgroup per 256 tokens)
-  const int n_tok_blocks = (d->tokens + 255) / 256;
-  a.codes_post = d->bits == 4 && n_tok_blocks <= 65535;
   if (d->head_dim == 64)
-    hipLaunchKernelGGL(tqk_key_block<64>, grid, dim3(128), 0, st, a);
+    launch_key<64>(st, a);
   else if (d->head_dim == 128)
-    hipLaunchKernelGGL(tqk_key_block<128>, grid, dim3(256), 0, st, a);
+    launch_key<128>(st, a);
   else
-    hipLaunchKernelGGL(tqk_key_block<256>, grid, dim3(512), 0, st, a);
-  if (a.codes_post) {
-    const dim3 cgrid(d->batch * d->n_heads, n_tok_blocks);
-    if (d->head_dim == 64)
-      hipLaunchKernelGGL(tqk_key_block_codes4<64>, cgrid, dim3(256), 0, st, a);
-    else if (d->head_dim == 128)
-      hipLaunchKernelGGL(tqk_key_block_codes4<128>, cgrid, dim3(256), 0, st, a);
-    else
-      hipLaunchKernelGGL(tqk_key_block_codes4<256>, cgrid, dim3(256), 0, st, a);
-  }
+    launch_key<256>(st, a);
   return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
 }
 

@@ -347,7 +347,7 @@ __device__ __forceinline__ void polar_fix(PolarStage<D, NTOK>& st, const float* 
     // and all add them up in order, one lane's after another (DPP)
     constexpr int CH = D < 128 ? D : 128;
     const int li = tid & 15;
-    for (int i0 = 0; i0 < n; i0 += NTH / 16) {
+    for (int i0 = 0; i0 + 4 * (tid >> 6) < n; i0 += NTH / 16) {  // (waves without a code stop)
       const int i = i0 + (tid >> 4), at = st.list[min(i, n - 1)], t = at / D, e = at % D;
       const float safe = fmaxf(st.nrm[t], 1e-30f);
       float y = 0.f;

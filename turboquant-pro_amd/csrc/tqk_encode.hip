@@ -661,9 +661,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
       __syncthreads();
       for (int e0 = 16 * wv; e0 < D; e0 += 16 * kEncWaves) {
         PiFrags<D, NT> pf;
-        const float* pi = a.p.pi;
-        asm volatile("" : "+s"(pi));  // (loaded here, not kept over the norms' registers)
-        load_pi(pf, pi, e0, lane, bnd, (1 << VB) - 1);
+        load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
         polar_codes<D, NT, VB, false, TROWS>(st, pf, &kt_s[0][0], D + 8, nb, e0, lane, bnd);
       }
       __syncthreads();
