@@ -22,12 +22,10 @@
 namespace {
 
 constexpr int kThreads = 256;
-// the fp16 group encode: eight waves; its LDS (under 80 KiB at head_dim 128) lets
+// the group encodes: eight waves; its LDS (under 80 KiB at head_dim 128) lets
 // two workgroups share a CU, four waves per SIMD
 constexpr int kEncThreads = 512;
 constexpr int kEncWaves = kEncThreads / 64;
-constexpr int kF32Threads = 256;
-constexpr int kF32Waves = kF32Threads / 64;
 
 // the order of stored codes, as PolarStage has it
 struct TokenRows { static constexpr bool value = false; };
@@ -729,14 +727,24 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
 
 // ---------------------------------------------------------------------------
 // Quantize-on-flush of an fp32 cache (input_f32): the same codes, stats and
-// side-list as the fp16 encode, in the same NumPy operation order, from fp32
-// rows read through L1/L2 (an fp32 group does not fit the LDS key tile).  The
-// side-list positions keep the reference's codes (argmin on the fp32 value);
-// value codes are per-token rows.  Value norms are not bounded: the VALU
-// decode, the one that serves fp32 caches, keeps its weights in fp32.
+// side-list as the fp16 encode, in the same NumPy operation order, with key and
+// value workgroups as there.  The keys go 64 channels at a time through an LDS
+// tile; a token's side-list bits are collected over the 64-channel pieces and its
+// entries written at the end.  The side-list positions keep the reference's
+// codes (argmin on the fp32 value); value codes are per-token rows.  Value norms
+// are not bounded: the VALU decode, the one that serves fp32 caches, keeps its
+// weights in fp32.  4 sequences x 5000 tokens x 8 heads x 128: 607 us with one
+// 256-thread workgroup per (group, head) reading the keys through L1 and L2 in
+// every phase, 226 us like this.
+__constant__ static const uint8_t kNf4Pair[32] = {0, 0, 0, 1,  1,  1,  1,  2,  2,  3,  3,  4,  4,  5,  6,  6,
+                                                  7, 8, 9, 9, 10, 11, 11, 12, 12, 13, 13, 14, 14, 14, 14, 14};
+
 template <int VB, int D>
-__global__ __launch_bounds__(kF32Threads) void tqk_encode_group_f32(EncodeArgs a) {
-  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+__global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group_f32(EncodeArgs a) {
+  const int unit = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
+  const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
+  if (unit >= a.n_items * a.d.n_kv_heads) return;
+  const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const tqk_cache_desc& d = a.d;
   const int b = a.items[2 * item], g = a.items[2 * item + 1];
@@ -745,171 +753,254 @@ __global__ __launch_bounds__(kF32Threads) void tqk_encode_group_f32(EncodeArgs a
   const int kout = d.outliers_per_channel;
   const size_t mbase = ((size_t)slot * Hkv + h) * D;
   const size_t obase = (size_t)slot * Hkv + h;
-  constexpr int kVBatch = 64;  // tokens per value batch: four threads each
+  constexpr int kVBatch = 128;  // tokens per value batch: four threads each
   constexpr int VROW = D * VB / 8;
+  constexpr int LD = 68;        // key tile row stride: eight tokens x eight channels nearly on 64 banks
 
-  __shared__ const float* krow_s[TQK_MAX_G];                // source row of each key token
-  __shared__ float stat_s[D][2];                             // (mean, amax) or (min, scale)
-  __shared__ float thr_s[D];                                 // outlier magnitude threshold
-  __shared__ __align__(16) uint8_t kc_s[TQK_MAX_G][D / 2];   // table index per (token, channel pair)
-  // scaled rows of a value batch as fp16 pairs (high halves, then low ones)
-  __shared__ __align__(16) uint16_t uv_s[kVBatch][2 * D + 8];
-  __shared__ __align__(16) PolarStage<D, kVBatch> st;
-  __shared__ const float* vrow_s[kVBatch];
-  __shared__ int32_t wsum_s[kF32Waves];
-
-  for (int t = tid; t < G; t += kF32Threads)
-    krow_s[t] = token_src<D, float>(a, a.p.hot_k, a.chunk_k, b, h, g * G + t);
-  __syncthreads();
-
-  float bnd[15];
-#pragma unroll
-  for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
-  constexpr int NC = D / kF32Waves, NT = NC >= 32 ? 2 : 1;
-  // PolarQuant of the group's tokens, kVBatch at a time: norms (four threads
-  // per token, pairwise_sumsq) and the scaled rows' fp16 pairs, estimated
-  // codes, the flagged ones recomputed from the fp32 rows, the bit streams
-  auto polar_phase = [&](const void* ring, const void* chunk, float* nout, uint8_t* rows, bool reversed) {
-    for (int t0 = 0; t0 < G; t0 += kVBatch) {
-      const int nb = min(kVBatch, G - t0);
-      if (tid == 0) st.nlist = 0;
-      const int tt = tid >> 2, q = tid & 3;
-      if (tt < nb) {
-        const int t = g * G + t0 + tt;
-        const float* sp = token_src<D, float>(a, ring, chunk, b, h, t);
-        if (q == 0) vrow_s[tt] = sp;
-        const float2* src = reinterpret_cast<const float2*>(sp);
-        float x0[D / 8], x1[D / 8];
-        uint32_t any = 0;
-#pragma unroll
-        for (int m = 0; m < D / 8; ++m) {
-          const float2 w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
-          x0[m] = w2.x;
-          x1[m] = w2.y;
-          any |= __float_as_uint(w2.x) | __float_as_uint(w2.y);
-        }
-        any |= __shfl_xor(any, 1, 4);
-        any |= __shfl_xor(any, 2, 4);
-        const float ss = pairwise_sumsq<D>(x0, x1, q);
-        const float nrm = __builtin_sqrtf(ss);
-        const bool zero = (any & 0x7FFFFFFFu) == 0u;
-        polar_stage_row<D>(&uv_s[tt][0], x0, x1, q, zero ? 0.f : kPiScale * __builtin_amdgcn_rcpf(nrm));
-        if (q == 0) {
-          polar_token(st, tt, ss, nrm, zero, 1.0f / (kPiScale * kPiScale));
-          nout[page_row(a.p.block_table, d.max_pages_per_seq, b, t, P, d.n_pages, h)] = nrm;
-        }
-      }
-      __syncthreads();
-      for (int e0 = NC * wv; e0 < NC * wv + NC; e0 += 16 * NT) {
-        PiFrags<D, NT> pf;
-        load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
-        polar_codes<D, NT, VB, true, false>(st, pf, &uv_s[0][0], 2 * D + 8, nb, e0, lane, bnd);
-      }
-      __syncthreads();
-      if (st.nlist > 0) {
-        polar_fix<D, VB, false, kF32Threads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
-          return *reinterpret_cast<const float4*>(vrow_s[t] + dd);
-        });
-        __syncthreads();
-      }
-      for (int f8 = tid; f8 < nb * (D / 32); f8 += kF32Threads) {
-        uint32_t w[VB];
-        pack_fields<VB>(st, f8, w);
-        const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + f8 / (D / 32), P,
-                                    d.n_pages, h);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(rows + row * VROW) + VB * (f8 % (D / 32));
-#pragma unroll
-        for (int k = 0; k < VB; ++k) dst[k] = reversed ? __builtin_bswap32(__builtin_bitreverse32(w[k])) : w[k];
-      }
-      __syncthreads();
-    }
+  struct KeyLds {
+    float tile[TQK_MAX_G][LD];      // 64 channels; then a row's 32 code bytes at its start
+    uint32_t om[TQK_MAX_G][D / 32]; // side-list bits of every token
+    float lev[16][64];              // NF4 levels of the channels, (channel / 2) + 32 (channel % 2)
+    float stat[64][2];              // (mean, amax) or (min, scale)
+    float thr[64];
+    uint32_t crowded;
+    int32_t wsum[kEncWaves];
+    uint8_t pair[32];
   };
+  struct ValueLds {
+    uint16_t uv[kVBatch][2 * D + 8];  // scaled rows as fp16 pairs (high halves, then low ones)
+    PolarStage<D, kVBatch> st;
+    const float* row[kVBatch];
+  };
+  union Lds {
+    KeyLds k;
+    ValueLds v;
+  };
+  __shared__ __align__(16) uint8_t lds_s[sizeof(Lds)];
 
-  if (d.key_grid != 2) {
-    auto X = [&](int s, int j) { return krow_s[s][j]; };
-    // ---- per-channel statistics, thread j: channel j
-    if (tid < D) {
-      const int j = tid;
-      float st0, st1;
-      if (d.key_grid == 1) {
-        float mn = X(0, j), mx = mn;
-        bool nan = (mn != mn);
-        for (int s = 1; s < G; ++s) {
-          const float xv = X(s, j);
-          nan |= (xv != xv);
-          mn = fminf(mn, xv);
-          mx = fmaxf(mx, xv);
-        }
-        st1 = nan ? __builtin_nanf("") : __fdiv_rn(fmaxf(__fsub_rn(mx, mn), 1e-8f), (float)((1 << d.key_bits) - 1));
-        st0 = nan ? __builtin_nanf("") : mn;
-      } else {
+  if (key_side && d.key_grid != 2) {
+    KeyLds& L = reinterpret_cast<Lds*>(lds_s)->k;
+    const int kb = d.key_bits;
+    const bool all = kout >= G;
+    if (tid < 32) L.pair[tid] = kNf4Pair[tid];
+    for (int c0 = 0; c0 < D; c0 += 64) {
+      // ---- 64 channels of the group's keys
+      if (tid == 0) L.crowded = 0u;
+      for (int idx = tid; idx < G * 16; idx += kEncThreads) {
+        const int t = idx >> 4, c = idx & 15;
+        *reinterpret_cast<float4*>(&L.tile[t][4 * c]) =
+            reinterpret_cast<const float4*>(token_src<D, float>(a, a.p.hot_k, a.chunk_k, b, h, g * G + t) + c0)[c];
+      }
+      __syncthreads();
+      // the zero point, a sum in token order
+      if (tid < 64 && d.key_grid != 1) {
+        const int j = c0 + tid;
         float mu;
         if (d.zero_point == 2) {
           mu = a.p.zp_mean[((size_t)g * Hkv + h) * D + j];
         } else {
           float acc = 0.0f;
-          for (int s = 0; s < G; ++s) acc = __fadd_rn(acc, X(s, j));
+          int s = 0;
+          for (; s + 16 <= G; s += 16) {
+            float x[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) x[u] = L.tile[s + u][tid];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) acc = __fadd_rn(acc, x[u]);
+          }
+          for (; s < G; ++s) acc = __fadd_rn(acc, L.tile[s][tid]);
           mu = (float)((double)acc / (double)G);
           if (d.zero_point == 1) mu = __fmul_rn(mu, ((d.dc_mask[j >> 5] >> (j & 31)) & 1u) ? 1.0f : 0.0f);
         }
-        float amax = 0.0f;
-        bool nan = (mu != mu);
-        for (int s = 0; s < G; ++s) {
-          const float dv = fabsf(__fsub_rn(X(s, j), mu));
-          nan |= (dv != dv);
-          amax = fmaxf(amax, dv);
-        }
-        st0 = mu;
-        st1 = nan ? __builtin_nanf("") : fmaxf(amax, 1e-8f);
+        L.stat[tid][0] = mu;
       }
-      stat_s[j][0] = st0;
-      stat_s[j][1] = st1;
-      a.p.gscale[mbase + j] = st1;
-      a.p.gmean[mbase + j] = st0;
-      // outlier threshold: the k-th largest |x| of the channel as the largest
-      // fp32 magnitude pattern T with #{ |x_s| >= T } >= k (NaN patterns order
-      // above inf, as np.partition places NaN last); the k <= 8 largest are
-      // kept directly, otherwise a bitwise search
-      if (kout > 0 && kout < G) {
-        uint32_t T = 0;
-        if (kout <= 8) {
-          uint32_t top[8];
+      // Channel ends and outlier thresholds, eight channels a wave, eight lanes
+      // a channel with every eighth token.  amax = max |x - mean| is taken at
+      // the ends (rounding is monotone).  The threshold is the k-th largest |x|
+      // as the largest fp32 magnitude pattern T with #{ |x_s| >= T } >= k (NaN
+      // patterns order above inf, as np.partition places NaN last): for k <= 8
+      // every lane's eight largest, merged; otherwise a bitwise search.
+      {
+        const int cl = 8 * wv + (lane & 7), part = lane >> 3;
+        float mn = __builtin_inff(), mx = -__builtin_inff();
+        uint32_t top[8];
 #pragma unroll
-          for (int i = 0; i < 8; ++i) top[i] = 0u;
-          for (int s = 0; s < G; ++s) {
-            uint32_t v = __float_as_uint(fabsf(X(s, j)));
+        for (int i = 0; i < 8; ++i) top[i] = 0u;
+        auto insert = [&](uint32_t v) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const uint32_t hi = max(top[i], v);
-              v = min(top[i], v);
-              top[i] = hi;
-            }
+          for (int i = 0; i < 8; ++i) {
+            const uint32_t hi = max(top[i], v);
+            v = min(top[i], v);
+            top[i] = hi;
           }
+        };
+        for (int s = part; s < G; s += 8) {
+          const float x = L.tile[s][cl];
+          mn = fminf(mn, x);
+          mx = fmaxf(mx, x);
+          insert(__float_as_uint(fabsf(x)));
+        }
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) {
+          mn = fminf(mn, __shfl_xor(mn, o, 64));
+          mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+          uint32_t other[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) other[i] = (uint32_t)__shfl_xor((int)top[i], o, 64);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) insert(other[i]);
+        }
+        const bool xnan = top[0] > 0x7F800000u;
+        uint32_t T = 0;
+        if (kout > 0 && kout <= 8) {
 #pragma unroll
           for (int i = 0; i < 8; ++i)
             if (i == kout - 1) T = top[i];
-        } else {
+        } else if (kout > 8 && kout < G) {
           for (int bit = 30; bit >= 0; --bit) {
             const uint32_t cand = T | (1u << bit);
             int cnt = 0;
-            for (int s = 0; s < G; ++s) cnt += __float_as_uint(fabsf(X(s, j))) >= cand ? 1 : 0;
+            for (int s = part; s < G; s += 8) cnt += __float_as_uint(fabsf(L.tile[s][cl])) >= cand ? 1 : 0;
+            cnt += __shfl_xor(cnt, 8, 64);
+            cnt += __shfl_xor(cnt, 16, 64);
+            cnt += __shfl_xor(cnt, 32, 64);
             if (cnt >= kout) T = cand;
           }
         }
-        thr_s[j] = __uint_as_float(T);  // a NaN threshold selects nothing, as |x| >= NaN
+        __syncthreads();  // the means
+        if (part == 0) {
+          L.thr[cl] = __uint_as_float(T);  // a NaN threshold selects nothing, as |x| >= NaN
+          float st0, st1;
+          if (d.key_grid == 1) {
+            st0 = xnan ? __builtin_nanf("") : mn;
+            st1 = xnan ? __builtin_nanf("")
+                       : __fdiv_rn(fmaxf(__fsub_rn(mx, mn), 1e-8f), (float)((1 << d.key_bits) - 1));
+          } else {
+            st0 = L.stat[cl][0];
+            const float lo = fabsf(__fsub_rn(mn, st0)), hi = fabsf(__fsub_rn(mx, st0));
+            st1 = xnan || lo != lo || hi != hi ? __builtin_nanf("") : fmaxf(fmaxf(lo, hi), 1e-8f);
+            // levels finite and far enough apart, as in the fp16 encode
+            const float r = __fmul_rn(__fadd_rn(fabsf(st0), st1), 0x1p-18f);
+            bool ok = true;
+            float c = __fadd_rn(st0, __fmul_rn(st1, kNF4[0]));
+            L.lev[0][(cl >> 1) + 32 * (cl & 1)] = c;
+#pragma unroll
+            for (int l = 1; l < 16; ++l) {
+              const float n = __fadd_rn(st0, __fmul_rn(st1, kNF4[l]));
+              ok &= __fsub_rn(n, c) >= r;
+              c = n;
+              L.lev[l][(cl >> 1) + 32 * (cl & 1)] = c;
+            }
+            // (normalised keys must not overflow: amax well inside fp32's range)
+            if (!(ok && __builtin_isfinite(c) && st1 < 0x1p100f && fabsf(st0) < 0x1p100f)) atomicOr(&L.crowded, 1u);
+          }
+          L.stat[cl][0] = st0;
+          L.stat[cl][1] = st1;
+          a.p.gscale[mbase + c0 + cl] = st1;
+          a.p.gmean[mbase + c0 + cl] = st0;
+        }
       }
+      __syncthreads();
+      // side-list bits, two threads per token, 32 channels each
+      if (kout > 0 && (tid >> 1) < G) {
+        const int t = tid >> 1, hf = tid & 1;
+        uint32_t m = 0;
+#pragma unroll
+        for (int c4 = 0; c4 < 8; ++c4) {
+          const float4 x = *reinterpret_cast<const float4*>(&L.tile[t][32 * hf + 4 * c4]);
+          const float4 th = *reinterpret_cast<const float4*>(&L.thr[32 * hf + 4 * c4]);
+          m |= (fabsf(x.x) >= th.x ? 1u : 0u) << (4 * c4);
+          m |= (fabsf(x.y) >= th.y ? 2u : 0u) << (4 * c4);
+          m |= (fabsf(x.z) >= th.z ? 4u : 0u) << (4 * c4);
+          m |= (fabsf(x.w) >= th.w ? 8u : 0u) << (4 * c4);
+        }
+        L.om[t][c0 / 32 + hf] = all ? 0xFFFFFFFFu : m;
+      }
+      __syncthreads();
+      // codes: a wave takes two tokens, a half-wave the 32 channel pairs of
+      // one; a row's 32 code bytes replace its first keys once they are read
+      const int half = lane >> 5, pr = lane & 31;
+      const float st00 = L.stat[2 * pr][0], st01 = L.stat[2 * pr][1];
+      const float st10 = L.stat[2 * pr + 1][0], st11 = L.stat[2 * pr + 1][1];
+      auto for_pairs = [&](auto code) {
+        for (int s = wv; s < (G + 1) / 2; s += kEncWaves) {
+          const int t = 2 * s + half;
+          const float2 xx = *reinterpret_cast<const float2*>(&L.tile[min(t, G - 1)][2 * pr]);
+          const uint32_t byte = code(xx.x, xx.y);
+          if (t < G) reinterpret_cast<uint8_t*>(&L.tile[t][0])[pr] = (uint8_t)byte;
+        }
+      };
+      if (d.key_grid == 1) {
+        const float qmax = (float)((1 << kb) - 1);
+        for_pairs([&](float x0, float x1) {
+          const float r0 = __builtin_rintf(__fdiv_rn(__fsub_rn(x0, st00), st01));
+          const float r1 = __builtin_rintf(__fdiv_rn(__fsub_rn(x1, st10), st11));
+          const uint32_t b0 = (uint32_t)fminf(fmaxf(r0, 0.0f), qmax);
+          const uint32_t b1 = (uint32_t)fminf(fmaxf(r1, 0.0f), qmax);
+          return kb == 4 ? ((rev4(b0) << 4) | rev4(b1)) : (b0 | (b1 << kb));
+        });
+      } else if (L.crowded == 0u) {
+        // by bucket: two neighbouring levels, the nearer one (the first on a tie)
+        const float inv0 = 15.9995f / st01, inv1 = 15.9995f / st11;
+        auto nearer = [&](float x, float mu, float inv, int col) {
+          const uint32_t i = min((uint32_t)fmaf(__fsub_rn(x, mu), inv, 16.0f), 31u);
+          const uint32_t k = L.pair[i];
+          const float lo = L.lev[k][col], hi = L.lev[k + 1][col];
+          return k + (fabsf(__fsub_rn(x, hi)) < fabsf(__fsub_rn(x, lo)) ? 1u : 0u);
+        };
+        for_pairs([&](float x0, float x1) {
+          const uint32_t b0 = nearer(x0, st00, inv0, pr), b1 = nearer(x1, st10, inv1, pr + 32);
+          return (rev4(b0) << 4) | rev4(b1);
+        });
+      } else {
+        for_pairs([&](float x0, float x1) {
+          uint32_t b0 = 0, b1 = 0;
+          float d0 = fabsf(__fsub_rn(x0, L.lev[0][pr])), d1 = fabsf(__fsub_rn(x1, L.lev[0][pr + 32]));
+#pragma unroll
+          for (int l = 1; l < 16; ++l) {
+            const float e0 = fabsf(__fsub_rn(x0, L.lev[l][pr])), e1 = fabsf(__fsub_rn(x1, L.lev[l][pr + 32]));
+            // np.argmin: strictly smaller wins; the first NaN wins over any number
+            if (e0 < d0 || (e0 != e0 && d0 == d0)) { d0 = e0; b0 = l; }
+            if (e1 < d1 || (e1 != e1 && d1 == d1)) { d1 = e1; b1 = l; }
+          }
+          return (rev4(b0) << 4) | rev4(b1);
+        });
+      }
+      __syncthreads();
+      // key code rows, one 32-channel chunk (16 table indices) per thread
+      const int KROW = k_row_bytes(kb, D);
+      for (int idx = tid; idx < G * 2; idx += kEncThreads) {
+        const int t = idx >> 1, ch = c0 / 32 + (idx & 1);
+        const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
+        const uint4 f16 = *reinterpret_cast<const uint4*>(&L.tile[t][4 * (idx & 1)]);
+        if (kb == 4) {
+          *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
+        } else {
+          const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
+          uint32_t o[3] = {0u, 0u, 0u};
+          for (int i = 0; i < 16; ++i) {
+            const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
+            const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
+            o[w] |= f << sh;
+            if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
+          }
+          uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
+          for (int w = 0; w < kb; ++w) dst[w] = o[w];
+        }
+      }
+      __syncthreads();  // the tile is the next channels'
     }
-    __syncthreads();
-
-    // ---- outlier side-list in flat (token, channel) order, one token per
-    // thread (the cumulative counts at every TQK_OBLK-token boundary as the
-    // fp16 encode writes them)
+    // ---- the side-list in flat (token, channel) order, two threads per token
+    // (cumulative counts at every TQK_OBLK-token boundary as the fp16 encode)
     if (kout > 0) {
-      const bool all = kout >= G;
+      constexpr int NW = D / 64;
+      const int tt = tid >> 1, w0 = NW * (tid & 1);
+      uint32_t om[NW];
       int cnt = 0;
-      if (tid < G) {
-        const float* row = krow_s[tid];
-        for (int j = 0; j < D; ++j) cnt += (all || fabsf(row[j]) >= thr_s[j]) ? 1 : 0;
+#pragma unroll
+      for (int k = 0; k < NW; ++k) {
+        om[k] = tt < G ? L.om[tt][w0 + k] : 0u;
+        cnt += __builtin_popcount(om[k]);
       }
       int incl = cnt;
 #pragma unroll
@@ -917,23 +1008,26 @@ __global__ __launch_bounds__(kF32Threads) void tqk_encode_group_f32(EncodeArgs a
         const int v = __shfl_up(incl, o, 64);
         if (lane >= o) incl += v;
       }
-      if (lane == 63) wsum_s[wv] = incl;
+      if (lane == 63) L.wsum[wv] = incl;
       __syncthreads();
       int wofs = 0, total = 0;
-      for (int w = 0; w < kF32Waves; ++w) {
-        if (w < wv) wofs += wsum_s[w];
-        total += wsum_s[w];
+#pragma unroll
+      for (int w = 0; w < kEncWaves; ++w) {
+        wofs += w < wv ? L.wsum[w] : 0;
+        total += L.wsum[w];
       }
       int off = wofs + incl - cnt;
-      if (tid < G && ((tid + 1) % TQK_OBLK) == 0 && (tid + 1) / TQK_OBLK <= TQK_NOB)
-        a.p.ocount[obase * TQK_NOB + (tid + 1) / TQK_OBLK - 1] = off + cnt;
+      if (tt < G && (tid & 1) && ((tt + 1) % TQK_OBLK) == 0 && (tt + 1) / TQK_OBLK <= TQK_NOB)
+        a.p.ocount[obase * TQK_NOB + (tt + 1) / TQK_OBLK - 1] = off + cnt;
       if (tid < TQK_NOB && TQK_OBLK * (tid + 1) > G) a.p.ocount[obase * TQK_NOB + tid] = total;
-      if (tid < G && cnt > 0) {
-        const float* row = krow_s[tid];
-        for (int j = 0; j < D && off < d.outlier_cap; ++j) {
-          const float xv = row[j];
-          if (all || fabsf(xv) >= thr_s[j]) {
-            a.p.oent[obase * d.outlier_cap + off] = (uint32_t)(tid * D + j) | ((uint32_t)f2h(xv) << 16);
+      if (cnt > 0) {
+        const float* row = token_src<D, float>(a, a.p.hot_k, a.chunk_k, b, h, g * G + tt);
+#pragma unroll
+        for (int k = 0; k < NW; ++k) {
+          while (om[k] && off < d.outlier_cap) {
+            const int j = 32 * (w0 + k) + __builtin_ctz(om[k]);
+            om[k] &= om[k] - 1u;
+            a.p.oent[obase * d.outlier_cap + off] = (uint32_t)(tt * D + j) | ((uint32_t)f2h(row[j]) << 16);
             ++off;
           }
         }
@@ -942,83 +1036,82 @@ __global__ __launch_bounds__(kF32Threads) void tqk_encode_group_f32(EncodeArgs a
     } else if (tid < TQK_NOB) {
       a.p.ocount[obase * TQK_NOB + tid] = 0;
     }
+    return;
+  }
 
-    // ---- codes: thread = (channel pair, token slice = wave), the reference's
-    // code everywhere (side-list positions included)
-    const int kb = d.key_bits;
-    const int per_q = (G + kF32Waves - 1) / kF32Waves;
-    const int s0 = wv * per_q, s1 = min(G, s0 + per_q);
-    for (int jp = lane; jp < D / 2; jp += 64) {
-      const float st00 = stat_s[2 * jp][0], st01 = stat_s[2 * jp][1];
-      const float st10 = stat_s[2 * jp + 1][0], st11 = stat_s[2 * jp + 1][1];
-      if (d.key_grid == 1) {
-        const float qmax = (float)((1 << kb) - 1);
-        for (int s = s0; s < s1; ++s) {
-          const float2 xx = *reinterpret_cast<const float2*>(krow_s[s] + 2 * jp);
-          const float r0 = __builtin_rintf(__fdiv_rn(__fsub_rn(xx.x, st00), st01));
-          const float r1 = __builtin_rintf(__fdiv_rn(__fsub_rn(xx.y, st10), st11));
-          const uint32_t b0 = (uint32_t)fminf(fmaxf(r0, 0.0f), qmax);
-          const uint32_t b1 = (uint32_t)fminf(fmaxf(r1, 0.0f), qmax);
-          kc_s[s][jp] = (uint8_t)(kb == 4 ? ((rev4(b0) << 4) | rev4(b1)) : (b0 | (b1 << kb)));
-        }
-      } else {
-        float c0[16], c1[16];
+  ValueLds& L = reinterpret_cast<Lds*>(lds_s)->v;
+  PolarStage<D, kVBatch>& st = L.st;
+  float bnd[15];
 #pragma unroll
-        for (int l = 0; l < 16; ++l) {
-          c0[l] = __fadd_rn(st00, __fmul_rn(st01, kNF4[l]));
-          c1[l] = __fadd_rn(st10, __fmul_rn(st11, kNF4[l]));
-        }
-        for (int s = s0; s < s1; ++s) {
-          const float2 xx = *reinterpret_cast<const float2*>(krow_s[s] + 2 * jp);
-          uint32_t b0 = 0, b1 = 0;
-          float d0 = fabsf(__fsub_rn(xx.x, c0[0])), d1 = fabsf(__fsub_rn(xx.y, c1[0]));
-#pragma unroll
-          for (int l = 1; l < 16; ++l) {
-            const float e0 = fabsf(__fsub_rn(xx.x, c0[l])), e1 = fabsf(__fsub_rn(xx.y, c1[l]));
-            // np.argmin: strictly smaller wins; the first NaN wins over any number
-            if (e0 < d0 || (e0 != e0 && d0 == d0)) { d0 = e0; b0 = l; }
-            if (e1 < d1 || (e1 != e1 && d1 == d1)) { d1 = e1; b1 = l; }
-          }
-          kc_s[s][jp] = (uint8_t)((rev4(b0) << 4) | rev4(b1));
-        }
-      }
-    }
-  } else {
-    // PolarQuant keys: the value encode on the key tokens, norms to knorm; key
-    // rows as the fp16 encode writes them (4-bit bytes bit-reversed)
-    polar_phase(a.p.hot_k, a.chunk_k, a.p.knorm, a.p.kcodes, VB == 4);
+  for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
+  // PolarQuant of the group's tokens, kVBatch at a time: norms (four threads
+  // per token, pairwise_sumsq) and the scaled rows' fp16 pairs, estimated
+  // codes, the flagged ones recomputed from the fp32 rows, the bit streams
+  const void* ring = key_side ? a.p.hot_k : a.p.hot_v;
+  const void* chunk = key_side ? a.chunk_k : a.chunk_v;
+  float* nout = key_side ? a.p.knorm : a.p.vnorm;
+  uint8_t* rows = key_side ? a.p.kcodes : a.p.vcodes;
+  const bool reversed = key_side && VB == 4;  // PolarQuant key rows, as the fp16 encode writes them
+  if (key_side) {
     if (tid < D) {
       a.p.gscale[mbase + tid] = 1.0f;
       a.p.gmean[mbase + tid] = 0.0f;
     }
     if (tid < TQK_NOB) a.p.ocount[obase * TQK_NOB + tid] = 0;
   }
-  if (d.key_grid != 2) {
-    __syncthreads();
-    // key code rows, one 32-channel chunk (16 table indices) per thread
-    const int KROW = k_row_bytes(d.key_bits, D);
-    for (int idx = tid; idx < G * (D / 32); idx += kF32Threads) {
-      const int t = idx / (D / 32), ch = idx % (D / 32);
-      const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t, P, d.n_pages, h);
-      const uint4 f16 = *reinterpret_cast<const uint4*>(&kc_s[t][16 * ch]);
-      if (d.key_bits == 4) {
-        *reinterpret_cast<uint4*>(a.p.kcodes + row * KROW + 16 * ch) = f16;
-      } else {
-        const int kb = d.key_bits;
-        const uint32_t fw[4] = {f16.x, f16.y, f16.z, f16.w};
-        uint32_t o[3] = {0u, 0u, 0u};
-        for (int i = 0; i < 16; ++i) {
-          const uint32_t f = (fw[i >> 2] >> (8 * (i & 3))) & 0xFFu;
-          const int bo = 2 * kb * i, w = bo >> 5, sh = bo & 31;
-          o[w] |= f << sh;
-          if (sh + 2 * kb > 32) o[w + 1] |= f >> (32 - sh);
-        }
-        uint32_t* dst = reinterpret_cast<uint32_t*>(a.p.kcodes + row * KROW + 4 * kb * ch);
-        for (int w = 0; w < kb; ++w) dst[w] = o[w];
+  for (int t0 = 0; t0 < G; t0 += kVBatch) {
+    const int nb = min(kVBatch, G - t0);
+    if (tid == 0) st.nlist = 0;
+    const int tt = tid >> 2, q = tid & 3;
+    if (tt < nb) {
+      const int t = g * G + t0 + tt;
+      const float* sp = token_src<D, float>(a, ring, chunk, b, h, t);
+      if (q == 0) L.row[tt] = sp;
+      const float2* src = reinterpret_cast<const float2*>(sp);
+      float x0[D / 8], x1[D / 8];
+      uint32_t any = 0;
+#pragma unroll
+      for (int m = 0; m < D / 8; ++m) {
+        const float2 w2 = src[4 * m + q];  // channels 8m + 2q, 8m + 2q + 1
+        x0[m] = w2.x;
+        x1[m] = w2.y;
+        any |= __float_as_uint(w2.x) | __float_as_uint(w2.y);
+      }
+      any |= __shfl_xor(any, 1, 4);
+      any |= __shfl_xor(any, 2, 4);
+      const float ss = pairwise_sumsq<D>(x0, x1, q);
+      const float nrm = __builtin_sqrtf(ss);
+      const bool zero = (any & 0x7FFFFFFFu) == 0u;
+      polar_stage_row<D>(&L.uv[tt][0], x0, x1, q, zero ? 0.f : kPiScale * __builtin_amdgcn_rcpf(nrm));
+      if (q == 0) {
+        polar_token(st, tt, ss, nrm, zero, 1.0f / (kPiScale * kPiScale));
+        nout[page_row(a.p.block_table, d.max_pages_per_seq, b, t, P, d.n_pages, h)] = nrm;
       }
     }
+    __syncthreads();
+    for (int e0 = 16 * wv; e0 < D; e0 += 16 * kEncWaves) {
+      PiFrags<D, 1> pf;
+      load_pi(pf, a.p.pi, e0, lane, bnd, (1 << VB) - 1);
+      polar_codes<D, 1, VB, true, false>(st, pf, &L.uv[0][0], 2 * D + 8, nb, e0, lane, bnd);
+    }
+    __syncthreads();
+    if (st.nlist > 0) {
+      polar_fix<D, VB, false, kEncThreads>(st, a.p.pi, nb, tid, bnd, [&](int t, int dd) {
+        return *reinterpret_cast<const float4*>(L.row[t] + dd);
+      });
+      __syncthreads();
+    }
+    for (int f8 = tid; f8 < nb * (D / 32); f8 += kEncThreads) {
+      uint32_t w[VB];
+      pack_fields<VB>(st, f8, w);
+      const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + t0 + f8 / (D / 32), P,
+                                  d.n_pages, h);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(rows + row * VROW) + VB * (f8 % (D / 32));
+#pragma unroll
+      for (int k = 0; k < VB; ++k) dst[k] = reversed ? __builtin_bswap32(__builtin_bitreverse32(w[k])) : w[k];
+    }
+    __syncthreads();
   }
-  polar_phase(a.p.hot_v, a.chunk_v, a.p.vnorm, a.p.vcodes, false);
 }
 
 
@@ -1155,23 +1248,22 @@ __global__ __launch_bounds__(kThreads) void tqk_dequant_group(DequantArgs a) {
 // one kernel instance per (value bits, head_dim)
 template <int D>
 void launch_by_vb(int vb, dim3 grid, hipStream_t st, const EncodeArgs& a) {
-  if (a.d.input_f32) {
-    if (vb == 2)
-      hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), grid, dim3(kF32Threads), 0, st, a);
-    else if (vb == 3)
-      hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), grid, dim3(kF32Threads), 0, st, a);
-    else
-      hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), grid, dim3(kF32Threads), 0, st, a);
-    return;
-  }
   // a key and a value workgroup per (item, kv head), see tqk_encode_group
   const dim3 g2(16 * ((grid.x * grid.y + 7) / 8));
-  if (vb == 2)
+  if (a.d.input_f32) {
+    if (vb == 2)
+      hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), g2, dim3(kEncThreads), 0, st, a);
+    else if (vb == 3)
+      hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), g2, dim3(kEncThreads), 0, st, a);
+    else
+      hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), g2, dim3(kEncThreads), 0, st, a);
+  } else if (vb == 2) {
     hipLaunchKernelGGL((tqk_encode_group<2, D>), g2, dim3(kEncThreads), 0, st, a);
-  else if (vb == 3)
+  } else if (vb == 3) {
     hipLaunchKernelGGL((tqk_encode_group<3, D>), g2, dim3(kEncThreads), 0, st, a);
-  else
+  } else {
     hipLaunchKernelGGL((tqk_encode_group<4, D>), g2, dim3(kEncThreads), 0, st, a);
+  }
 }
 template <int D>
 void launch_by_vb(int vb, dim3 grid, hipStream_t st, const DequantArgs& a) {
