@@ -245,6 +245,19 @@ int tqk_dequant_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t
                        const int32_t* items, float* kout, float* vout, void* stream);
 
 /*
+ * Every cached token of `batch` sequences as dense keys and values kout, vout
+ * [batch][n_kv_heads][max_len][head_dim]: the coded groups reconstructed as
+ * tqk_dequant_groups does, the hot window as it is held, each rounded to the
+ * output type (out_type 0: fp32, 1: fp16, 2: bf16; to nearest even).  seq_lens
+ * [batch] i32 (device), every entry in [1, max_len]; rows past a sequence's
+ * length are not written.  The dense K/V of the reference's HF layer
+ * (turboquant_pro/hf_cache.py:205-214).
+ */
+int tqk_dequant_dense(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,
+                      const int32_t* seq_lens, int32_t max_len, int32_t out_type, void* kout,
+                      void* vout, void* stream);
+
+/*
  * Stateless block quantizers: one (B, H, S, D) block, every (b, h) pair one
  * quantization group of S tokens (any S >= 1), fp16 or fp32 input, outputs in
  * the reference containers' layouts.  The plugin / block-store path

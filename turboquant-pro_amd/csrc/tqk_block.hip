@@ -850,29 +850,38 @@ struct ValueDequantArgs {
   float* out;
 };
 
-// one thread per token: y = vcent[code]; x_e = sequential over j of y_j * Pi[j][e]; x * norm
+// 64 tokens per workgroup: y = vcent[code] staged in LDS (a thread takes 32 codes),
+// x_e = sequential over j of y_j * Pi[j][e] (rotate_rows), times the norm
 template <int VB, int D>
-__global__ __launch_bounds__(kKbThreads) void tqk_value_block_dequant(ValueDequantArgs a) {
+__global__ __launch_bounds__(kKbThreads, 2) void tqk_value_block_dequant(ValueDequantArgs a) {
   constexpr int VROW = D * VB / 8;
   const tqk_block_desc& d = a.d;
-  const size_t n = (size_t)d.batch * d.n_heads * d.tokens;
-  const size_t t = (size_t)blockIdx.x * kKbThreads + threadIdx.x;
-  if (t >= n) return;
-  const uint8_t* vr = a.packed + t * VROW;
-  float y[D];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const size_t n = (size_t)d.batch * d.n_heads * d.tokens, tok0 = (size_t)blockIdx.x * kVbTokens;
+  const int nb = (int)(n - tok0 < (size_t)kVbTokens ? n - tok0 : (size_t)kVbTokens);
+  __shared__ __align__(16) float y_s[kVbTokens][D];
+  __shared__ float nrm_s[kVbTokens];
+  __shared__ float cent_s[16];
+  if (tid < nb) nrm_s[tid] = a.norms[tok0 + tid];
+  if (tid >= 64 && tid < 64 + (1 << VB)) cent_s[tid - 64] = a.vcent[tid - 64];
+  __syncthreads();
+  for (int i = tid; i < nb * (D / 32); i += kKbThreads) {
+    const int t = i / (D / 32), c32 = i % (D / 32);
+    const uint8_t* src = a.packed + (tok0 + t) * VROW + 4 * VB * c32;
+    uint32_t w[VB];
+    __builtin_memcpy(w, src, sizeof(w));  // (a row may start at any byte)
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    const int bitpos = j * VB;
-    const uint32_t w = vr[bitpos >> 3] | ((uint32_t)vr[min((bitpos >> 3) + 1, VROW - 1)] << 8);
-    y[j] = a.vcent[(w >> (bitpos & 7)) & ((1u << VB) - 1)];
+    for (int k = 0; k < 32; k += 4)
+      *reinterpret_cast<float4*>(&y_s[t][32 * c32 + k]) =
+          make_float4(cent_s[stream_code<VB>(w, k)], cent_s[stream_code<VB>(w, k + 1)],
+                      cent_s[stream_code<VB>(w, k + 2)], cent_s[stream_code<VB>(w, k + 3)]);
   }
-  const float nrm = a.norms[t];
-  float* o = a.out + t * D;
-  for (int e = 0; e < D; ++e) {
-    float x = 0.f;
-#pragma unroll
-    for (int j = 0; j < D; ++j) x = __fadd_rn(x, __fmul_rn(y[j], a.pi[j * D + e]));
-    o[e] = __fmul_rn(x, nrm);
+  __syncthreads();
+  for (int e0 = 16 * wv; e0 < D; e0 += 16 * (kKbThreads / 64)) {
+    const int e = e0 + (lane & 15);
+    rotate_rows<D>(a.pi, y_s, nb, e, lane, [&](int t, float x) {
+      a.out[(tok0 + t) * D + e] = __fmul_rn(x, nrm_s[t]);
+    });
   }
 }
 
@@ -1016,7 +1025,7 @@ int tqk_dequant_value_block(const tqk_block_desc* d, const uint8_t* packed, cons
   if (!packed || !norms || !pi || !vcent || !out) return TQK_EINVAL;
   const size_t n = (size_t)d->batch * d->n_heads * d->tokens;
   ValueDequantArgs a{*d, packed, norms, pi, vcent, out};
-  const dim3 grid((unsigned)((n + kKbThreads - 1) / kKbThreads));
+  const dim3 grid((unsigned)((n + kVbTokens - 1) / kVbTokens));
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (d->head_dim == 64)
     launch_value<64>(d->bits, grid, st, a);

@@ -123,6 +123,97 @@ __device__ __forceinline__ void add_row_dpp(float& y, const float (&f)[8]) {
   if constexpr (K + 1 < NL) add_row_dpp<K + 1, NL>(y, f);
 }
 
+// y0 += u_a[d] * col[d], y1 += u_b[d] * col[d] for d = 8K .. 8K + 7 and on to d =
+// 8 NL - 1, each product and sum separately rounded, in d order; u_a[d] lives in
+// register d % 8 of lane d / 8 of the 16-lane row.  Plain operators, so that the
+// broadcast folds into the multiply as its DPP operand: only for units built
+// with -ffp-contract=off.
+template <int K, int NL, int N>
+__device__ __forceinline__ void rotate_row_dpp(float& y0, float& y1, const float (&ua)[8], const float (&ub)[8],
+                                               const float (&col)[N]) {
+  static_assert(NL <= 16 && 8 * NL <= N, "a chunk spans at most one 16-lane row");
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const float p0 = dpp_row_bcast<K>(ua[r]) * col[8 * K + r];
+    const float p1 = dpp_row_bcast<K>(ub[r]) * col[8 * K + r];
+    y0 = y0 + p0;
+    y1 = y1 + p1;
+  }
+  if constexpr (K + 1 < NL) rotate_row_dpp<K + 1, NL>(y0, y1, ua, ub, col);
+}
+
+// PolarQuant reconstruction before the norm: x_e = sum over j, in order, of
+// y_j * pi[j][e], every product and sum separately rounded (turboquant_pro/
+// core.py:619-654), of nb <= 64 rows in LDS for the channel e of this lane;
+// store(token, x_e) takes the results.  Bound by its 2 D VALU operations a
+// value: a lane keeps column e of pi, a 16-lane row takes one token of a step
+// and broadcasts its values by DPP.  Rows longer than 128 channels go in
+// 128-channel chunks, every step's sums carried on.  All 64 lanes run it.
+template <int D, typename Store>
+__device__ __forceinline__ void rotate_rows(const float* __restrict__ pi, const float (*y_s)[D], int nb, int e,
+                                            int lane, Store store) {
+  constexpr int CH = D < 128 ? D : 128;
+  const int rt = lane >> 4, lc = (lane & 15) % (CH / 8);
+  auto load_y = [&](int t, int c, float (&u)[8]) {
+    const float4* r = reinterpret_cast<const float4*>(&y_s[min(t, nb - 1)][CH * c + 8 * lc]);
+    const float4 a = r[0], b = r[1];
+    u[0] = a.x; u[1] = a.y; u[2] = a.z; u[3] = a.w;
+    u[4] = b.x; u[5] = b.y; u[6] = b.z; u[7] = b.w;
+  };
+  auto load_col = [&](int c, float (&col)[CH]) {
+#pragma unroll
+    for (int k = 0; k < CH; ++k) col[k] = pi[(size_t)(CH * c + k) * D + e];
+  };
+  if constexpr (D <= 128) {
+    float col[CH];
+    load_col(0, col);
+    for (int j0 = 0; j0 < nb; j0 += 8) {
+      float ua[8], ub[8];
+      load_y(j0 + rt, 0, ua);
+      load_y(j0 + 4 + rt, 0, ub);
+      float y0 = 0.f, y1 = 0.f;
+      rotate_row_dpp<0, CH / 8>(y0, y1, ua, ub, col);
+      // keeps the sums out of the conditional stores: sunk into them, the
+      // multiplies would leave their broadcasts behind as separate moves
+      asm volatile("" : "+v"(y0), "+v"(y1));
+      if (j0 + rt < nb) store(j0 + rt, y0);
+      if (j0 + 4 + rt < nb) store(j0 + 4 + rt, y1);
+    }
+  } else {
+    float ya[8], yb[8];
+#pragma unroll
+    for (int st = 0; st < 8; ++st) ya[st] = yb[st] = 0.f;
+    for (int c = 0; c < D / CH; ++c) {
+      float col[CH];
+      load_col(c, col);
+#pragma unroll
+      for (int st = 0; st < 8; ++st) {
+        if (8 * st < nb) {
+          float ua[8], ub[8];
+          load_y(8 * st + rt, c, ua);
+          load_y(8 * st + 4 + rt, c, ub);
+          rotate_row_dpp<0, CH / 8>(ya[st], yb[st], ua, ub, col);
+          asm volatile("" : "+v"(ya[st]), "+v"(yb[st]));
+        }
+      }
+    }
+#pragma unroll
+    for (int st = 0; st < 8; ++st) {
+      if (8 * st + rt < nb) store(8 * st + rt, ya[st]);
+      if (8 * st + 4 + rt < nb) store(8 * st + 4 + rt, yb[st]);
+    }
+  }
+}
+
+// code i of VB dwords holding a 32-code bit stream
+template <int VB>
+__device__ __forceinline__ uint32_t stream_code(const uint32_t (&w)[VB], int i) {
+  const int bit = VB * i;
+  uint32_t c = w[bit >> 5] >> (bit & 31);
+  if ((bit & 31) + VB > 32) c |= w[(bit >> 5) + 1] << (32 - (bit & 31));
+  return c & ((1u << VB) - 1u);
+}
+
 // ---------------------------------------------------------------------------
 // PolarQuant codes.  The code of a rotated channel is #{ boundaries < y_e } for
 // the reference's y_e: the sum over d, in order, of u_d * pi[e][d], every

@@ -1154,95 +1154,193 @@ __global__ __launch_bounds__(kThreads) void tqk_append_hot_kernel(HotArgs a) {
   }
 }
 
+constexpr int kDqTokens = 64;  // tokens per reconstruction workgroup
+
 struct DequantArgs {
   tqk_cache_desc d;
   tqk_cache_ptrs p;
-  const int32_t* items;
-  float* kout;
-  float* vout;
+  const int32_t* items;     // (b, g) pairs of the groups, or nullptr: every token of every sequence
+  const int32_t* seq_lens;  // without items: [batch] lengths
+  int chunks;               // kDqTokens-token chunks of a group; without items, of a sequence
+  int max_len;              // without items: rows of a sequence in kout / vout
+  void* kout;
+  void* vout;
 };
 
-// grid (n_items, Hkv), one token per thread: reconstruct keys (grid value then
-// the fp16 outlier overwrite) and values ((cent[code] @ Pi) * norm, NumPy order).
-template <int VB, int D>
-__global__ __launch_bounds__(kThreads) void tqk_dequant_group(DequantArgs a) {
+// a reconstructed fp32 value in the output's type, rounded to nearest even (the
+// barrier keeps a product before it from being rounded to fp16 directly)
+__device__ __forceinline__ void put_as(float* o, float x) { *o = x; }
+__device__ __forceinline__ void put_as(_Float16* o, float x) {
+  asm volatile("" : "+v"(x));
+  *o = (_Float16)x;
+}
+__device__ __forceinline__ void put_as(__bf16* o, float x) { *o = (__bf16)x; }
+
+// Keys and values of 64 tokens of one kv head: keys as grid value, then the fp16
+// outlier overwrite; values ((cent[code] @ Pi) * norm, NumPy order), PolarQuant
+// keys likewise; hot tokens (without items) converted.  Bound: the 2 D VALU
+// operations of every rotated value (rotate_rows).  One token per thread with Pi
+// from memory, a workgroup per group, took 260 us for 224 group-heads of 256
+// tokens (head_dim 128), and a dense prefill of 2 x 4000 tokens x 8 heads (encode,
+// this, and torch's transposes, concatenation and conversion) 503 us; written
+// in place in the output's type it takes 191 us.
+template <int VB, int D, typename T>
+__global__ __launch_bounds__(kThreads, 2) void tqk_dequant_tokens(DequantArgs a) {
   constexpr int VROW = D * VB / 8;
-  const int item = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const tqk_cache_desc& d = a.d;
-  const int b = a.items[2 * item], g = a.items[2 * item + 1];
+  const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int u = blockIdx.x / a.chunks, c = blockIdx.x % a.chunks;
   const int G = d.group_tokens, P = d.page_tokens, Hkv = d.n_kv_heads;
+  const int cpg = (G + kDqTokens - 1) / kDqTokens;  // chunks per group
+  int b, g, t0;        // t0: first token of the chunk in its group
+  T *ko, *vo;          // the chunk's first output rows
+  if (a.items) {
+    b = a.items[2 * u];
+    g = a.items[2 * u + 1];
+    t0 = c * kDqTokens;
+    const size_t row = ((size_t)u * Hkv + h) * G + t0;
+    ko = static_cast<T*>(a.kout) + row * D;
+    vo = static_cast<T*>(a.vout) + row * D;
+  } else {
+    b = u;
+    g = c / cpg;
+    t0 = (c % cpg) * kDqTokens;
+    const int L = a.seq_lens[b], ng = n_groups_of(L, d.hot_window, G);
+    const size_t base = ((size_t)b * Hkv + h) * a.max_len;
+    const int max_cold = n_groups_of(a.max_len, d.hot_window, G) * cpg;
+    if (c >= max_cold) {
+      // the hot window
+      const int s0 = ng * G + (c - max_cold) * kDqTokens, n = min(kDqTokens, L - s0);
+      const size_t ring = ((size_t)b * Hkv + h) * d.hot_ring;
+      for (int i = tid; i < n * D; i += kThreads) {
+        const int s = s0 + i / D, j = i % D;
+        const size_t src = (ring + s % d.hot_ring) * D + j, dst = (base + s) * D + j;
+        if (d.input_f32) {
+          put_as(static_cast<T*>(a.kout) + dst, static_cast<const float*>(a.p.hot_k)[src]);
+          put_as(static_cast<T*>(a.vout) + dst, static_cast<const float*>(a.p.hot_v)[src]);
+        } else {
+          put_as(static_cast<T*>(a.kout) + dst, h2f(static_cast<const uint16_t*>(a.p.hot_k)[src]));
+          put_as(static_cast<T*>(a.vout) + dst, h2f(static_cast<const uint16_t*>(a.p.hot_v)[src]));
+        }
+      }
+      return;
+    }
+    if (g >= ng) return;
+    ko = static_cast<T*>(a.kout) + (base + g * G + t0) * D;
+    vo = static_cast<T*>(a.vout) + (base + g * G + t0) * D;
+  }
+  const int nb = min(kDqTokens, G - t0);
   const int slot = a.p.group_table[(size_t)b * d.max_groups_per_seq + g];
-  const size_t mbase = ((size_t)slot * Hkv + h) * D;
-  float* ko = a.kout + ((size_t)item * Hkv + h) * G * D;
-  float* vo = a.vout + ((size_t)item * Hkv + h) * G * D;
-  if (tid < G) {
-    const size_t row = page_row(a.p.block_table, d.max_pages_per_seq, b, g * G + tid, P, d.n_pages, h);
+  const size_t mbase = ((size_t)slot * Hkv + h) * D, obase = (size_t)slot * Hkv + h;
+
+  __shared__ __align__(16) float y_s[kDqTokens][D];
+  __shared__ float nrm_s[2][kDqTokens];  // key norms (PolarQuant), value norms
+  __shared__ int row_s[kDqTokens];       // row of every token in the head's pages
+  __shared__ float cent_s[16];
+  if (tid < nb) {
+    const int t = g * G + t0 + tid;
+    const int phys = a.p.block_table[(size_t)b * d.max_pages_per_seq + t / P];
+    row_s[tid] = phys * P + t % P;
+    const size_t row = (size_t)h * d.n_pages * P + row_s[tid];
+    nrm_s[0][tid] = d.key_grid == 2 ? a.p.knorm[row] : 0.f;
+    nrm_s[1][tid] = a.p.vnorm[row];
+  }
+  if (tid >= 64 && tid < 64 + (1 << VB)) cent_s[tid - 64] = a.p.vcent[tid - 64];
+  __syncthreads();
+  const size_t head = (size_t)h * d.n_pages * P;
+
+  // centroids of the chunk's rows: a thread takes 32 codes (VB dwords), 32
+  // channels of a token
+  auto rows_to_lds = [&](const uint8_t* rows, bool reversed) {
+    for (int i = tid; i < nb * (D / 32); i += kThreads) {
+      const int t = i / (D / 32), c32 = i % (D / 32);
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(rows + (head + row_s[t]) * VROW) + VB * c32;
+      uint32_t w[VB];
+#pragma unroll
+      for (int k = 0; k < VB; ++k) w[k] = reversed ? __builtin_bswap32(__builtin_bitreverse32(src[k])) : src[k];
+#pragma unroll
+      for (int k = 0; k < 32; k += 4)
+        *reinterpret_cast<float4*>(&y_s[t][32 * c32 + k]) =
+            make_float4(cent_s[stream_code<VB>(w, k)], cent_s[stream_code<VB>(w, k + 1)],
+                        cent_s[stream_code<VB>(w, k + 2)], cent_s[stream_code<VB>(w, k + 3)]);
+    }
+  };
+  auto rotate_out = [&](T* out, const float* nrm) {
+    for (int e0 = 16 * wv; e0 < D; e0 += 16 * (kThreads / 64)) {
+      const int e = e0 + (lane & 15);
+      rotate_rows<D>(a.p.pi, y_s, nb, e, lane, [&](int t, float x) {
+        put_as(out + (size_t)t * D + e, __fmul_rn(x, nrm[t]));
+      });
+    }
+  };
+
+  if (d.key_grid == 2) {
+    // PolarQuant keys (key_bits == value_bits): (cent[code] @ Pi) * norm
+    rows_to_lds(a.p.kcodes, VB == 4);
+    __syncthreads();
+    rotate_out(ko, nrm_s[0]);
+    __syncthreads();
+  } else {
+    // four channels (two table indices) a thread
     const int kb = d.key_bits, KROW = k_row_bytes(kb, D);
-    uint32_t rw[D / 8];
-    const uint32_t* kr = reinterpret_cast<const uint32_t*>(a.p.kcodes + row * KROW);
-    for (int w = 0; w < KROW / 4; ++w) rw[w] = kr[w];
-    if (d.key_grid == 2) {
-      // PolarQuant keys: (cent[code] @ Pi) * norm, as the values below
-      float yk[D];
-      for (int jj = 0; jj < D / 2; ++jj) {
-        const uint32_t f = k_pair_index(rw, kb, jj);
-        yk[2 * jj] = a.p.vcent[k_code_even(f, kb)];
-        yk[2 * jj + 1] = a.p.vcent[k_code_odd(f, kb)];
+    for (int i = tid; i < nb * (D / 4); i += kThreads) {
+      const int t = i / (D / 4), j = 4 * (i % (D / 4));
+      const uint8_t* src = a.p.kcodes + (head + row_s[t]) * KROW;
+      uint32_t f[2];
+      if (kb == 4) {
+        const uint32_t two = *reinterpret_cast<const uint16_t*>(src + j / 2);
+        f[0] = two & 0xFFu;
+        f[1] = two >> 8;
+      } else {
+        // bits kb * j .. of the row's stream (the 32-channel chunks follow on)
+        const int bit = kb * j;
+        const uint32_t v = ((uint32_t)src[bit >> 3] | (uint32_t)src[min((bit >> 3) + 1, KROW - 1)] << 8) >> (bit & 7);
+        f[0] = v & ((1u << (2 * kb)) - 1u);
+        f[1] = (v >> (2 * kb)) & ((1u << (2 * kb)) - 1u);
       }
-      const float kn = a.p.knorm[row];
-      for (int e = 0; e < D; ++e) {
-        float x = 0.f;
+      const float4 sc = *reinterpret_cast<const float4*>(a.p.gscale + mbase + j);
+      const float4 mu = *reinterpret_cast<const float4*>(a.p.gmean + mbase + j);
+      T* o = ko + (size_t)t * D + j;
+      put_as(o, __fadd_rn(__fmul_rn(sc.x, key_level(d.key_grid, k_code_even(f[0], kb))), mu.x));
+      put_as(o + 1, __fadd_rn(__fmul_rn(sc.y, key_level(d.key_grid, k_code_odd(f[0], kb))), mu.y));
+      put_as(o + 2, __fadd_rn(__fmul_rn(sc.z, key_level(d.key_grid, k_code_even(f[1], kb))), mu.z));
+      put_as(o + 3, __fadd_rn(__fmul_rn(sc.w, key_level(d.key_grid, k_code_odd(f[1], kb))), mu.w));
+    }
+  }
+  if (D == TQK_D && v_tiled(G, P, D, d.input_f32)) {
+    // unit (lg, c8) of a 16-token tile: tokens 4 lg .. + 3 x channels 8 c8 .. + 7
+    for (int i = tid; i < nb * (D / 32); i += kThreads) {
+      const int tile = i >> 6, lg = (i >> 4) & 3, c8 = i & 15;
+      const uint32_t* src = reinterpret_cast<const uint32_t*>(
+          a.p.vcodes + (head + row_s[16 * tile]) * VROW + v_unit_offset(lg, c8, VROW));
+      uint32_t w[VB];
 #pragma unroll
-        for (int j = 0; j < D; ++j) x = __fadd_rn(x, __fmul_rn(yk[j], a.p.pi[j * D + e]));
-        ko[(size_t)tid * D + e] = __fmul_rn(x, kn);
-      }
-    } else {
-      for (int jj = 0; jj < D / 2; ++jj) {
-        const uint32_t f = k_pair_index(rw, kb, jj);
-        const int j0 = 2 * jj, j1 = 2 * jj + 1;
-        ko[(size_t)tid * D + j0] =
-            __fadd_rn(__fmul_rn(a.p.gscale[mbase + j0], key_level(d.key_grid, k_code_even(f, kb))), a.p.gmean[mbase + j0]);
-        ko[(size_t)tid * D + j1] =
-            __fadd_rn(__fmul_rn(a.p.gscale[mbase + j1], key_level(d.key_grid, k_code_odd(f, kb))), a.p.gmean[mbase + j1]);
+      for (int k = 0; k < VB; ++k) w[k] = src[k];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int n = 0; n < 8; n += 4)
+          *reinterpret_cast<float4*>(&y_s[16 * tile + 4 * lg + t][8 * c8 + n]) =
+              make_float4(cent_s[stream_code<VB>(w, 4 * n + t)], cent_s[stream_code<VB>(w, 4 * n + 4 + t)],
+                          cent_s[stream_code<VB>(w, 4 * n + 8 + t)], cent_s[stream_code<VB>(w, 4 * n + 12 + t)]);
       }
     }
-    float y[D];
-    if (D == TQK_D && v_tiled(G, P, D, d.input_f32)) {
-      // unit (lg, c) of the token's 16-token tile; tile rows start at row - (t % 16)
-      const int tt = (g * G + tid) % 16;
-      const uint8_t* tile = a.p.vcodes + (row - tt) * VROW;
-      const int lg = tt >> 2, uu = tt & 3;
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const uint8_t* un = tile + v_unit_offset(lg, j >> 3, VROW);
-        const int bit = v_unit_bit(uu, j & 7, VB);
-        const uint32_t w = un[bit >> 3] | ((uint32_t)un[min((bit >> 3) + 1, VROW / 4 - 1)] << 8);
-        y[j] = a.p.vcent[(w >> (bit & 7)) & ((1u << VB) - 1)];
-      }
-    } else {
-      const uint8_t* vr = a.p.vcodes + row * VROW;
-#pragma unroll
-      for (int j = 0; j < D; ++j) {
-        const int bitpos = j * VB;
-        uint32_t w = vr[bitpos >> 3] | ((uint32_t)vr[min((bitpos >> 3) + 1, VROW - 1)] << 8);
-        y[j] = a.p.vcent[(w >> (bitpos & 7)) & ((1u << VB) - 1)];
-      }
-    }
-    const float nrm = a.p.vnorm[row];
-    for (int e = 0; e < D; ++e) {
-      float x = 0.f;
-#pragma unroll
-      for (int j = 0; j < D; ++j) x = __fadd_rn(x, __fmul_rn(y[j], a.p.pi[j * D + e]));
-      vo[(size_t)tid * D + e] = __fmul_rn(x, nrm);
-    }
+  } else {
+    rows_to_lds(a.p.vcodes, false);
   }
   __syncthreads();
-  const size_t obase = (size_t)slot * Hkv + h;
-  const int no = min(a.p.ocount[obase * TQK_NOB + TQK_NOB - 1], d.outlier_cap);
-  for (int e = tid; e < no; e += kThreads) {
-    const uint32_t ent = a.p.oent[obase * d.outlier_cap + e];
-    ko[ent & 0xFFFFu] = h2f((uint16_t)(ent >> 16));
+  if (d.key_grid != 2 && d.outliers_per_channel > 0) {
+    // the chunk's side-list entries (its bounds are 32-token blocks)
+    const int32_t* oc = a.p.ocount + obase * TQK_NOB;
+    const int cap = d.outlier_cap, q = t0 / TQK_OBLK;
+    const int lo = min(q > 0 ? oc[q - 1] : 0, cap);
+    const int hi = min(oc[min(q + kDqTokens / TQK_OBLK, TQK_NOB) - 1], cap);
+    for (int e = lo + tid; e < hi; e += kThreads) {
+      const uint32_t ent = a.p.oent[obase * cap + e];
+      put_as(ko + (int)(ent & 0xFFFFu) - t0 * D, h2f((uint16_t)(ent >> 16)));
+    }
   }
+  rotate_out(vo, nrm_s[1]);
 }
 
 // one kernel instance per (value bits, head_dim)
@@ -1265,14 +1363,25 @@ void launch_by_vb(int vb, dim3 grid, hipStream_t st, const EncodeArgs& a) {
     hipLaunchKernelGGL((tqk_encode_group<4, D>), g2, dim3(kEncThreads), 0, st, a);
   }
 }
-template <int D>
-void launch_by_vb(int vb, dim3 grid, hipStream_t st, const DequantArgs& a) {
+template <int D, typename T>
+void launch_dequant(int vb, dim3 grid, hipStream_t st, const DequantArgs& a) {
   if (vb == 2)
-    hipLaunchKernelGGL((tqk_dequant_group<2, D>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((tqk_dequant_tokens<2, D, T>), grid, dim3(kThreads), 0, st, a);
   else if (vb == 3)
-    hipLaunchKernelGGL((tqk_dequant_group<3, D>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((tqk_dequant_tokens<3, D, T>), grid, dim3(kThreads), 0, st, a);
   else
-    hipLaunchKernelGGL((tqk_dequant_group<4, D>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((tqk_dequant_tokens<4, D, T>), grid, dim3(kThreads), 0, st, a);
+}
+template <typename T>
+int launch_dequant(dim3 grid, void* stream, const DequantArgs& a) {
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (a.d.head_dim == 64)
+    launch_dequant<64, T>(a.d.value_bits, grid, st, a);
+  else if (a.d.head_dim == 128)
+    launch_dequant<128, T>(a.d.value_bits, grid, st, a);
+  else
+    launch_dequant<256, T>(a.d.value_bits, grid, st, a);
+  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
 }
 
 }  // namespace
@@ -1345,21 +1454,28 @@ int tqk_dequant_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t
   if (!p || n_items < 0 || (n_items > 0 && (!items || !kout || !vout))) return TQK_EINVAL;
   if (n_items == 0) return TQK_OK;
   if (d->key_grid == 2 && !p->knorm) return TQK_EINVAL;
-  DequantArgs a;
-  a.d = *d;
-  a.p = *p;
-  a.items = items;
-  a.kout = kout;
-  a.vout = vout;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  const dim3 grid(n_items, d->n_kv_heads);
-  if (d->head_dim == 64)
-    launch_by_vb<64>(d->value_bits, grid, st, a);
-  else if (d->head_dim == 128)
-    launch_by_vb<128>(d->value_bits, grid, st, a);
-  else
-    launch_by_vb<256>(d->value_bits, grid, st, a);
-  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
+  const int chunks = (d->group_tokens + kDqTokens - 1) / kDqTokens;
+  const DequantArgs a{*d, *p, items, nullptr, chunks, 0, kout, vout};
+  return launch_dequant<float>(dim3((unsigned)n_items * (unsigned)chunks, d->n_kv_heads), stream, a);
+}
+
+int tqk_dequant_dense(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,
+                      const int32_t* seq_lens, int32_t max_len, int32_t out_type, void* kout,
+                      void* vout, void* stream) {
+  int rc = tqk_check_desc(d);
+  if (rc != TQK_OK) return rc;
+  if (!p || batch <= 0 || max_len <= 0 || !seq_lens || !kout || !vout) return TQK_EINVAL;
+  if (d->key_grid == 2 && !p->knorm) return TQK_EINVAL;
+  if (out_type < 0 || out_type > 2) return TQK_EINVAL;
+  const int G = d->group_tokens, cpg = (G + kDqTokens - 1) / kDqTokens;
+  const long long chunks = (long long)n_groups_of(max_len, d->hot_window, G) * cpg +
+                           (min(max_len, d->hot_window) + kDqTokens - 1) / kDqTokens;
+  if (chunks * batch >= (1LL << 31)) return TQK_EINVAL;
+  const DequantArgs a{*d, *p, nullptr, seq_lens, (int)chunks, max_len, kout, vout};
+  const dim3 grid((unsigned)(chunks * batch), d->n_kv_heads);
+  if (out_type == 0) return launch_dequant<float>(grid, stream, a);
+  if (out_type == 1) return launch_dequant<_Float16>(grid, stream, a);
+  return launch_dequant<__bf16>(grid, stream, a);
 }
 
 }  // extern "C"

@@ -134,19 +134,15 @@ class TurboQuantLayer(CacheLayerMixin):
         """The whole cache as dense ``(B, H, L, D)`` K/V in ``dtype`` (the model
         dtype by default): coded groups through the GPU dequant (fp32), then
         the hot window."""
-        pool = self.pool
-        B, H, D, G = self.batch, self.n_kv_heads, self.head_dim, pool.group_tokens
-        ng = pool.n_groups(0)
-        keys, values = [], []
-        if ng:
-            kk, vv = pool.dequant_groups([(b, g) for b in range(B) for g in range(ng)])
-            keys.append(kk.view(B, ng, H, G, D).permute(0, 2, 1, 3, 4).reshape(B, H, ng * G, D))
-            values.append(vv.view(B, ng, H, G, D).permute(0, 2, 1, 3, 4).reshape(B, H, ng * G, D))
-        hot = [pool.hot_window_tokens(b) for b in range(B)]
-        keys.append(torch.stack([h[0] for h in hot]).float())
-        values.append(torch.stack([h[1] for h in hot]).float())
         dt = self.dtype if dtype is None else dtype
-        return torch.cat(keys, dim=2).to(dt), torch.cat(values, dim=2).to(dt)
+        if self.get_seq_length() == 0:
+            shape = (self.batch, self.n_kv_heads, 0, self.head_dim)
+            return (torch.empty(shape, dtype=dt, device=self.pool.device),
+                    torch.empty(shape, dtype=dt, device=self.pool.device))
+        if dt in (torch.float32, torch.float16, torch.bfloat16):
+            return self.pool.dense(dt)
+        k, v = self.pool.dense()
+        return k.to(dt), v.to(dt)
 
     def decode(self, query, scaling: float):
         """Fused decode of one query token per sequence: ``(B, Hq, 1, D)`` ->

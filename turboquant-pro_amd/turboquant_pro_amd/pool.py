@@ -417,6 +417,27 @@ class TQKVPool:
                                                self._stream()), "tqk_dequant_groups")
         return kout, vout
 
+    def dense(self, dtype=None):
+        """Every sequence's whole cache as dense ``(B, Hkv, L, D)`` keys and
+        values of ``dtype`` (fp32, fp16 or bf16; fp32 by default), L the longest
+        length: the coded groups reconstructed, then the hot window, each
+        rounded to nearest even.  Rows past a sequence's length are undefined."""
+        torch = _torch()
+        self.check()
+        kinds = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
+        dt = torch.float32 if dtype is None else dtype
+        if dt not in kinds:
+            raise ValueError(f"dense keys and values are fp32, fp16 or bf16, not {dt}")
+        if min(self.lengths) <= 0:
+            raise RuntimeError("cache is empty")
+        B, L = self.max_batch, max(self.lengths)
+        k = torch.empty((B, self.n_kv_heads, L, self.head_dim), dtype=dt, device=self.device)
+        v = torch.empty_like(k)
+        N.check(N.lib().tqk_dequant_dense(ctypes.byref(self.desc), ctypes.byref(self.ptrs), B,
+                                          self.seq_lens.data_ptr(), L, kinds[dt], k.data_ptr(),
+                                          v.data_ptr(), self._stream()), "tqk_dequant_dense")
+        return k, v
+
     def hot_window_tokens(self, b: int):
         """``(Hkv, n_hot, D)`` keys and values of sequence b's hot window, in the
         pool's input dtype."""
