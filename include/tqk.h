@@ -235,6 +235,21 @@ int tqk_append_hot(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t bat
                    void* stream);
 
 /*
+ * A whole append of up to 64 sequences that completes at most 128 groups: the
+ * groups that the new tokens complete are encoded (tqk_encode_groups; `overflow`
+ * as there, may be null), the surviving tokens copied into the ring
+ * (tqk_append_hot), and seq_lens[b] (device) set to prev_len[b] + n_new[b].
+ * prev_len and n_new are HOST arrays of `batch` entries, passed with the
+ * launches (no copy to the device); n_new[b] in [0, chunk_tokens].  Beyond those
+ * limits TQK_EINVAL, with nothing launched.  TurboQuantKVCache.append
+ * (turboquant_pro/core.py:986-1038).
+ */
+int tqk_append_tokens(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,
+                      const int32_t* prev_len, const int32_t* n_new, const void* chunk_k,
+                      const void* chunk_v, int32_t chunk_tokens, int32_t* seq_lens,
+                      int32_t* overflow, void* stream);
+
+/*
  * Reconstruct fp32 keys and values of `n_items` groups (items as in
  * tqk_encode_groups): kout/vout [n_items][n_kv_heads][G][D].  The GPU form of
  * PerChannelKV.decompress (turboquant_pro/per_channel_kv.py:497-539) and

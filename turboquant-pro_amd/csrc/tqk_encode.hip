@@ -31,17 +31,27 @@ constexpr int kEncWaves = kEncThreads / 64;
 struct TokenRows { static constexpr bool value = false; };
 struct TiledRows { static constexpr bool value = true; };
 
+// What an append of a few sequences passes with the launch instead of in device
+// memory: a copy to the device and its launch cost more than the append itself.
+constexpr int kInlineSeqs = 64, kInlineItems = 128;
+struct InlineItems {
+  int32_t prev[kInlineSeqs];
+  int32_t item[2 * kInlineItems];
+};
+
 struct EncodeArgs {
   tqk_cache_desc d;
   tqk_cache_ptrs p;
-  const int32_t* items;
+  const int32_t* items;     // nullptr: in.item, in.prev
   const int32_t* prev_len;
   const void* chunk_k;  // fp16, or fp32 (input_f32)
   const void* chunk_v;
   int chunk_tokens;
   int n_items;
   int32_t* overflow;
+  InlineItems in;
 };
+__device__ __forceinline__ int item_word(const EncodeArgs& a, int i) { return a.items ? a.items[i] : a.in.item[i]; }
 
 // Source row (D values of type T: fp16 bits or fp32) of token t of sequence
 // b, kv head h: the hot ring for tokens already in the cache, the appended
@@ -50,7 +60,7 @@ template <int D, typename T = uint16_t>
 __device__ __forceinline__ const T* token_src(const EncodeArgs& a, const void* ring,
                                               const void* chunk, int b, int h, int t) {
   const tqk_cache_desc& d = a.d;
-  const int prev = a.prev_len[b];
+  const int prev = a.items ? a.prev_len[b] : a.in.prev[b];
   if (t < prev)
     return static_cast<const T*>(ring) +
            (((size_t)b * d.n_kv_heads + h) * d.hot_ring + (t % d.hot_ring)) * D;
@@ -172,7 +182,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const tqk_cache_desc& d = a.d;
-  const int b = a.items[2 * item], g = a.items[2 * item + 1];
+  const int b = item_word(a, 2 * item), g = item_word(a, 2 * item + 1);
   const int G = d.group_tokens, P = d.page_tokens, Hkv = d.n_kv_heads;
   const int slot = a.p.group_table[(size_t)b * d.max_groups_per_seq + g];
   const int kout = d.outliers_per_channel;
@@ -747,7 +757,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
   const int lane = tid & 63, wv = tid >> 6;
   const tqk_cache_desc& d = a.d;
-  const int b = a.items[2 * item], g = a.items[2 * item + 1];
+  const int b = item_word(a, 2 * item), g = item_word(a, 2 * item + 1);
   const int G = d.group_tokens, P = d.page_tokens, Hkv = d.n_kv_heads;
   const int slot = a.p.group_table[(size_t)b * d.max_groups_per_seq + g];
   const int kout = d.outliers_per_channel;
@@ -1119,12 +1129,15 @@ struct HotArgs {
   tqk_cache_desc d;
   uint8_t* hot_k;
   uint8_t* hot_v;
-  const int32_t* prev_len;
+  const int32_t* prev_len;  // nullptr: the inline lengths
   const int32_t* n_new;
   const int32_t* hot_start;
   const uint8_t* chunk_k;
   const uint8_t* chunk_v;
   int chunk_tokens;
+  int32_t* seq_lens;        // with inline lengths: the new lengths are written here
+  int32_t in_prev[kInlineSeqs];
+  int32_t in_new[kInlineSeqs];
 };
 
 constexpr int kHotSlice = 64;  // tokens per workgroup of the ring copy
@@ -1136,8 +1149,18 @@ constexpr int kHotSlice = 64;  // tokens per workgroup of the ring copy
 __global__ __launch_bounds__(kThreads) void tqk_append_hot_kernel(HotArgs a) {
   const int b = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
   const tqk_cache_desc& d = a.d;
-  const int prev = a.prev_len[b], nn = a.n_new[b];
-  const int t0 = max(prev, a.hot_start[b]), t1 = prev + nn;
+  int prev, nn, start;
+  if (a.prev_len) {
+    prev = a.prev_len[b];
+    nn = a.n_new[b];
+    start = a.hot_start[b];
+  } else {
+    prev = a.in_prev[b];
+    nn = a.in_new[b];
+    start = n_groups_of(prev + nn, d.hot_window, d.group_tokens) * d.group_tokens;
+    if (h == 0 && blockIdx.z == 0 && tid == 0) a.seq_lens[b] = prev + nn;
+  }
+  const int t0 = max(prev, start), t1 = prev + nn;
   const int R = d.hot_ring;
   const size_t rb = ((size_t)b * d.n_kv_heads + h) * R;
   const size_t cb = ((size_t)b * d.n_kv_heads + h) * a.chunk_tokens;
@@ -1384,6 +1407,30 @@ int launch_dequant(dim3 grid, void* stream, const DequantArgs& a) {
   return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
 }
 
+int launch_encode(const EncodeArgs& a, void* stream) {
+  const tqk_cache_desc& d = a.d;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (d.key_grid == 0 && d.zero_point == 2 && !a.p.zp_mean) return TQK_EINVAL;
+  if (d.key_grid == 2 && !a.p.knorm) return TQK_EINVAL;
+  const dim3 grid(a.n_items, d.n_kv_heads);
+  if (d.head_dim == 64)
+    launch_by_vb<64>(d.value_bits, grid, st, a);
+  else if (d.head_dim == 128)
+    launch_by_vb<128>(d.value_bits, grid, st, a);
+  else
+    launch_by_vb<256>(d.value_bits, grid, st, a);
+  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
+}
+
+int launch_hot(const HotArgs& a, int batch, void* stream) {
+  // the surviving tokens of a sequence number at most min(chunk, ring)
+  const int span = min(a.chunk_tokens, a.d.hot_ring);
+  const int slices = max(1, (span + kHotSlice - 1) / kHotSlice);
+  hipLaunchKernelGGL(tqk_append_hot_kernel, dim3(batch, a.d.n_kv_heads, slices), dim3(kThreads), 0,
+                     reinterpret_cast<hipStream_t>(stream), a);
+  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1397,7 +1444,7 @@ int tqk_encode_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t 
   if (!p || batch <= 0 || n_items < 0 || chunk_tokens < 0) return TQK_EINVAL;
   if (n_items == 0) return TQK_OK;
   if (!items || !prev_len) return TQK_EINVAL;
-  EncodeArgs a;
+  EncodeArgs a{};
   a.d = *d;
   a.p = *p;
   a.items = items;
@@ -1407,17 +1454,7 @@ int tqk_encode_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t 
   a.chunk_tokens = chunk_tokens;
   a.n_items = n_items;
   a.overflow = overflow;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (d->key_grid == 0 && d->zero_point == 2 && !p->zp_mean) return TQK_EINVAL;
-  if (d->key_grid == 2 && !p->knorm) return TQK_EINVAL;
-  const dim3 grid(n_items, d->n_kv_heads);
-  if (d->head_dim == 64)
-    launch_by_vb<64>(d->value_bits, grid, st, a);
-  else if (d->head_dim == 128)
-    launch_by_vb<128>(d->value_bits, grid, st, a);
-  else
-    launch_by_vb<256>(d->value_bits, grid, st, a);
-  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
+  return launch_encode(a, stream);
 }
 
 int tqk_append_hot(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,
@@ -1429,7 +1466,7 @@ int tqk_append_hot(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t bat
   if (!p || batch <= 0 || !prev_len || !n_new || !hot_start || !chunk_k || !chunk_v ||
       chunk_tokens <= 0)
     return TQK_EINVAL;
-  HotArgs a;
+  HotArgs a{};
   a.d = *d;
   a.hot_k = static_cast<uint8_t*>(p->hot_k);
   a.hot_v = static_cast<uint8_t*>(p->hot_v);
@@ -1439,12 +1476,50 @@ int tqk_append_hot(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t bat
   a.chunk_k = static_cast<const uint8_t*>(chunk_k);
   a.chunk_v = static_cast<const uint8_t*>(chunk_v);
   a.chunk_tokens = chunk_tokens;
-  // the surviving tokens of a sequence number at most min(chunk, ring)
-  const int span = min(chunk_tokens, d->hot_ring);
-  const int slices = max(1, (span + kHotSlice - 1) / kHotSlice);
-  hipLaunchKernelGGL(tqk_append_hot_kernel, dim3(batch, d->n_kv_heads, slices), dim3(kThreads), 0,
-                     reinterpret_cast<hipStream_t>(stream), a);
-  return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
+  return launch_hot(a, batch, stream);
+}
+
+int tqk_append_tokens(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,
+                      const int32_t* prev_len, const int32_t* n_new, const void* chunk_k,
+                      const void* chunk_v, int32_t chunk_tokens, int32_t* seq_lens,
+                      int32_t* overflow, void* stream) {
+  int rc = tqk_check_desc(d);
+  if (rc != TQK_OK) return rc;
+  if (!p || !prev_len || !n_new || !chunk_k || !chunk_v || !seq_lens || chunk_tokens <= 0 || batch <= 0 ||
+      batch > kInlineSeqs)
+    return TQK_EINVAL;
+  EncodeArgs e{};
+  HotArgs a{};
+  for (int b = 0; b < batch; ++b) {
+    if (prev_len[b] < 0 || n_new[b] < 0 || n_new[b] > chunk_tokens) return TQK_EINVAL;
+    e.in.prev[b] = a.in_prev[b] = prev_len[b];
+    a.in_new[b] = n_new[b];
+    const int g1 = n_groups_of(prev_len[b] + n_new[b], d->hot_window, d->group_tokens);
+    for (int g = n_groups_of(prev_len[b], d->hot_window, d->group_tokens); g < g1; ++g) {
+      if (e.n_items == kInlineItems) return TQK_EINVAL;
+      e.in.item[2 * e.n_items] = b;
+      e.in.item[2 * e.n_items + 1] = g;
+      ++e.n_items;
+    }
+  }
+  if (e.n_items > 0) {
+    e.d = *d;
+    e.p = *p;
+    e.chunk_k = chunk_k;
+    e.chunk_v = chunk_v;
+    e.chunk_tokens = chunk_tokens;
+    e.overflow = overflow;
+    rc = launch_encode(e, stream);
+    if (rc != TQK_OK) return rc;
+  }
+  a.d = *d;
+  a.hot_k = static_cast<uint8_t*>(p->hot_k);
+  a.hot_v = static_cast<uint8_t*>(p->hot_v);
+  a.chunk_k = static_cast<const uint8_t*>(chunk_k);
+  a.chunk_v = static_cast<const uint8_t*>(chunk_v);
+  a.chunk_tokens = chunk_tokens;
+  a.seq_lens = seq_lens;
+  return launch_hot(a, batch, stream);
 }
 
 int tqk_dequant_groups(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t n_items,

@@ -21,11 +21,14 @@ TQK_EWORKSPACE = 4
 
 ABI_VERSION = 9
 
+# limits of tqk_append_tokens: sequences, and groups that one append completes
+APPEND_SEQS, APPEND_GROUPS = 64, 128
+
 # Every symbol include/tqk.h declares (checked by the CPU test suite).
 EXPORTS = (
     "tqk_version", "tqk_check_desc", "tqk_decode_workspace_bytes", "tqk_decode",
     "tqk_decode_noalloc", "tqk_decode_partials", "tqk_decode_splits", "tqk_decode_merge", "tqk_encode_groups",
-    "tqk_append_hot", "tqk_dequant_groups", "tqk_dequant_dense", "tqk_encode_key_block", "tqk_encode_value_block",
+    "tqk_append_hot", "tqk_append_tokens", "tqk_dequant_groups", "tqk_dequant_dense", "tqk_encode_key_block", "tqk_encode_value_block",
     "tqk_dequant_key_block", "tqk_dequant_value_block",
 )
 
@@ -72,6 +75,7 @@ def load(path: str) -> ctypes.CDLL:
         "tqk_decode_merge": ([pd, pp, i32, i32, vp, vp, sz, vp], ctypes.c_int),
         "tqk_encode_groups": ([pd, pp, i32, i32, vp, vp, vp, vp, i32, vp, vp], ctypes.c_int),
         "tqk_append_hot": ([pd, pp, i32, vp, vp, vp, vp, vp, i32, vp], ctypes.c_int),
+        "tqk_append_tokens": ([pd, pp, i32, vp, vp, vp, vp, i32, vp, vp, vp], ctypes.c_int),
         "tqk_dequant_groups": ([pd, pp, i32, vp, vp, vp, vp], ctypes.c_int),
         "tqk_dequant_dense": ([pd, pp, i32, vp, i32, i32, vp, vp, vp], ctypes.c_int),
         "tqk_encode_key_block": ([pb, vp, vp, vp, vp, vp, vp, vp, vp, vp], ctypes.c_int),

@@ -314,37 +314,55 @@ class TQKVPool:
         new = [p + n for p, n in zip(prev, n_new)]
         if max(new) > self.max_seq_len:
             raise ValueError(f"sequence length {max(new)} exceeds max_seq_len={self.max_seq_len}")
-        items = []
-        for b in range(B):
-            for g in range(n_groups_for(prev[b], self.hot_window), n_groups_for(new[b], self.hot_window)):
-                items += [b, g]
-        hot_start = [n_groups_for(L, self.hot_window) * self.group_tokens for L in new]
+        spans = [(n_groups_for(p, self.hot_window), n_groups_for(L, self.hot_window))
+                 for p, L in zip(prev, new)]
+        n_items = sum(g1 - g0 for g0, g1 in spans)
+        L = N.lib()
+        st = self._stream()
+        if n_items:
+            self._overflow.zero_()
+        if T > 0 and B <= N.APPEND_SEQS and n_items <= N.APPEND_GROUPS:
+            # a few sequences and groups go with the launches: no copy to the
+            # device, and the lengths are written by the ring copy
+            ints = ctypes.c_int32 * B
+            N.check(L.tqk_append_tokens(ctypes.byref(self.desc), ctypes.byref(self.ptrs), B, ints(*prev),
+                                        ints(*n_new), k.data_ptr(), v.data_ptr(), T,
+                                        self.seq_lens.data_ptr(), self._overflow.data_ptr(), st),
+                    "tqk_append_tokens")
+            if n_items and check_overflow:
+                self._read_flags()
+            self.lengths = new
+            return
+        items = [x for b, (g0, g1) in enumerate(spans) for g in range(g0, g1) for x in (b, g)]
+        hot_start = [g1 * self.group_tokens for _, g1 in spans]
         # pinned and asynchronous: the caching host allocator keeps the block
         # until the copy, queued behind earlier work on the stream, has run
         host = torch.tensor(prev + n_new + hot_start + items, dtype=torch.int32).pin_memory()
         dev = host.to(self.device, non_blocking=True)
         prev_d, nnew_d, hs_d = dev[:B], dev[B:2 * B], dev[2 * B:3 * B]
         items_d = dev[3 * B:]
-        L = N.lib()
-        st = self._stream()
         if items:
-            self._overflow.zero_()
             N.check(L.tqk_encode_groups(ctypes.byref(self.desc), ctypes.byref(self.ptrs), B,
-                                        len(items) // 2, items_d.data_ptr(), prev_d.data_ptr(),
+                                        n_items, items_d.data_ptr(), prev_d.data_ptr(),
                                         k.data_ptr(), v.data_ptr(), T,
                                         self._overflow.data_ptr(), st), "tqk_encode_groups")
             if check_overflow:
-                flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
-                flag.copy_(self._overflow, non_blocking=True)
-                ev = torch.cuda.Event()
-                ev.record(torch.cuda.current_stream(self.device))
-                self._pending.append((ev, flag))
+                self._read_flags()
         if T > 0:
             N.check(L.tqk_append_hot(ctypes.byref(self.desc), ctypes.byref(self.ptrs), B,
                                      prev_d.data_ptr(), nnew_d.data_ptr(), hs_d.data_ptr(),
                                      k.data_ptr(), v.data_ptr(), T, st), "tqk_append_hot")
         self.lengths = new
         torch.add(prev_d, nnew_d, out=self.seq_lens)
+
+    def _read_flags(self) -> None:
+        """Queue the copy of the encode's flags to pinned memory (``check``)."""
+        torch = _torch()
+        flag = torch.empty(1, dtype=torch.int32, pin_memory=True)
+        flag.copy_(self._overflow, non_blocking=True)
+        ev = torch.cuda.Event()
+        ev.record(torch.cuda.current_stream(self.device))
+        self._pending.append((ev, flag))
 
     # ------------------------------------------------------------------ #
     def workspace(self, batch: int, max_len: int):
