@@ -14,6 +14,7 @@
 // and adds the hot-window part (turboquant_pro/kv_fused.py:139-153).
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "tqk_common.h"
 
@@ -64,10 +65,32 @@ struct MergeArgs {
 constexpr int kThreads = 256;
 constexpr int kVOEnt = 2048;  // VALU decode: side-list entries staged in LDS per group
 
+// The wave's sum or maximum in every lane, on the VALU (rotations inside the
+// 16-lane rows, then the two permlane swaps): a butterfly of ds_bpermute is six
+// LDS round trips in a row.
+template <bool IS_MAX>
+__device__ __forceinline__ float wave_reduce(float x) {
+  auto op = [](float a, float b) { return IS_MAX ? fmaxf(a, b) : a + b; };
+  auto ror = [](float v, auto n) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x120 + decltype(n)::value,
+                                                                 0xF, 0xF, true));
+  };
+  x = op(x, ror(x, std::integral_constant<int, 8>{}));
+  x = op(x, ror(x, std::integral_constant<int, 4>{}));
+  x = op(x, ror(x, std::integral_constant<int, 2>{}));
+  x = op(x, ror(x, std::integral_constant<int, 1>{}));
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto r16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = op(__builtin_bit_cast(float, (uint32_t)r16[0]), __builtin_bit_cast(float, (uint32_t)r16[1]));
+  const uint32_t w = __builtin_bit_cast(uint32_t, x);
+  const auto r32 = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return op(__builtin_bit_cast(float, (uint32_t)r32[0]), __builtin_bit_cast(float, (uint32_t)r32[1]));
+}
+
 template <int GQ, bool IS_MAX>
 __device__ __forceinline__ void block_reduce(float (&v)[GQ], float (*red)[GQ]) {
 #pragma unroll
-  for (int i = 0; i < GQ; ++i) v[i] = IS_MAX ? wave_max(v[i]) : wave_sum(v[i]);
+  for (int i = 0; i < GQ; ++i) v[i] = wave_reduce<IS_MAX>(v[i]);
   if ((threadIdx.x & 63) == 0) {
 #pragma unroll
     for (int i = 0; i < GQ; ++i) red[threadIdx.x >> 6][i] = v[i];
@@ -140,6 +163,41 @@ __device__ __forceinline__ void outlier_walk(const uint32_t* oe, int lo, int end
   }
 }
 
+// The code of channel j in a key row (2- and 3-bit rows are one little-endian
+// stream)
+__device__ __forceinline__ uint32_t key_code(const uint8_t* row, int kb, int j) {
+  if (kb == 4) {
+    const uint32_t w = row[j >> 1];
+    return rev4((j & 1) ? w & 15u : w >> 4);
+  }
+  const int byte = (kb * j) >> 3, last = (kb * (j | 31) + kb - 1) >> 3;  // (the 32-channel chunk's last byte)
+  const uint32_t w = (uint32_t)row[byte] | (uint32_t)row[min(byte + 1, last)] << 8;
+  return (w >> ((kb * j) & 7)) & ((1u << kb) - 1u);
+}
+
+// outlier_walk over a list staged in LDS.  An fp16 cache stores the level of the
+// mean at its side-list positions, so dense_j is the mean there; an fp32 cache
+// keeps the reference's codes, staged beside the list.
+template <int GQ, int D>
+__device__ __forceinline__ void staged_walk(const uint32_t* oe, const uint8_t* code, bool f32, int lo, int end,
+                                            uint32_t first, const float* lev, const float* a_s,
+                                            const float* mu_s, const float (*q_s)[D], float (&s)[GQ]) {
+  int hi = end;
+  while (lo < hi) {  // first entry of the run at or after (token, 0)
+    const int mid = (lo + hi) >> 1;
+    if ((oe[mid] & 0xFFFFu) < first) lo = mid + 1; else hi = mid;
+  }
+  for (int e = lo; e < end; ++e) {
+    const uint32_t ent = oe[e], pos = ent & 0xFFFFu;
+    if (pos >= first + D) break;
+    const int j = (int)(pos - first);
+    const float dense = f32 ? a_s[j] * lev[code[e]] + mu_s[j] : mu_s[j];
+    const float delta = h2f((uint16_t)(ent >> 16)) - dense;
+#pragma unroll
+    for (int i = 0; i < GQ; ++i) s[i] += q_s[i][j] * delta;
+  }
+}
+
 // A token's dense key scores s[i] += w_i(pair) . levels(pair), pair by pair
 // in channel order, by 32-channel chunks (KB words of the row each, read once
 // per chunk): the 16 pairs of a chunk take their fields at fixed bit offsets
@@ -204,7 +262,13 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
   __shared__ float2 w2_s[NP][GQ];
   // the group's side-list, when it holds at most kVOEnt entries (the token
   // threads' searches and walks then read LDS, not memory)
+  // with an fp32 cache's key codes beside it: read from memory by the walks, a
+  // code is a serial latency an entry (16 x 8192 tokens x 8 heads at head_dim
+  // 256: 204 us, staged 177)
   __shared__ uint32_t oe_s[kVOEnt];
+  __shared__ uint8_t oc_s[kVOEnt];
+  __shared__ float lev_s[16];
+  __shared__ int row_s[kThreads];  // row of every token of the group in the head's pages
   // the group's value code rows, staged by the token threads (one row each,
   // wide loads) for the value pass, whose threads walk the tokens of a slice
   // (not at 8 heads: the staging loads, live across the key loop, take all
@@ -217,7 +281,13 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
   __shared__ float vl_s[1 << (2 * VB)][2];
   __shared__ float red_s[4][GQ];
   __shared__ float a_s[D], mu_s[D];
-  __shared__ float accr_s[NQ][GQ][D];
+  // the token slices' sums at the end take the value rows' place where they fit
+  // (an fp32 cache at head_dim 128 and 4 heads: four workgroups a CU instead of
+  // three)
+  constexpr bool kOwnAcc = !kStageV || sizeof(vrow_s) < sizeof(float) * NQ * GQ * D;
+  __shared__ float accr_own[kOwnAcc ? NQ : 1][kOwnAcc ? GQ : 1][kOwnAcc ? D : 1];
+  float (*accr_s)[GQ][D] = reinterpret_cast<float (*)[GQ][D]>(
+      kOwnAcc ? static_cast<void*>(accr_own) : static_cast<void*>(vrow_s));
 
   // GQ is the kernel's power-of-two head count; the last GQ - gq heads are
   // zero-query padding whose states are never written
@@ -238,6 +308,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
     kl_s[tid][0] = polar ? a.p.vcent[c0 & cm] : key_level(a.d.key_grid, c0);
     kl_s[tid][1] = polar ? a.p.vcent[c1 & cm] : key_level(a.d.key_grid, c1);
   }
+  if (tid < 16) lev_s[tid] = key_level(a.d.key_grid, tid);
   // value pair table: field f of two channels' codes -> their two centroids
   if (tid < (1 << (2 * VB))) {
     vl_s[tid][0] = a.p.vcent[tid & ((1 << VB) - 1)];
@@ -301,6 +372,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
       const bool oe_lds = !(GQ >= 8 && D >= 256) && n_oe <= kVOEnt;
       if (oe_lds)
         for (int e = tid; e < n_oe; e += kThreads) oe_s[e] = a.p.oent[obase * d.outlier_cap + e];
+      if (kAhead && f32) row_s[tid] = phys * P + (g * G + tid) % P;
       if (tid < D) {
         const float av = a.p.gscale[mbase + tid];
         const float mv = a.p.gmean[mbase + tid];
@@ -310,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
 #pragma unroll
         for (int i = 0; i < GQ; ++i) {
           reinterpret_cast<float*>(&w2_s[tid >> 1][i])[tid & 1] = (polar ? qr_s[i][tid] : q_s[i][tid]) * av;
-          bias_part[i] = wave_sum(q_s[i][tid] * mv);
+          bias_part[i] = wave_reduce<false>(q_s[i][tid] * mv);
         }
         if ((tid & 63) == 0) {
 #pragma unroll
@@ -324,6 +396,14 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
         bias[i] = red_s[0][i];
         if constexpr (NW == 2) bias[i] = red_s[0][i] + red_s[1][i];
         if constexpr (NW == 4) bias[i] = (red_s[0][i] + red_s[1][i]) + (red_s[2][i] + red_s[3][i]);
+      }
+      if (oe_lds && f32) {
+#pragma unroll 4
+        for (int e = tid; e < n_oe; e += kThreads) {
+          const uint32_t pos = oe_s[e] & 0xFFFFu;
+          const uint8_t* kr = a.p.kcodes + ((size_t)h * d.n_pages * P + row_s[pos / D]) * k_row_bytes(d.key_bits, D);
+          oc_s[e] = (uint8_t)key_code(kr, d.key_bits, (int)(pos % D));
+        }
       }
       __syncthreads();
 
@@ -412,7 +492,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
           const int end = min(kAhead ? oc_hi : oc[blk], cap);
           const uint32_t first = (uint32_t)tid * D;
           if (oe_lds) {
-            outlier_walk<GQ, D>(oe_s, lo0, end, first, kr, kb, a.d.key_grid, a_s, mu_s, q_s, s);
+            staged_walk<GQ, D>(oe_s, oc_s, f32, lo0, end, first, lev_s, a_s, mu_s, q_s, s);
           } else {
             // (at 8 heads and head_dim 256 from the row's registers: the
             // row pointer held across the walk there takes all 256 VGPRs)
@@ -539,6 +619,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
   }
 
   // combine the token slices and write the split's state
+  if constexpr (!kOwnAcc) __syncthreads();
 #pragma unroll
   for (int i = 0; i < GQ; ++i) {
     accr_s[tq][i][2 * jp] = acc0[i];
@@ -2364,11 +2445,14 @@ Plan make_plan(const tqk_cache_desc* d, int batch, int max_len) {
   } else {
     // VALU kernel: a workgroup pays its set-up (query, code tables, the
     // split's partial, the merge's share) once for its gps groups, about a
-    // group's time, and about three of its workgroups fit a CU.  Pick gps from
-    // the bound of at most 4096 coded workgroups (which bounds the partials)
-    // up to 8x that, minimising rounds of the CUs times (gps + 1), the hot
-    // splits' workgroups counted in the rounds.
-    const long slots = 3L * device_cus();
+    // group's time, and three of its workgroups fit a CU, four up to head_dim
+    // 128 and 4 heads (LDS).  Pick gps from the bound of at most 4096 coded
+    // workgroups (which bounds the partials) up to 8x that, minimising rounds
+    // of the CUs times (gps + 1), the hot splits' workgroups counted in the
+    // rounds: 16 x 8192 tokens x 8 heads in an fp32 cache, gps 3 / 5 / 8: 121 /
+    // 116 / 148 us; head_dim 256: 171 / 223 / 193 us.
+    const bool four = d->head_dim <= 128 && d->n_q_heads <= 4 * d->n_kv_heads;
+    const long slots = (four ? 4L : 3L) * device_cus();
     const long pairs = (long)batch * d->n_kv_heads;
     const int g_lo = units > 4096 ? (int)((units + 4095) / 4096) : 1;
     const int g_hi = ngmax > g_lo ? (8 * g_lo < ngmax ? 8 * g_lo : ngmax) : g_lo;
