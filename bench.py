@@ -269,9 +269,6 @@ def _cpu_model():
     return "unknown"
 
 
-VALU_OPS_PEAK = 256 * 4 * 16 * 2.4e9  # separately rounded fp32 ops/s: 256 CUs x 4 SIMD x 16 lanes x 2.4 GHz
-
-
 def encode_bench(torch, cfg, fills, chunk=4096):
     """Prefill encode: the config's batch appended in ``chunk``-token chunks up
     to its context (group flushes through the encode kernel, hot-ring copies),
@@ -279,9 +276,7 @@ def encode_bench(torch, cfg, fills, chunk=4096):
     (512 B per token-head) + the coded groups out in the reference's container
     sizes (116 B per cold token-head at K4/V3 plus 4864 B of stats and
     side-list per group-head).  The encode is bound by
-    the value rotation's 2 * 128^2 separately rounded fp32 operations per
-    token-head (no FMA, no packed math: the bit-exactness contract), reported
-    against the chip's unpacked VALU issue rate."""
+    its VALU work; ``hbm_frac`` is those bytes against the 8 TB/s roof."""
     from turboquant_pro_amd import TQKVPool
     B, Hkv, Hq, L, vb = cfg["B"], cfg["Hkv"], cfg["Hq"], cfg["L"], cfg["vbits"]
     gen = torch.Generator(device="cuda")
@@ -311,14 +306,11 @@ def encode_bench(torch, cfg, fills, chunk=4096):
     per_token = 128 * kb // 8 + 128 * vb // 8 + 4 + (4 if polar else 0)
     per_group = 0 if polar else 2 * 128 * 4 + n_out * 6
     nbytes = B * Hkv * (L * 2 * 128 * 2 + n_cold * per_token) + B * Hkv * n_groups(L) * per_group
-    # PolarQuant keys go through the same rotation as the values
-    rot_ops = B * Hkv * n_cold * 2 * 128 * 128 * (2 if polar else 1)
     return {"metric": "prefill encode GB/s (fp16 K+V in + coded groups out)",
             "value": round(nbytes / (ms * 1e-3) / 1e9, 1), "unit": "GB/s",
             "ms_per_fill": round(ms, 3), "tokens_per_s": round(B * L / (ms * 1e-3)),
             "fills": len(times), "bytes": nbytes,
-            "rotation_ops_per_s": round(rot_ops / (ms * 1e-3) / 1e12, 2),
-            "valu_frac": round(rot_ops / (ms * 1e-3) / VALU_OPS_PEAK, 3),
+            "hbm_frac": round(nbytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 3),
             "config": {"name": cfg.get("name", ""), "batch": B, "context": L, "n_kv_heads": Hkv,
                        "chunk": chunk, "value_bits": vb, "keys": key_form(cfg)}}
 
