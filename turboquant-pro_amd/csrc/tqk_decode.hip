@@ -2445,27 +2445,29 @@ Plan make_plan(const tqk_cache_desc* d, int batch, int max_len) {
   } else {
     // VALU kernel: a workgroup pays its set-up (query, code tables, the
     // split's partial, the merge's share) once for its gps groups, about a
-    // group's time, and three of its workgroups fit a CU, four up to head_dim
-    // 128 and 4 heads (LDS).  Pick gps from the bound of at most 4096 coded
-    // workgroups (which bounds the partials) up to 8x that, minimising rounds
-    // of the CUs times (gps + 1), the hot splits' workgroups counted in the
-    // rounds: 16 x 8192 tokens x 8 heads in an fp32 cache, gps 3 / 5 / 8: 121 /
-    // 116 / 148 us; head_dim 256: 171 / 223 / 193 us.
-    const bool four = d->head_dim <= 128 && d->n_q_heads <= 4 * d->n_kv_heads;
-    const long slots = (four ? 4L : 3L) * device_cus();
+    // group's time, and three of its workgroups fit a CU.  Pick gps from the
+    // bound of at most 4096 coded workgroups (which bounds the partials) up to
+    // 8x that, minimising rounds of the CUs times (gps + 1), the hot splits'
+    // workgroups counted in the rounds.  Up to head_dim 128 and 4 heads four
+    // fit (LDS; not with 4-bit value rows at 128 and 4 heads): there a larger
+    // gps is taken if it costs less with four.  16 x 8192 tokens x 8 heads in
+    // an fp32 cache, gps 3 / 5 / 8: 121 / 116 / 148 us.  A smaller one is not:
+    // its set-ups cost more than the model says (32 x 8129 tokens x 2 heads at
+    // head_dim 64, gps 3 / 1: 31 / 43 us).
     const long pairs = (long)batch * d->n_kv_heads;
     const int g_lo = units > 4096 ? (int)((units + 4095) / 4096) : 1;
     const int g_hi = ngmax > g_lo ? (8 * g_lo < ngmax ? 8 * g_lo : ngmax) : g_lo;
-    double best = 1e30;
+    auto cost = [&](int g, int per_cu) {
+      const long blocks = pairs * ((ngmax + g - 1) / g + pl.n_hot_splits), slots = (long)per_cu * device_cus();
+      return (double)((blocks + slots - 1) / slots) * (g + 1);
+    };
     gps = g_lo;
-    for (int g = g_lo; g <= g_hi; ++g) {
-      const long blocks = pairs * ((ngmax + g - 1) / g + pl.n_hot_splits);
-      const long rounds = (blocks + slots - 1) / slots;
-      const double cost = (double)rounds * (g + 1);
-      if (cost < best - 1e-9) {
-        best = cost;
-        gps = g;
-      }
+    for (int g = g_lo + 1; g <= g_hi; ++g)
+      if (cost(g, 3) < cost(gps, 3) - 1e-9) gps = g;
+    if (d->head_dim <= 128 && d->n_q_heads <= 4 * d->n_kv_heads &&
+        !(d->value_bits == 4 && d->head_dim == 128 && d->n_q_heads > 2 * d->n_kv_heads)) {
+      for (int g = gps + 1; g <= g_hi; ++g)
+        if (cost(g, 4) < cost(gps, 4) - 1e-9) gps = g;
     }
   }
   pl.groups_per_split = gps;
