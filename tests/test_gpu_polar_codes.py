@@ -3,7 +3,8 @@ bit against the oracle's ordered sums (turboquant_pro/core.py:542-617): rows
 of zeros, of fp16 subnormals, of magnitudes whose squares vanish or overflow,
 of NaN, and rotations that put whole channels on a code boundary (identity on
 one-hot rows: more flagged codes than the list holds) or lie outside the
-estimate's bound (rows of length 100)."""
+estimate's bound (rows of length 100; rows of length 1e-6, whose fp16 halves
+are subnormal)."""
 
 import numpy as np
 import pytest
@@ -25,7 +26,7 @@ def _rotation(name, D):
     if name == "identity":
         return np.eye(D, dtype=np.float32), np.eye(D, dtype=np.float32)
     pi, pi_t = O.rotation(3, D)
-    f = np.float32(100.0 if name == "long" else 1.0)
+    f = np.float32({"long": 100.0, "short": 1e-6}.get(name, 1.0))
     return np.ascontiguousarray(pi * f), np.ascontiguousarray(pi_t * f)
 
 
@@ -51,7 +52,8 @@ def _rows(seed, H, L, D, f32):
     (128, 3, 512, "float16", "random"), (128, 3, 512, "float16", "identity"), (128, 2, 64, "float16", "long"),
     (128, 4, 130, "float16", "random"), (64, 3, 512, "float16", "random"), (256, 4, 512, "float16", "identity"),
     (256, 2, 37, "float16", "random"), (128, 3, 512, "float32", "random"), (64, 4, 64, "float32", "identity"),
-    (256, 3, 300, "float32", "random"), (128, 2, 33, "float32", "long")])
+    (256, 3, 300, "float32", "random"), (128, 2, 33, "float32", "long"),
+    (128, 3, 512, "float16", "short"), (64, 3, 512, "float32", "short")])
 def test_pool_codes_match_oracle(D, vb, W, dtype, rot):
     from turboquant_pro_amd import TQKVPool
     print(f"[polar codes] D={D} V{vb} W={W} {dtype} {rot}", flush=True)

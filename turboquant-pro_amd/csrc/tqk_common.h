@@ -246,8 +246,10 @@ constexpr float kPiScale = 256.0f;  // fp16 pairs of pi (and of u): far from fp1
 // The 16 * NT rows of pi from e0 on as MFMA operands (lane: row e0 + 16 nt +
 // lane % 16, channels 32 ks + 8 (lane / 16) .. + 7), and the bound on an
 // estimate's distance from the ordered sum: infinite (every code recomputed)
-// for rows that are not finite or longer than 50, and for boundaries that do
-// not ascend (the code's search needs them to).
+// for rows that are not finite, longer than 50 or shorter than 2^-8 (the fp16
+// pairs of a short row's channels are subnormal: they err by 2^-33 a channel,
+// sqrt(D) 2^-33 in all, however short the row is, while the bound shrinks with
+// it), and for boundaries that do not ascend (the code's search needs them to).
 template <int D, int NT>
 struct PiFrags {
   h8_t hi[D / 32][NT], lo[D / 32][NT];
@@ -278,7 +280,7 @@ __device__ __forceinline__ void load_pi(PiFrags<D, NT>& f, const float* __restri
     }
     ss += __shfl_xor(ss, 16, 64);
     ss += __shfl_xor(ss, 32, 64);
-    bad |= !(ss <= 2500.0f);
+    bad |= !(ss >= 0x1p-16f && ss <= 2500.0f);
     most = fmaxf(most, ss);
   }
 #pragma unroll
