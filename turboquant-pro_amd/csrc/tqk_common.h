@@ -219,9 +219,9 @@ __device__ __forceinline__ uint32_t stream_code(const uint32_t (&w)[VB], int i) 
 // the reference's y_e: the sum over d, in order, of u_d * pi[e][d], every
 // product and sum separately rounded (a NaN y_e takes the last code, as
 // searchsorted does).  Only the code is stored, so y_e itself is needed only
-// where it lies close to a boundary: the matrix cores give an estimate with a
-// proven error bound, every estimate further than the bound from all
-// boundaries has the reference's code, and the others (about 1 in 700 at 3
+// where it lies close to a boundary: the matrix cores give an estimate whose
+// error has a bound, every estimate further than the bound from all boundaries
+// has the reference's code, and the others (about 1 in 780 at 3
 // bits and head_dim 128) are listed and recomputed in the reference's order.
 // (Evaluating the ordered sum everywhere took 256 VALU instructions per channel
 // and bounded the whole encode: 16 sequences x 8192 tokens x 8 heads appended
@@ -229,19 +229,26 @@ __device__ __forceinline__ uint32_t stream_code(const uint32_t (&w)[VB], int i) 
 //
 // The estimate: x (fp16 as it is, or the fp32 row scaled to |u| <= 256 and
 // split into an fp16 pair) times 256 * pi split into an fp16 pair, summed in
-// fp32 by MFMA, scaled back by 1 / norm.  Against the real sum
-// sum_d u_d pi[e][d], with |u| <= 1 and N = |pi[e]|:
+// fp32 by MFMA, the products of low halves in an accumulator of their own
+// (among the high ones each of those MFMAs would truncate at full scale too:
+// twice the bound for fp16 rows and three times for fp32 ones), scaled back by
+// 1 / norm.  Against the real sum sum_d u_d pi[e][d], with |u| <= 1 and N =
+// |pi[e]| in [2^-8, 50]:
 //   the ordered sum errs by at most D 2^-24 N            (D roundings)
 //   the MFMA sums by at most (D / 32) 33 2^-23 N         (every one of a step's
 //                            32 products and its sum truncated at full scale)
+//   the low halves' sums, at most 2^-10 N, by as much of that in two such sums
+//   the addition of the two sums by 2^-24 N
 //   the dropped low x low products and the pairs' own rounding 3 2^-22 N, the
-//   scaling by 1 / norm 2^-22 N
-// which stays below D 2^-22 N for D = 64, 128 and 256.
+//   scaling by 1 / norm and u's own rounding 2^-22 N, low halves of pi below
+//   fp16's normal range sqrt(D) 2^-33
+// together below 0.86 D 2^-22 N for D = 64, 128 and 256.
 // ---------------------------------------------------------------------------
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 
 constexpr float kPiScale = 256.0f;  // fp16 pairs of pi (and of u): far from fp16's subnormals
+constexpr float kEstimateBound = 0.9f;  // on an estimate's distance from the ordered sum, in D 2^-22 N
 
 // The 16 * NT rows of pi from e0 on as MFMA operands (lane: row e0 + 16 nt +
 // lane % 16, channels 32 ks + 8 (lane / 16) .. + 7), and the bound on an
@@ -286,7 +293,7 @@ __device__ __forceinline__ void load_pi(PiFrags<D, NT>& f, const float* __restri
 #pragma unroll
   for (int o = 1; o < 16; o <<= 1) most = fmaxf(most, __shfl_xor(most, o, 64));
   for (int k = 1; k < nbnd; ++k) bad |= !(bnd[k - 1] < bnd[k]);
-  f.delta = __any(bad) ? __builtin_inff() : 1.01f * (float)D * 0x1p-22f * __builtin_sqrtf(most);
+  f.delta = __any(bad) ? __builtin_inff() : kEstimateBound * (float)D * 0x1p-22f * __builtin_sqrtf(most);
 }
 
 // #{ b < y } by binary search, and the distance m to the nearest boundary:
@@ -363,9 +370,9 @@ __device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFra
   const int c16 = lane & 15, lg = lane >> 4;
   for (int t0 = 0; t0 < nb; t0 += 16) {
     const uint16_t* row = xs + (size_t)min(t0 + c16, nb - 1) * stride + 8 * lg;
-    f4_t acc[NT];
+    f4_t acc[NT], low[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = low[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
       const h8_t xh = *reinterpret_cast<const h8_t*>(row + 32 * ks);
@@ -375,12 +382,12 @@ __device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFra
       for (int nt = 0; nt < NT; ++nt) {
         if constexpr (TROWS) {
           acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.hi[ks][nt], acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.lo[ks][nt], acc[nt], 0, 0, 0);
-          if constexpr (LO) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, pf.hi[ks][nt], acc[nt], 0, 0, 0);
+          low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.lo[ks][nt], low[nt], 0, 0, 0);
+          if constexpr (LO) low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, pf.hi[ks][nt], low[nt], 0, 0, 0);
         } else {
           acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xh, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.lo[ks][nt], xh, acc[nt], 0, 0, 0);
-          if constexpr (LO) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xl, acc[nt], 0, 0, 0);
+          low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.lo[ks][nt], xh, low[nt], 0, 0, 0);
+          if constexpr (LO) low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xl, low[nt], 0, 0, 0);
         }
       }
     }
@@ -395,7 +402,7 @@ __device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFra
       uint32_t near = 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float y = acc[nt][r] * tk[r].x;
+        const float y = (acc[nt][r] + low[nt][r]) * tk[r].x;
         float m;
         f |= code_margin<VB>(y, bnd, m) << (VB * r);
         near |= (m > tk[r].y * pf.delta) ? 0u : (1u << r);
