@@ -1,22 +1,26 @@
-"""The key-block encode's two outlier-threshold paths agree.
+"""The key-block encode over its routes: ``tqk_key_block_stats`` and what follows
+it over the chip, and ``tqk_key_block``, one workgroup per (batch, head), for
+blocks with outliers too small for what the former hand on through the packed
+output.  Both find the threshold of turboquant_pro/per_channel_kv.py:274-280
+(np.partition's k-th largest magnitude, every magnitude at or above it an
+entry).
 
-With ``outlier_cap`` of at least head_dim, ``tqk_encode_key_block`` finds the
-thresholds in ``tqk_key_block_thresholds`` (a lane per channel, waves over
-the tokens, two magnitude bits a pass) and hands them to ``tqk_key_block``
-through the side-list row; with a smaller cap ``tqk_key_block`` searches one
-bit a pass in one thread per channel.  Both find the threshold of
-turboquant_pro/per_channel_kv.py:274-280 (np.partition's k-th largest
-magnitude, every magnitude at or above it an entry).  The same block must
-give the same codes, scale, zero point and side-list count both ways, the
-small cap's entries being the first ones of the large cap's: fp16 and fp32
-input, asym-NF4 and uniform 4-bit keys, lognormal channel scales, magnitude
-ties at the threshold and a NaN.
+``test_threshold_paths_agree``: a side-list capacity below head_dim gives the
+same codes, scale, zero point and count as a large one, its entries being the
+first ones of the large one's: fp16 and fp32 input, asym-NF4 and uniform 4-bit
+keys, lognormal channel scales, magnitude ties at the threshold and a NaN.
+``test_routes_match_oracle``: both routes against the oracle on either side of
+the rule between them, at the edges of the 256-token chunks and 512-token
+tiles, with every element an outlier, with small capacities, and with input and
+packed output at addresses that are multiples of one element and one byte.
 """
 
 import ctypes
 
 import numpy as np
 import pytest
+
+from oracle import tq_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -65,8 +69,8 @@ def test_threshold_paths_agree(dtype, uniform, S):
     x[0, 1, 17, 9] = np.nan             # a NaN orders above every magnitude
     xt = torch.from_numpy(x).to(getattr(torch, dtype)).cuda()
     k = outliers_per_channel(S, 0.02)
-    big = _encode(xt, uniform, k, 4 * k * D)   # thresholds over the chip
-    small = _encode(xt, uniform, k, D // 2)    # one thread per channel
+    big = _encode(xt, uniform, k, 4 * k * D)
+    small = _encode(xt, uniform, k, D // 2)
     for name, a, b in zip(("codes", "scale", "zero", "count"), big[:4], small[:4]):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8)), name
     cnt = big[3]
@@ -76,3 +80,69 @@ def test_threshold_paths_agree(dtype, uniform, S):
         assert np.array_equal(big[4][i, :n], small[4][i, :n]), f"positions of (b, h) {i}"
         assert np.array_equal(big[5][i, :n].view(np.uint16), small[5][i, :n].view(np.uint16)), \
             f"values of (b, h) {i}"
+
+
+@pytest.mark.parametrize("D,bits,grid,S,frac,dtype,cap,x_off,p_off", [
+    # the rule: D + chunks + S D / 32 dwords in S D bits / 32 of them
+    (128, 2, "uniform", 32, 0.05, "float32", 0, 0, 0), (128, 2, "uniform", 33, 0.05, "float32", 0, 0, 0),
+    (128, 2, "uniform", 33, 0.05, "float16", 0, 1, 3), (64, 3, "uniform", 16, 0.1, "float16", 0, 0, 0),
+    (64, 3, "uniform", 17, 0.1, "float16", 0, 0, 0), (64, 3, "uniform", 18, 0.1, "float32", 0, 1, 1),
+    (256, 4, "nf4", 10, 0.1, "float32", 0, 0, 0), (256, 4, "nf4", 11, 0.1, "float32", 0, 0, 0),
+    (256, 4, "nf4", 11, 0.1, "float16", 0, 0, 2), (128, 4, "nf4", 1, 0.02, "float16", 0, 0, 0),
+    # chunks and tiles
+    (64, 4, "nf4", 256, 0.02, "float16", 0, 0, 0), (64, 4, "uniform", 257, 0.02, "float32", 0, 0, 0),
+    (128, 4, "nf4", 512, 0.02, "float32", 0, 0, 0), (128, 3, "uniform", 513, 0.02, "float16", 0, 0, 0),
+    (256, 4, "nf4", 513, 0.02, "float16", 0, 0, 0), (256, 2, "uniform", 512, 0.02, "float32", 0, 0, 0),
+    # every element an outlier, and none
+    (128, 4, "nf4", 9, 1.0, "float32", 0, 0, 0), (64, 4, "nf4", 300, 1.0, "float16", 0, 0, 0),
+    (128, 4, "nf4", 300, 0.0, "float32", 0, 1, 1), (256, 2, "uniform", 40, 0.0, "float16", 0, 1, 2),
+    # small capacities, odd addresses
+    (128, 4, "nf4", 700, 0.02, "float32", 5, 0, 0), (256, 4, "uniform", 300, 0.02, "float16", 100, 0, 0),
+    (128, 4, "nf4", 700, 0.02, "float32", 0, 1, 0), (64, 4, "nf4", 700, 0.02, "float16", 0, 3, 1),
+    (256, 4, "uniform", 300, 0.02, "float16", 0, 1, 0), (128, 4, "nf4", 300, 0.02, "float32", 0, 0, 2)])
+def test_routes_match_oracle(D, bits, grid, S, frac, dtype, cap, x_off, p_off):
+    from turboquant_pro_amd import _native as N
+    from turboquant_pro_amd.plugins import _block_desc
+    print(f"[key-block] routes D={D} bits={bits} {grid} S={S} frac={frac} {dtype} cap={cap} "
+          f"off={x_off},{p_off}", flush=True)
+    B, H, uniform = 1, 3, grid == "uniform"
+    rng = np.random.default_rng(S + D + bits)
+    x = rng.standard_normal((H, S, D)).astype(np.float32)
+    x *= np.exp(0.7 * rng.standard_normal((H, 1, D))).astype(np.float32)
+    x[0, :, 5] = np.float32(0.5) * np.sign(x[0, :, 5])   # ties, of both signs
+    x[1, :, 7] = 0.0
+    x = x.astype(dtype).astype(np.float32)
+    k = O.outlier_count_per_channel(S, frac) if frac else 0
+    want = O.encode_keys_uniform(x, frac, bits) if uniform else O.encode_keys(x, frac)
+    cap = cap or max(S * D, 1)
+    n = H * S * D
+    xt = torch.zeros(n + 8, dtype=getattr(torch, dtype), device="cuda")
+    xt[x_off:x_off + n] = torch.from_numpy(x.reshape(-1)).cuda().to(xt.dtype)
+    nb = n * bits // 8
+    kp = torch.full((nb + 16,), 0xA5, dtype=torch.uint8, device="cuda")
+    scale = torch.zeros((H, D), dtype=torch.float32, device="cuda")
+    zero = torch.zeros_like(scale)
+    count = torch.full((H,), -1, dtype=torch.int32, device="cuda")
+    pos = torch.full((H + 1, cap), -1, dtype=torch.int32, device="cuda")
+    val = torch.zeros((H + 1, cap), dtype=torch.float16, device="cuda")
+    d = _block_desc((B, H, S, D), bits, int(uniform), 0, k, cap, int(dtype == "float32"), None)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    N.check(N.lib().tqk_encode_key_block(
+        ctypes.byref(d), xt.data_ptr() + x_off * xt.element_size(), None, kp.data_ptr() + p_off, scale.data_ptr(),
+        zero.data_ptr(), pos.data_ptr(), val.data_ptr(), count.data_ptr(), st), "tqk_encode_key_block")
+    torch.cuda.synchronize()
+    got = kp.cpu().numpy()
+    assert np.array_equal(got[p_off:p_off + nb], want.packed)
+    assert np.all(got[:p_off] == 0xA5) and np.all(got[p_off + nb:] == 0xA5)
+    assert np.array_equal(scale.cpu().numpy(), want.nf4_scale)
+    assert np.array_equal(zero.cpu().numpy(), want.nf4_mean)
+    assert np.all(pos[H].cpu().numpy() == -1)
+    idx = np.zeros(0, np.int64) if want.outlier_idx is None else want.outlier_idx.astype(np.int64)
+    for h in range(H):
+        m = idx // (S * D) == h
+        assert int(count[h]) == int(m.sum())
+        e = min(int(m.sum()), cap)
+        assert np.array_equal(pos[h, :e].cpu().numpy(), (idx[m] - h * S * D)[:e])
+        assert np.all(pos[h, e:].cpu().numpy() == -1)
+        if e:
+            assert np.array_equal(val[h, :e].cpu().numpy().view(np.uint16), want.outlier_val[m][:e].view(np.uint16))

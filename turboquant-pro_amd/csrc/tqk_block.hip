@@ -118,8 +118,9 @@ struct KeyBlockArgs {
 // count), tqk_key_block_list (the same grid: the side-list, each chunk at the
 // offset that the counts before it give) and tqk_key_block_codes (the same
 // grid).  Until the codes are written, the (b, h)'s part of the packed output
-// holds what the first kernels hand on: D thresholds, n_chunks counts, and D
-// bits a token (KbScratch).  Bound: the stats kernel's ordered sum, 16000 tokens
+// holds what the first kernels hand on, from its first dword boundary: D
+// thresholds, n_chunks counts, and D bits a token (KbScratch).  Neither the
+// side-list's capacity nor the alignment of x and packed matters.  Bound: the stats kernel's ordered sum, 16000 tokens
 // one after another at about five cycles each, and its passes over the block.
 // One 1 x 8 x 16000 x 128 fp32 block: 3147 us with the thresholds on a workgroup
 // per 64 channels (16 passes) and statistics and side-list on one per (b, h),
@@ -136,7 +137,8 @@ struct KbScratch {
 };
 __device__ __forceinline__ KbScratch kb_scratch(const KeyBlockArgs& a, int bh) {
   const int D = a.d.head_dim;
-  uint32_t* base = reinterpret_cast<uint32_t*>(a.packed) + (size_t)bh * ((size_t)a.d.tokens * D * a.d.bits / 32);
+  uint8_t* p = a.packed + (size_t)bh * ((size_t)a.d.tokens * D * a.d.bits / 8);
+  uint32_t* base = reinterpret_cast<uint32_t*>(p + (-reinterpret_cast<uintptr_t>(p) & 3u));
   return {base, base + D, base + D + a.n_chunks};
 }
 
@@ -368,17 +370,17 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_list(KeyBlockArgs a) {
   const bool all = d.outliers_per_channel >= S;
   const KbScratch sc = kb_scratch(a, bh);
   const int s = c * kKbChunk + tid;
-  __shared__ int sum_s[2][kKbChunk / 64];
-  // entries in the chunks before this one, and in all of them
-  int before = 0, total = 0;
+  __shared__ uint32_t sum_s[2][kKbChunk / 64];
+  // entries in the chunks before this one, and in all of them (S * D < 2^32)
+  uint32_t before = 0, total = 0;
   if (all) {
-    before = c * kKbChunk * D;
-    total = S * D;
+    before = (uint32_t)c * kKbChunk * D;
+    total = (uint32_t)S * D;
   } else {
     for (int i = tid; i < a.n_chunks; i += kKbChunk) {
-      const int n = (int)sc.count[i];
+      const uint32_t n = sc.count[i];
       total += n;
-      before += i < c ? n : 0;
+      before += i < c ? n : 0u;
     }
     before = wave_sum(before);
     total = wave_sum(total);
@@ -391,28 +393,28 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_list(KeyBlockArgs a) {
     total = sum_s[1][0] + sum_s[1][1] + sum_s[1][2] + sum_s[1][3];
     __syncthreads();
   }
-  if (c == 0 && tid == 0) a.out_count[bh] = total;
+  if (c == 0 && tid == 0) a.out_count[bh] = (int32_t)total;
   uint32_t w[D / 32];
-  int cnt = 0;
+  uint32_t cnt = 0;
 #pragma unroll
   for (int k = 0; k < D / 32; ++k) {
     w[k] = s < S ? (all ? 0xFFFFFFFFu : sc.mask[(size_t)s * (D / 32) + k]) : 0u;
-    cnt += __builtin_popcount(w[k]);
+    cnt += (uint32_t)__builtin_popcount(w[k]);
   }
-  int incl = cnt;
+  uint32_t incl = cnt;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o, 64);
+    const uint32_t v = __shfl_up(incl, o, 64);
     if (lane >= o) incl += v;
   }
   if (lane == 63) sum_s[0][wv] = incl;
   __syncthreads();
-  int off = before + incl - cnt;
+  uint32_t off = before + incl - cnt;
   for (int i = 0; i < wv; ++i) off += sum_s[0][i];
   const size_t lb = (size_t)bh * d.outlier_cap, row = ((size_t)bh * S + s) * D;
 #pragma unroll
   for (int k = 0; k < D / 32; ++k) {
-    while (w[k] && off < d.outlier_cap) {
+    while (w[k] && off < (uint32_t)d.outlier_cap) {
       const int j = 32 * k + __builtin_ctz(w[k]);
       w[k] &= w[k] - 1u;
       a.out_pos[lb + off] = (uint32_t)s * D + (uint32_t)j;
@@ -447,8 +449,8 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) 
       const float r = __builtin_rintf(__fdiv_rn(__fsub_rn(xv, a.zero[(size_t)bh * D + j]), a.scale[(size_t)bh * D + j]));
       put_code_ref(rw, j, bits, (uint32_t)fminf(fmaxf(r, 0.0f), qmax));
     }
-    uint32_t* dst = reinterpret_cast<uint32_t*>(a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8));
-    for (int w = 0; w < D * bits / 32; ++w) dst[w] = rw[w];
+    uint8_t* dst = a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8);  // (at any byte)
+    for (int w = 0; w < D * bits / 32; ++w) __builtin_memcpy(dst + 4 * w, &rw[w], 4);
     return;
   }
   const int jp = tid % NPR, sq = tid / NPR;
@@ -463,12 +465,15 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) 
 #pragma unroll
       for (int u = 0; u < N; ++u) {
         const size_t i = base + (size_t)min(s + u, s1 - 1) * D + 2 * jp;
+        // (the pair may start at any element's boundary)
         if constexpr (F32) {
-          const float2 p = *reinterpret_cast<const float2*>(reinterpret_cast<const float*>(a.x) + i);
-          v0[u] = p.x;
-          v1[u] = p.y;
+          float p[2];
+          __builtin_memcpy(p, reinterpret_cast<const float*>(a.x) + i, sizeof(p));
+          v0[u] = p[0];
+          v1[u] = p[1];
         } else {
-          const uint32_t p = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const uint16_t*>(a.x) + i);
+          uint32_t p;
+          __builtin_memcpy(&p, reinterpret_cast<const uint16_t*>(a.x) + i, sizeof(p));
           v0[u] = h2f((uint16_t)p);
           v1[u] = h2f((uint16_t)(p >> 16));
         }
@@ -532,9 +537,8 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) 
   }
 }
 
-// The same in one workgroup of 2 * D threads per (b, h): side-list capacities
-// below head_dim, and blocks whose packed output cannot hold KbScratch (a few
-// tokens, or not at a multiple of four bytes).
+// The same in one workgroup of 2 * D threads per (b, h): blocks with outliers
+// whose packed output cannot hold KbScratch (a few tokens).
 template <int D>
 __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
   constexpr int T = 2 * D;  // threads
@@ -906,9 +910,8 @@ int check_block(const tqk_block_desc* d, bool key) {
 }
 
 // Key blocks go over the chip where the packed output has room for KbScratch
-// (dwords: 4-byte aligned) and the side-list could hold a row: 61 us at 1 x 8 x
-// 33 x 128 (fp32), 70 at 64 tokens, where one workgroup per (b, h) takes 104
-// and 277.
+// (with no outliers nothing is handed on): 61 us at 1 x 8 x 33 x 128 (fp32), 70
+// at 64 tokens, where one workgroup per (b, h) takes 104 and 277.
 template <int D, bool F32>
 void launch_key_chip(hipStream_t st, const KeyBlockArgs& a) {
   const unsigned bh = (unsigned)(a.d.batch * a.d.n_heads), n = bh * (unsigned)a.n_chunks;
@@ -923,13 +926,10 @@ void launch_key_chip(hipStream_t st, const KeyBlockArgs& a) {
 template <int D>
 void launch_key(hipStream_t st, const KeyBlockArgs& a) {
   const long long words = (long long)a.d.tokens * D * a.d.bits / 32;
-  const long long need = D + a.n_chunks + (long long)a.d.tokens * (D / 32);
-  const bool outliers = a.d.outliers_per_channel > 0;
-  const bool chip = (!outliers || (a.d.outlier_cap >= D && need <= words)) &&
-                    (reinterpret_cast<uintptr_t>(a.packed) & 3u) == 0u &&
-                    (reinterpret_cast<uintptr_t>(a.x) & 7u) == 0u &&
-                    (long long)a.d.batch * a.d.n_heads * a.n_chunks < (1LL << 31) &&
-                    (long long)a.d.tokens * D < (1LL << 31);
+  const long long pad = (reinterpret_cast<uintptr_t>(a.packed) & 3u) ? 1 : 0;  // to the first dword boundary
+  const long long need = pad + D + a.n_chunks + (long long)a.d.tokens * (D / 32);
+  const bool chip = (a.d.outliers_per_channel == 0 || need <= words) &&
+                    (long long)a.d.batch * a.d.n_heads * a.n_chunks < (1LL << 31);
   if (!chip)
     hipLaunchKernelGGL(tqk_key_block<D>, dim3(a.d.batch * a.d.n_heads), dim3(2 * D), 0, st, a);
   else if (a.d.input_f32)
