@@ -146,3 +146,38 @@ def test_routes_match_oracle(D, bits, grid, S, frac, dtype, cap, x_off, p_off):
         assert np.all(pos[h, e:].cpu().numpy() == -1)
         if e:
             assert np.array_equal(val[h, :e].cpu().numpy().view(np.uint16), want.outlier_val[m][:e].view(np.uint16))
+
+
+@pytest.mark.parametrize("D,frac", [(256, 0.0), (64, 0.3)])
+def test_more_heads_than_a_launch_takes(D, frac):
+    """262147 heads of head_dim 256 (and 1048579 of 64, with a side-list) would be more than
+    2^32 threads in one launch; the first and last of them and those around the cuts as in
+    blocks of their own."""
+    from turboquant_pro_amd import _native as N
+    from turboquant_pro_amd.plugins import _block_desc
+    cut, S = (1 << 21) // (D // 16), 1 if frac == 0.0 else 13
+    H, k = 2 * cut + 3, int(round(S * frac))
+    print(f"[key-block] {H} heads of {S} x {D}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(D)
+    x = torch.randn((H, S, D), generator=gen, device="cuda", dtype=torch.float16)
+
+    def encode(x):
+        n, cap = x.shape[0], 2 * D * max(k, 1)
+        kp = torch.zeros((n, S * D // 2), dtype=torch.uint8, device="cuda")
+        scale = torch.zeros((n, D), dtype=torch.float32, device="cuda")
+        zero = torch.zeros_like(scale)
+        count = torch.full((n,), -1, dtype=torch.int32, device="cuda")
+        pos = torch.zeros((n, cap), dtype=torch.int32, device="cuda")
+        val = torch.zeros((n, cap), dtype=torch.float16, device="cuda")
+        d = _block_desc((1, n, S, D), 4, 0, 0, k, cap, 0, None)
+        st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        N.check(N.lib().tqk_encode_key_block(
+            ctypes.byref(d), x.data_ptr(), None, kp.data_ptr(), scale.data_ptr(), zero.data_ptr(), pos.data_ptr(),
+            val.data_ptr(), count.data_ptr(), st), "tqk_encode_key_block")
+        return kp, scale, zero, count, pos, val
+
+    whole = encode(x)
+    for a, b in ((0, 2), (cut - 2, cut + 2), (2 * cut - 2, 2 * cut + 3)):
+        for got, want in zip(whole, encode(x[a:b].contiguous())):
+            assert torch.equal(got[a:b], want)
+    assert int(whole[3].min()) >= D * k

@@ -109,6 +109,7 @@ struct KeyBlockArgs {
   uint16_t* out_val;
   int32_t* out_count;
   int n_chunks;  // kKbChunk-token chunks of a (b, h)
+  int bh0;       // first (b, h) of the launch
 };
 
 // ---- key blocks over the chip -------------------------------------------------
@@ -162,7 +163,7 @@ template <int D, bool F32>
 __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockArgs a) {
   constexpr int NW = kKbStatThreads / 64, PER = kKbTile / (4 * NW);  // loads per thread and tile
   const tqk_block_desc& d = a.d;
-  const int bh = blockIdx.x / (D / 16), c0 = 16 * (blockIdx.x % (D / 16));
+  const int bh = a.bh0 + blockIdx.x / (D / 16), c0 = 16 * (blockIdx.x % (D / 16));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ch = lane & 15, sub = lane >> 4;
   const int S = d.tokens, kout = d.outliers_per_channel;
   const bool select = kout > 0 && kout < S, sum = d.key_grid == 0 && d.zero_point != 2;
@@ -324,7 +325,7 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
 template <int D, bool F32>
 __global__ __launch_bounds__(kKbChunk) void tqk_key_block_masks(KeyBlockArgs a) {
   constexpr int NC = D / 64, N = 16;
-  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int bh = a.bh0 + blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = a.d.tokens;
   const KbScratch sc = kb_scratch(a, bh);
   const int s0 = c * kKbChunk + 64 * wv, n = min(64, S - s0);
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_masks(KeyBlockArgs a) 
 template <int D, bool F32>
 __global__ __launch_bounds__(kKbChunk) void tqk_key_block_list(KeyBlockArgs a) {
   const tqk_block_desc& d = a.d;
-  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int bh = a.bh0 + blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = d.tokens;
   const bool all = d.outliers_per_channel >= S;
   const KbScratch sc = kb_scratch(a, bh);
@@ -435,7 +436,7 @@ template <int D, bool F32>
 __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) {
   constexpr int NPR = D / 2, NS = kKbChunk / NPR, PER = kKbChunk / NS;
   const tqk_block_desc& d = a.d;
-  const int bh = blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
+  const int bh = a.bh0 + blockIdx.x / a.n_chunks, c = blockIdx.x % a.n_chunks;
   const int tid = threadIdx.x, S = d.tokens;
   const size_t base = (size_t)bh * S * D;
   const int t0 = c * kKbChunk, t1 = min(S, t0 + kKbChunk);
@@ -912,24 +913,29 @@ int check_block(const tqk_block_desc* d, bool key) {
 // Key blocks go over the chip where the packed output has room for KbScratch
 // (with no outliers nothing is handed on): 61 us at 1 x 8 x 33 x 128 (fp32), 70
 // at 64 tokens, where one workgroup per (b, h) takes 104 and 277.
+// A launch takes fewer than 2^32 threads: as many (b, h) at a time as that allows
+// (131072 at head_dim 256).
 template <int D, bool F32>
-void launch_key_chip(hipStream_t st, const KeyBlockArgs& a) {
-  const unsigned bh = (unsigned)(a.d.batch * a.d.n_heads), n = bh * (unsigned)a.n_chunks;
-  hipLaunchKernelGGL((tqk_key_block_stats<D, F32>), dim3(bh * (D / 16)), dim3(kKbStatThreads), 0, st, a);
-  if (a.d.outliers_per_channel > 0) {
-    if (a.d.outliers_per_channel < a.d.tokens)
-      hipLaunchKernelGGL((tqk_key_block_masks<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
-    hipLaunchKernelGGL((tqk_key_block_list<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+void launch_key_chip(hipStream_t st, KeyBlockArgs a) {
+  const int n_bh = a.d.batch * a.d.n_heads;
+  const int most = min((1 << 21) / (D / 16), max(1, (1 << 23) / a.n_chunks));
+  for (; a.bh0 < n_bh; a.bh0 += most) {
+    const unsigned bh = (unsigned)min(most, n_bh - a.bh0), n = bh * (unsigned)a.n_chunks;
+    hipLaunchKernelGGL((tqk_key_block_stats<D, F32>), dim3(bh * (D / 16)), dim3(kKbStatThreads), 0, st, a);
+    if (a.d.outliers_per_channel > 0) {
+      if (a.d.outliers_per_channel < a.d.tokens)
+        hipLaunchKernelGGL((tqk_key_block_masks<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+      hipLaunchKernelGGL((tqk_key_block_list<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
+    }
+    hipLaunchKernelGGL((tqk_key_block_codes<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
   }
-  hipLaunchKernelGGL((tqk_key_block_codes<D, F32>), dim3(n), dim3(kKbChunk), 0, st, a);
 }
 template <int D>
 void launch_key(hipStream_t st, const KeyBlockArgs& a) {
   const long long words = (long long)a.d.tokens * D * a.d.bits / 32;
   const long long pad = (reinterpret_cast<uintptr_t>(a.packed) & 3u) ? 1 : 0;  // to the first dword boundary
   const long long need = pad + D + a.n_chunks + (long long)a.d.tokens * (D / 32);
-  const bool chip = (a.d.outliers_per_channel == 0 || need <= words) &&
-                    (long long)a.d.batch * a.d.n_heads * a.n_chunks < (1LL << 31);
+  const bool chip = a.d.outliers_per_channel == 0 || need <= words;
   if (!chip)
     hipLaunchKernelGGL(tqk_key_block<D>, dim3(a.d.batch * a.d.n_heads), dim3(2 * D), 0, st, a);
   else if (a.d.input_f32)
@@ -971,7 +977,7 @@ int tqk_encode_key_block(const tqk_block_desc* d, const void* x, const float* zp
   if (d->key_grid == 0 && d->zero_point == 2 && !zp) return TQK_EINVAL;
   if (d->outliers_per_channel > 0 && d->outlier_cap > 0 && (!out_pos || !out_val)) return TQK_EINVAL;
   const int n_chunks = (d->tokens + kKbChunk - 1) / kKbChunk;
-  KeyBlockArgs a{*d, x, zp, packed, scale, zero, out_pos, out_val, out_count, n_chunks};
+  KeyBlockArgs a{*d, x, zp, packed, scale, zero, out_pos, out_val, out_count, n_chunks, 0};
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (d->head_dim == 64)
     launch_key<64>(st, a);
