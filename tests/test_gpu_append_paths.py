@@ -64,3 +64,21 @@ def test_beyond_limits_refused():
                                        k.data_ptr(), k.data_ptr(), T, pool.seq_lens.data_ptr(), None, pool._stream())
         assert rc == N.TQK_EINVAL, (prev, n, batch)
     assert pool.seq_lens.tolist() == [0]
+
+
+def test_more_groups_than_a_launch_takes():
+    """65537 one-token groups of 64 heads would be more than 2^32 threads in one
+    launch: the same cache as in three appends."""
+    from turboquant_pro_amd import TQKVPool
+    H, D, L = 64, 64, 65538
+    print(f"[append paths] {L - 1} groups of {H} heads", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    k, v = (torch.randn((1, H, L, D), generator=gen, device="cuda", dtype=torch.float16) for _ in range(2))
+    pools = [TQKVPool(n_kv_heads=H, head_dim=D, max_batch=1, max_seq_len=L, hot_window=1, seed=0, outlier_frac=0.0)
+             for _ in range(2)]
+    pools[0].append(k, v)
+    for a, b in ((0, 30000), (30000, 60000), (60000, L)):
+        pools[1].append(k[:, :, a:b], v[:, :, a:b])
+    for name in ("seq_lens", "kcodes", "vcodes", "vnorm", "gscale", "gmean", "ocount", "hot_k", "hot_v"):
+        assert torch.equal(getattr(pools[0], name), getattr(pools[1], name)), name
+    assert int(torch.count_nonzero(pools[0].vnorm)) == H * (L - 1)

@@ -48,6 +48,7 @@ struct EncodeArgs {
   const void* chunk_v;
   int chunk_tokens;
   int n_items;
+  int unit0;  // first (item, kv head) of the launch, a multiple of 8
   int32_t* overflow;
   InlineItems in;
 };
@@ -176,7 +177,7 @@ __device__ __forceinline__ uint16_t nf4_threshold(float c0, float c1) {
 // over 16 levels, 624 us like this.
 template <int VB, int D>
 __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group(EncodeArgs a) {
-  const int unit = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
+  const int unit = a.unit0 + (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
   const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
   if (unit >= a.n_items * a.d.n_kv_heads) return;
   const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
@@ -751,7 +752,7 @@ __constant__ static const uint8_t kNf4Pair[32] = {0, 0, 0, 1,  1,  1,  1,  2,  2
 
 template <int VB, int D>
 __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group_f32(EncodeArgs a) {
-  const int unit = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
+  const int unit = a.unit0 + (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
   const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
   if (unit >= a.n_items * a.d.n_kv_heads) return;
   const int item = unit % a.n_items, h = unit / a.n_items, tid = threadIdx.x;
@@ -1366,24 +1367,29 @@ __global__ __launch_bounds__(kThreads, 2) void tqk_dequant_tokens(DequantArgs a)
   rotate_out(vo, nrm_s[1]);
 }
 
-// one kernel instance per (value bits, head_dim)
+// one kernel instance per (value bits, head_dim); a key and a value workgroup per
+// (item, kv head), see tqk_encode_group, as many as fewer than 2^32 threads allow
+// at a time
 template <int D>
-void launch_by_vb(int vb, dim3 grid, hipStream_t st, const EncodeArgs& a) {
-  // a key and a value workgroup per (item, kv head), see tqk_encode_group
-  const dim3 g2(16 * ((grid.x * grid.y + 7) / 8));
-  if (a.d.input_f32) {
-    if (vb == 2)
-      hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), g2, dim3(kEncThreads), 0, st, a);
-    else if (vb == 3)
-      hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), g2, dim3(kEncThreads), 0, st, a);
-    else
-      hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), g2, dim3(kEncThreads), 0, st, a);
-  } else if (vb == 2) {
-    hipLaunchKernelGGL((tqk_encode_group<2, D>), g2, dim3(kEncThreads), 0, st, a);
-  } else if (vb == 3) {
-    hipLaunchKernelGGL((tqk_encode_group<3, D>), g2, dim3(kEncThreads), 0, st, a);
-  } else {
-    hipLaunchKernelGGL((tqk_encode_group<4, D>), g2, dim3(kEncThreads), 0, st, a);
+void launch_by_vb(int vb, hipStream_t st, EncodeArgs a) {
+  constexpr int kMost = 1 << 21;
+  const int units = a.n_items * a.d.n_kv_heads;
+  for (; a.unit0 < units; a.unit0 += kMost) {
+    const dim3 grid(16 * ((min(kMost, units - a.unit0) + 7) / 8));
+    if (a.d.input_f32) {
+      if (vb == 2)
+        hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), grid, dim3(kEncThreads), 0, st, a);
+      else if (vb == 3)
+        hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), grid, dim3(kEncThreads), 0, st, a);
+      else
+        hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), grid, dim3(kEncThreads), 0, st, a);
+    } else if (vb == 2) {
+      hipLaunchKernelGGL((tqk_encode_group<2, D>), grid, dim3(kEncThreads), 0, st, a);
+    } else if (vb == 3) {
+      hipLaunchKernelGGL((tqk_encode_group<3, D>), grid, dim3(kEncThreads), 0, st, a);
+    } else {
+      hipLaunchKernelGGL((tqk_encode_group<4, D>), grid, dim3(kEncThreads), 0, st, a);
+    }
   }
 }
 template <int D, typename T>
@@ -1412,13 +1418,12 @@ int launch_encode(const EncodeArgs& a, void* stream) {
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (d.key_grid == 0 && d.zero_point == 2 && !a.p.zp_mean) return TQK_EINVAL;
   if (d.key_grid == 2 && !a.p.knorm) return TQK_EINVAL;
-  const dim3 grid(a.n_items, d.n_kv_heads);
   if (d.head_dim == 64)
-    launch_by_vb<64>(d.value_bits, grid, st, a);
+    launch_by_vb<64>(d.value_bits, st, a);
   else if (d.head_dim == 128)
-    launch_by_vb<128>(d.value_bits, grid, st, a);
+    launch_by_vb<128>(d.value_bits, st, a);
   else
-    launch_by_vb<256>(d.value_bits, grid, st, a);
+    launch_by_vb<256>(d.value_bits, st, a);
   return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
 }
 
