@@ -240,8 +240,9 @@ int tqk_append_hot(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t bat
  * as there, may be null), the surviving tokens copied into the ring
  * (tqk_append_hot), and seq_lens[b] (device) set to prev_len[b] + n_new[b].
  * prev_len and n_new are HOST arrays of `batch` entries, passed with the
- * launches (no copy to the device); n_new[b] in [0, chunk_tokens].  Beyond those
- * limits TQK_EINVAL, with nothing launched.  TurboQuantKVCache.append
+ * launches (no copy to the device); n_new[b] in [0, chunk_tokens], the new groups
+ * within max_groups_per_seq and max_pages_per_seq.  Beyond those limits
+ * TQK_EINVAL, with nothing launched.  TurboQuantKVCache.append
  * (turboquant_pro/core.py:986-1038).
  */
 int tqk_append_tokens(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t batch,

@@ -137,3 +137,31 @@ def test_noalloc_rejects_plans_beyond_its_scratch():
     assert rc == N.TQK_EWORKSPACE
     rc = lib.tqk_decode_noalloc(ctypes.byref(d), ctypes.byref(ptrs), 0, fake, fake, 100, fake, None)
     assert rc == N.TQK_EINVAL
+
+
+def test_append_tokens_refuses_lengths_past_the_tables():
+    """The lengths are on the host: an append whose groups would index past the
+    slot or page table, or whose length overflows, is refused before a launch."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("the refusals are told from launches by the missing device")
+    N, lib = _lib()
+    ints = ctypes.c_int32 * 2
+    buf = ctypes.create_string_buffer(64)
+    p = N.CachePtrs()
+
+    def rc(prev, n, **kw):
+        d = _desc(N, **kw)
+        return lib.tqk_append_tokens(ctypes.byref(d), ctypes.byref(p), 2, ints(0, prev), ints(0, n), buf, buf,
+                                     4096, buf, None, None)
+
+    full = 512 + 256 * 126   # 126 groups and a full hot window
+    assert rc(full - 1, 1) == N.TQK_EHIP          # (accepted: no device)
+    assert rc(full, 1) == N.TQK_EINVAL            # a 127th group: past both tables
+    assert rc(full, 1, max_groups_per_seq=127) == N.TQK_EINVAL
+    assert rc(full, 1, max_pages_per_seq=127) == N.TQK_EINVAL
+    assert rc(full, 1, max_groups_per_seq=127, max_pages_per_seq=127) == N.TQK_EHIP
+    assert rc(full, 1, max_groups_per_seq=127, page_tokens=64, max_pages_per_seq=507) == N.TQK_EINVAL
+    assert rc(2**31 - 1, 1) == N.TQK_EINVAL       # the new length is no int32
+    assert rc(2**31 - 4097, 4096, max_groups_per_seq=2**31 - 1, max_pages_per_seq=2**31 - 1) == N.TQK_EHIP
+    assert rc(full + 1, 1) == N.TQK_EHIP          # completes no group: the tables are not read

@@ -1499,8 +1499,14 @@ int tqk_append_tokens(const tqk_cache_desc* d, const tqk_cache_ptrs* p, int32_t 
     if (prev_len[b] < 0 || n_new[b] < 0 || n_new[b] > chunk_tokens) return TQK_EINVAL;
     e.in.prev[b] = a.in_prev[b] = prev_len[b];
     a.in_new[b] = n_new[b];
+    if (n_new[b] > INT32_MAX - prev_len[b]) return TQK_EINVAL;
     const int g1 = n_groups_of(prev_len[b] + n_new[b], d->hot_window, d->group_tokens);
-    for (int g = n_groups_of(prev_len[b], d->hot_window, d->group_tokens); g < g1; ++g) {
+    int g = n_groups_of(prev_len[b], d->hot_window, d->group_tokens);
+    // the new groups' slots and pages are in the tables
+    if (g < g1 && (g1 > d->max_groups_per_seq ||
+                   (long long)g1 * d->group_tokens > (long long)d->max_pages_per_seq * d->page_tokens))
+      return TQK_EINVAL;
+    for (; g < g1; ++g) {
       if (e.n_items == kInlineItems) return TQK_EINVAL;
       e.in.item[2 * e.n_items] = b;
       e.in.item[2 * e.n_items + 1] = g;
