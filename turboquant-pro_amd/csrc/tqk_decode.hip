@@ -2457,18 +2457,26 @@ Plan make_plan(const tqk_cache_desc* d, int batch, int max_len) {
     const long pairs = (long)batch * d->n_kv_heads;
     const int g_lo = units > 4096 ? (int)((units + 4095) / 4096) : 1;
     const int g_hi = ngmax > g_lo ? (8 * g_lo < ngmax ? 8 * g_lo : ngmax) : g_lo;
+    const long ncu = device_cus();  // (once: asking the runtime for the device in every cost was 2 us a decode)
     auto cost = [&](int g, int per_cu) {
-      const long blocks = pairs * ((ngmax + g - 1) / g + pl.n_hot_splits), slots = (long)per_cu * device_cus();
+      const long blocks = pairs * ((ngmax + g - 1) / g + pl.n_hot_splits), slots = per_cu * ncu;
       return (double)((blocks + slots - 1) / slots) * (g + 1);
     };
     gps = g_lo;
-    for (int g = g_lo + 1; g <= g_hi; ++g)
-      if (cost(g, 3) < cost(gps, 3) - 1e-9) gps = g;
+    auto raise_to_cheapest = [&](int per_cu) {
+      double best = cost(gps, per_cu);
+      for (int g = gps + 1; g <= g_hi; ++g) {
+        const double c = cost(g, per_cu);
+        if (c < best - 1e-9) {
+          best = c;
+          gps = g;
+        }
+      }
+    };
+    raise_to_cheapest(3);
     if (d->head_dim <= 128 && d->n_q_heads <= 4 * d->n_kv_heads &&
-        !(d->value_bits == 4 && d->head_dim == 128 && d->n_q_heads > 2 * d->n_kv_heads)) {
-      for (int g = gps + 1; g <= g_hi; ++g)
-        if (cost(g, 4) < cost(gps, 4) - 1e-9) gps = g;
-    }
+        !(d->value_bits == 4 && d->head_dim == 128 && d->n_q_heads > 2 * d->n_kv_heads))
+      raise_to_cheapest(4);
   }
   pl.groups_per_split = gps;
   pl.n_cold_splits = ngmax > 0 ? (ngmax + gps - 1) / gps : 0;
