@@ -308,7 +308,8 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
     kl_s[tid][0] = polar ? a.p.vcent[c0 & cm] : key_level(a.d.key_grid, c0);
     kl_s[tid][1] = polar ? a.p.vcent[c1 & cm] : key_level(a.d.key_grid, c1);
   }
-  if (tid < 16) lev_s[tid] = key_level(a.d.key_grid, tid);
+  const bool has_codes = f32 && d.outliers_per_channel > 0;  // the side-list's key codes are staged
+  if (has_codes && tid < 16) lev_s[tid] = key_level(a.d.key_grid, tid);
   // value pair table: field f of two channels' codes -> their two centroids
   if (tid < (1 << (2 * VB))) {
     vl_s[tid][0] = a.p.vcent[tid & ((1 << VB) - 1)];
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
       const bool oe_lds = !(GQ >= 8 && D >= 256) && n_oe <= kVOEnt;
       if (oe_lds)
         for (int e = tid; e < n_oe; e += kThreads) oe_s[e] = a.p.oent[obase * d.outlier_cap + e];
-      if (kAhead && f32) row_s[tid] = phys * P + (g * G + tid) % P;
+      if (kAhead && has_codes) row_s[tid] = phys * P + (g * G + tid) % P;
       if (tid < D) {
         const float av = a.p.gscale[mbase + tid];
         const float mv = a.p.gmean[mbase + tid];
@@ -397,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
         if constexpr (NW == 2) bias[i] = red_s[0][i] + red_s[1][i];
         if constexpr (NW == 4) bias[i] = (red_s[0][i] + red_s[1][i]) + (red_s[2][i] + red_s[3][i]);
       }
-      if (oe_lds && f32) {
+      if (oe_lds && has_codes) {
 #pragma unroll 4
         for (int e = tid; e < n_oe; e += kThreads) {
           const uint32_t pos = oe_s[e] & 0xFFFFu;
@@ -595,25 +596,29 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
       softmax_update<GQ>(sc_s, n, m_run, l_run, acc0, acc1, red_s, 1.0f);
       const int tend = min(n, tq * TS + TS);
       constexpr int kVUh = GQ >= 8 && D >= 256 ? 1 : 4;
+      // (a loop of its own per input type: with the choice inside, every
+      // token's load may be waited for before the next one is issued)
+      auto hot_values = [&](auto load) {
 #pragma unroll kVUh
-      for (int tt = tq * TS; tt < tend; ++tt) {
-        const size_t vrow = (hbase + (t0 + tt) % R) * D;
-        float c0, c1;
-        if (f32) {
-          const float2 two = reinterpret_cast<const float2*>(static_cast<const float*>(a.p.hot_v) + vrow)[jp];
-          c0 = two.x;
-          c1 = two.y;
-        } else {
-          const uint32_t two = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.p.hot_v) + vrow)[jp];
-          c0 = h2f((uint16_t)(two & 0xFFFFu));
-          c1 = h2f((uint16_t)(two >> 16));
-        }
+        for (int tt = tq * TS; tt < tend; ++tt) {
+          const float2 c = load((hbase + (t0 + tt) % R) * D);
 #pragma unroll
-        for (int i = 0; i < GQ; ++i) {
-          const float pp = sc_s[i][tt];
-          acc0[i] += pp * c0;
-          acc1[i] += pp * c1;
+          for (int i = 0; i < GQ; ++i) {
+            const float pp = sc_s[i][tt];
+            acc0[i] += pp * c.x;
+            acc1[i] += pp * c.y;
+          }
         }
+      };
+      if (f32) {
+        hot_values([&](size_t vrow) {
+          return reinterpret_cast<const float2*>(static_cast<const float*>(a.p.hot_v) + vrow)[jp];
+        });
+      } else {
+        hot_values([&](size_t vrow) {
+          const uint32_t two = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.p.hot_v) + vrow)[jp];
+          return make_float2(h2f((uint16_t)(two & 0xFFFFu)), h2f((uint16_t)(two >> 16)));
+        });
       }
     }
   }
