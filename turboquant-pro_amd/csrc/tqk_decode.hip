@@ -65,6 +65,9 @@ struct MergeArgs {
 constexpr int kThreads = 256;
 constexpr int kVOEnt = 2048;  // VALU decode: side-list entries staged in LDS per group
 
+// workgroups whose LDS a CU holds (160 KiB, given out in pieces of 1280 bytes)
+constexpr int lds_workgroups(size_t bytes) { return (int)(128 / ((bytes + 1279) / 1280)); }
+
 // The wave's sum or maximum in every lane, on the VALU (rotations inside the
 // 16-lane rows, then the two permlane swaps): a butterfly of ds_bpermute is six
 // LDS round trips in a row.
@@ -266,9 +269,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
   // code is a serial latency an entry (16 x 8192 tokens x 8 heads at head_dim
   // 256: 204 us, staged 177)
   __shared__ uint32_t oe_s[kVOEnt];
-  __shared__ uint8_t oc_s[kVOEnt];
   __shared__ float lev_s[16];
-  __shared__ int row_s[kThreads];  // row of every token of the group in the head's pages
   // the group's value code rows, staged by the token threads (one row each,
   // wide loads) for the value pass, whose threads walk the tokens of a slice
   // (not at 8 heads: the staging loads, live across the key loop, take all
@@ -288,6 +289,30 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
   __shared__ float accr_own[kOwnAcc ? NQ : 1][kOwnAcc ? GQ : 1][kOwnAcc ? D : 1];
   float (*accr_s)[GQ][D] = reinterpret_cast<float (*)[GQ][D]>(
       kOwnAcc ? static_cast<void*>(accr_own) : static_cast<void*>(vrow_s));
+
+  // an fp32 cache's key codes beside the side-list, and the rows of the group's
+  // tokens in the head's pages, which lead to them.  Where these 3 KiB would cost
+  // a CU a workgroup the codes take the place of the sums above (if those have
+  // one: written after the last group's walks) and the rows that of the first
+  // head's scores (written after the codes are staged): one head with 4-bit rows
+  // at head_dim 256, 16 x 12000 tokens x 4 heads in fp32, 220 us with two
+  // workgroups a CU, 138 with three.
+  constexpr size_t kRest = sizeof(q_s) + sizeof(qr_s) + sizeof(w2_s) + sizeof(oe_s) + sizeof(lev_s) + sizeof(vrow_s) +
+                           sizeof(sc_s) + sizeof(kl_s) + sizeof(vl_s) + sizeof(red_s) + sizeof(a_s) + sizeof(mu_s) +
+                           sizeof(accr_own) + 64;  // (64: the placeholders below, and alignment)
+  constexpr bool kShare = lds_workgroups(kRest + (kOwnAcc ? 0 : kVOEnt)) >
+                          lds_workgroups(kRest + kVOEnt + 4 * kThreads);
+  __shared__ uint8_t oc_own[kShare && kOwnAcc ? 1 : kVOEnt];
+  __shared__ int row_own[kShare ? 1 : kThreads];
+  uint8_t* oc_s = kShare && kOwnAcc ? reinterpret_cast<uint8_t*>(accr_own) : oc_own;
+  auto put_row = [&](int t, int row) {
+    if constexpr (kShare) sc_s[0][t] = __int_as_float(row);
+    else row_own[t] = row;
+  };
+  auto get_row = [&](int t) {
+    if constexpr (kShare) return __float_as_int(sc_s[0][t]);
+    else return row_own[t];
+  };
 
   // GQ is the kernel's power-of-two head count; the last GQ - gq heads are
   // zero-query padding whose states are never written
@@ -373,7 +398,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
       const bool oe_lds = !(GQ >= 8 && D >= 256) && n_oe <= kVOEnt;
       if (oe_lds)
         for (int e = tid; e < n_oe; e += kThreads) oe_s[e] = a.p.oent[obase * d.outlier_cap + e];
-      if (kAhead && has_codes) row_s[tid] = phys * P + (g * G + tid) % P;
+      if (kAhead && has_codes) put_row(tid, phys * P + (g * G + tid) % P);
       if (tid < D) {
         const float av = a.p.gscale[mbase + tid];
         const float mv = a.p.gmean[mbase + tid];
@@ -402,7 +427,7 @@ __global__ __launch_bounds__(kThreads) void tqk_decode_split_valu(DecodeArgs a) 
 #pragma unroll 4
         for (int e = tid; e < n_oe; e += kThreads) {
           const uint32_t pos = oe_s[e] & 0xFFFFu;
-          const uint8_t* kr = a.p.kcodes + ((size_t)h * d.n_pages * P + row_s[pos / D]) * k_row_bytes(d.key_bits, D);
+          const uint8_t* kr = a.p.kcodes + ((size_t)h * d.n_pages * P + get_row(pos / D)) * k_row_bytes(d.key_bits, D);
           oc_s[e] = (uint8_t)key_code(kr, d.key_bits, (int)(pos % D));
         }
       }
