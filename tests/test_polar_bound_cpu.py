@@ -22,21 +22,24 @@ def _bound():
     return float(m.group(1))
 
 
-def _mfmas(acc, lo):
-    """MFMAs into the accumulator per 32 channels and 16 x 16 tile (the same in the kernel's two branches)."""
+def _mfmas(lo):
+    """MFMAs per 32 channels and 16 x 16 tile: those of low halves, and after all of them those of high ones."""
     body = HEADER[HEADER.index("void polar_codes("):HEADER.index("void set_code(")]
-    lines = [x for x in body.splitlines() if acc + "[nt] = __builtin_amdgcn_mfma" in x]
-    only = sum("if constexpr (LO)" in x for x in lines)
-    return (len(lines) - (0 if lo else only)) // 2
+    loops = [x for x in re.split(r"for \(int ks = 0; ks < D / 32; \+\+ks\)", body)[1:]]
+    assert len(loops) == 2 and body.count("__builtin_amdgcn_mfma") == 2   # (one of the two operand orders)
+    first, second = loops[0], loops[1].split(";")[0]
+    low = first.count("add(row + 32 * ks, pf.lo[ks])") + lo * first.count("if constexpr (LO) add(row + D + 32 * ks, pf.hi[ks])")
+    assert first.count("add(") == 2 and second.strip() == "add(row + 32 * ks, pf.hi[ks])"
+    return low, 1
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("lo", [False, True], ids=["fp16", "fp32"])
 def test_bound_counts_every_mfma(D, lo):
-    assert (_mfmas("acc", lo), _mfmas("low", lo)) == ((1, 2) if lo else (1, 1))
+    low, high = _mfmas(lo)
+    assert (low, high) == ((2, 1) if lo else (1, 1))
     ordered = D * 2.0 ** -24
-    step = (D / 32) * 33 * 2.0 ** -23
-    mfma = step * (_mfmas("acc", lo) + 2.0 ** -10 * _mfmas("low", lo)) + 2.0 ** -24
+    mfma = (D / 32) * 33 * 2.0 ** -23 * (high + 2.0 ** -10 * low)
     rest = 3 * 2.0 ** -22 + 2.0 ** -22 + D ** 0.5 * 2.0 ** -33 / 2.0 ** -8
     assert ordered + mfma + rest <= 0.99 * _bound() * D * 2.0 ** -22   # 0.99: |u| and N themselves are rounded
 
@@ -69,14 +72,14 @@ def _worst(D, lo, length, seed=0):
     ph, pl = _pair((pi * f32(256)).astype(f32))
     s = (f32(256) * (f32(1) / nrm)).astype(f32)
     xh, xl = _pair((x * s).astype(f32)) if lo else (x.astype(f64), None)
-    acc, low = np.zeros((2, len(x), D))
-    for c in range(0, D, 32):
-        k = slice(c, c + 32)
-        acc = _mfma(acc, xh[:, k], ph[:, k])
-        low = _mfma(low, xh[:, k], pl[:, k])
+    acc = np.zeros((len(x), D))
+    steps = [slice(c, c + 32) for c in range(0, D, 32)]
+    for k in steps:
+        acc = _mfma(acc, xh[:, k], pl[:, k])
         if lo:
-            low = _mfma(low, xl[:, k], ph[:, k])
-    acc = (acc + low).astype(f32).astype(f64)
+            acc = _mfma(acc, xl[:, k], ph[:, k])
+    for k in steps:
+        acc = _mfma(acc, xh[:, k], ph[:, k])
     est = acc / 65536 if lo else acc * ((f32(1) / nrm) / f32(256)).astype(f64)
     N = np.sqrt((pi.astype(f64) ** 2).sum(axis=1))
     return float((np.abs(est - y) / (_bound() * D * 2.0 ** -22 * N)).max())

@@ -229,16 +229,14 @@ __device__ __forceinline__ uint32_t stream_code(const uint32_t (&w)[VB], int i) 
 //
 // The estimate: x (fp16 as it is, or the fp32 row scaled to |u| <= 256 and
 // split into an fp16 pair) times 256 * pi split into an fp16 pair, summed in
-// fp32 by MFMA, the products of low halves in an accumulator of their own
-// (among the high ones each of those MFMAs would truncate at full scale too:
-// twice the bound for fp16 rows and three times for fp32 ones), scaled back by
-// 1 / norm.  Against the real sum sum_d u_d pi[e][d], with |u| <= 1 and N =
+// fp32 by MFMA, all products of low halves before those of high ones (among
+// them each of those MFMAs would truncate at full scale too: twice the bound
+// for fp16 rows and three times for fp32 ones), scaled back by 1 / norm.  Against the real sum sum_d u_d pi[e][d], with |u| <= 1 and N =
 // |pi[e]| in [2^-8, 50]:
 //   the ordered sum errs by at most D 2^-24 N            (D roundings)
 //   the MFMA sums by at most (D / 32) 33 2^-23 N         (every one of a step's
 //                            32 products and its sum truncated at full scale)
-//   the low halves' sums, at most 2^-10 N, by as much of that in two such sums
-//   the addition of the two sums by 2^-24 N
+//   the low halves' sum before, at most 2^-10 N, by twice as much of that
 //   the dropped low x low products and the pairs' own rounding 3 2^-22 N, the
 //   scaling by 1 / norm and u's own rounding 2^-22 N, low halves of pi below
 //   fp16's normal range sqrt(D) 2^-33
@@ -370,27 +368,25 @@ __device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFra
   const int c16 = lane & 15, lg = lane >> 4;
   for (int t0 = 0; t0 < nb; t0 += 16) {
     const uint16_t* row = xs + (size_t)min(t0 + c16, nb - 1) * stride + 8 * lg;
-    f4_t acc[NT], low[NT];
+    f4_t acc[NT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = low[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    auto add = [&](const uint16_t* x, const h8_t (&p)[NT]) {
+      const h8_t xv = *reinterpret_cast<const h8_t*>(x);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+        acc[nt] = TROWS ? __builtin_amdgcn_mfma_f32_16x16x32_f16(xv, p[nt], acc[nt], 0, 0, 0)
+                        : __builtin_amdgcn_mfma_f32_16x16x32_f16(p[nt], xv, acc[nt], 0, 0, 0);
+    };
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
-      const h8_t xh = *reinterpret_cast<const h8_t*>(row + 32 * ks);
-      h8_t xl = {};
-      if constexpr (LO) xl = *reinterpret_cast<const h8_t*>(row + D + 32 * ks);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        if constexpr (TROWS) {
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.hi[ks][nt], acc[nt], 0, 0, 0);
-          low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, pf.lo[ks][nt], low[nt], 0, 0, 0);
-          if constexpr (LO) low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, pf.hi[ks][nt], low[nt], 0, 0, 0);
-        } else {
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xh, acc[nt], 0, 0, 0);
-          low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.lo[ks][nt], xh, low[nt], 0, 0, 0);
-          if constexpr (LO) low[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(pf.hi[ks][nt], xl, low[nt], 0, 0, 0);
-        }
-      }
+      add(row + 32 * ks, pf.lo[ks]);
+      if constexpr (LO) add(row + D + 32 * ks, pf.hi[ks]);
     }
+    // (the rows are read again: at head_dim 128 no registers are left to hold them)
+    if constexpr (D <= 128) asm volatile("" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) add(row + 32 * ks, pf.hi[ks]);
     // the lane's four results of a tile: tokens t0 + 4 lg + r of channel e0 +
     // 16 nt + c16 (TROWS), else channels e0 + 16 nt + 4 lg + r of token t0 + c16
     float2 tk[4];
@@ -402,7 +398,7 @@ __device__ __forceinline__ void polar_codes(PolarStage<D, NTOK>& st, const PiFra
       uint32_t near = 0;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float y = (acc[nt][r] + low[nt][r]) * tk[r].x;
+        const float y = acc[nt][r] * tk[r].x;
         float m;
         f |= code_margin<VB>(y, bnd, m) << (VB * r);
         near |= (m > tk[r].y * pf.delta) ? 0u : (1u << r);
