@@ -91,12 +91,15 @@ __device__ __forceinline__ void topk_insert(u16x2_t (&t)[K], u16x2_t v) {
 // with #{m >= T} >= k is exactly this k-th largest value (with multiplicity),
 // so it equals the bitwise threshold search's result.
 template <int K>
-__device__ __forceinline__ uint32_t kth_largest(const u16x2_t (&m)[TQK_MAX_G / 8], int k) {
+__device__ __forceinline__ uint32_t kth_largest(const u16x2_t (&m)[TQK_MAX_G / 8], int k, int G) {
   u16x2_t t[K];
 #pragma unroll
   for (int i = 0; i < K; ++i) t[i] = u16x2_t{0, 0};
 #pragma unroll
-  for (int i = 0; i < TQK_MAX_G / 8; ++i) topk_insert<K>(t, m[i]);
+  for (int i = 0; i < TQK_MAX_G / 8; ++i) {
+    if (i % 8 == 0 && 8 * i >= G) break;  // (the rest are no tokens)
+    topk_insert<K>(t, m[i]);
+  }
   {
     u16x2_t sw[K];
 #pragma unroll
@@ -272,7 +275,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
         // at a time, pairs past G repeat the last token
         auto for_quarter = [&](auto f) {
 #pragma unroll 1
-          for (int i0 = 0; i0 < TQK_MAX_G / 8; i0 += 8) {
+          for (int i0 = 0; 8 * i0 < G; i0 += 8) {
             uint16_t x[16];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
@@ -348,15 +351,17 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
 #pragma unroll
           for (int i = 0; i < TQK_MAX_G / 8; ++i) {
             const int s = 8 * i + 2 * part;  // tokens past G count as magnitude 0
-            m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
-                            (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
+            m2[i] = u16x2_t{0, 0};
+            if (8 * (i & ~7) < G)
+              m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
+                              (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
             if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // (the gathered halves are packed as they come)
           }
           uint32_t T = 0;
           if (kout <= 5) {
-            T = kth_largest<5>(m2, kout);
+            T = kth_largest<5>(m2, kout, G);
           } else if (kout <= 8) {
-            T = kth_largest<8>(m2, kout);
+            T = kth_largest<8>(m2, kout, G);
           } else {
             for (int bit = 14; bit >= 0; --bit) {
               const uint32_t cand = T | (1u << bit);
