@@ -22,10 +22,16 @@
 namespace {
 
 constexpr int kThreads = 256;
-// the group encodes: eight waves; its LDS (under 80 KiB at head_dim 128) lets
-// two workgroups share a CU, four waves per SIMD
-constexpr int kEncThreads = 512;
-constexpr int kEncWaves = kEncThreads / 64;
+// The group encodes by the largest group they take (MG tokens).  256: eight
+// waves; the LDS (under 80 KiB at head_dim 128) lets two workgroups share a CU,
+// four waves per SIMD.  64 (and 128, fp16 at head_dim 64): four waves and a
+// smaller key tile, so that four workgroups do: a short group is a chain of latencies, in which eight
+// waves wait no shorter than four.  8 sequences x 2000 tokens x 8 heads, NF4 keys
+// with a side-list, us by eight waves / by four: groups of 8 tokens at head_dim 64
+// 598 / 365, of 32 at 64 183 / 129, at 128 in fp32 300 / 265, at 256 850 / 502.
+constexpr int enc_threads(int MG) { return MG > 128 ? 512 : 256; }
+// tokens of a batch of PolarQuant rows: four threads each
+constexpr int enc_batch(int MG) { return enc_threads(MG) / 4; }
 
 // the order of stored codes, as PolarStage has it
 struct TokenRows { static constexpr bool value = false; };
@@ -90,14 +96,13 @@ __device__ __forceinline__ void topk_insert(u16x2_t (&t)[K], u16x2_t v) {
 // merged, then the lanes' lists over the two permlane swaps.  The largest T
 // with #{m >= T} >= k is exactly this k-th largest value (with multiplicity),
 // so it equals the bitwise threshold search's result.
-template <int K>
-__device__ __forceinline__ uint32_t kth_largest(const u16x2_t (&m)[TQK_MAX_G / 8], int k, int G) {
+template <int K, int N>
+__device__ __forceinline__ uint32_t kth_largest(const u16x2_t (&m)[N], int k, int G) {
   u16x2_t t[K];
 #pragma unroll
   for (int i = 0; i < K; ++i) t[i] = u16x2_t{0, 0};
 #pragma unroll
-  for (int i = 0; i < TQK_MAX_G / 8; ++i) {
-    if (i % 8 == 0 && 8 * i >= G) break;  // (the rest are no tokens)
+  for (int i = 0; i < N; ++i) {
     topk_insert<K>(t, m[i]);
   }
   {
@@ -178,8 +183,10 @@ __device__ __forceinline__ uint16_t nf4_threshold(float c0, float c1) {
 // sequences x 8192 tokens x 8 heads at head_dim 128, appended in 4096-token
 // chunks: 868 us with both sides in one 256-thread workgroup and the argmin
 // over 16 levels, 624 us like this.
-template <int VB, int D>
-__global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group(EncodeArgs a) {
+template <int VB, int D, int MG>
+__global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_group(EncodeArgs a) {
+  constexpr int kEncThreads = enc_threads(MG), kEncWaves = kEncThreads / 64, kVBatch = enc_batch(MG);
+  using Stage = PolarStage<D, kVBatch>;
   const int unit = a.unit0 + (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
   const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
   if (unit >= a.n_items * a.d.n_kv_heads) return;
@@ -197,7 +204,11 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   // take the key codes: the codes of token t overwrite the first D / 2 bytes of
   // row t once the wave that owns the row has read it (kc_row).  On the value
   // side the area holds the rows and stage of a value batch.
-  __shared__ __align__(16) uint16_t kt_s[TQK_MAX_G][D + 8];
+  constexpr size_t kBatchBytes = sizeof(uint16_t) * kVBatch * (D + 8);
+  constexpr size_t kTileBytes = sizeof(uint16_t) * MG * (D + 8);
+  static_assert(kBatchBytes % 16 == 0, "the stage follows the batch's rows");
+  __shared__ __align__(16) uint8_t area_s[kTileBytes > kBatchBytes + sizeof(Stage) ? kTileBytes : kBatchBytes + sizeof(Stage)];
+  uint16_t (*kt_s)[D + 8] = reinterpret_cast<uint16_t (*)[D + 8]>(area_s);
   __shared__ float stat_s[D][2];             // per channel: (mean, amax) or (min, scale)
   // per channel: 0x8000 - the fp16 magnitude threshold T (so m + it has bit 15
   // set exactly when m >= T; 0 for a NaN T), read eight channels at a time by
@@ -205,7 +216,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   __shared__ __align__(16) uint16_t tbias_s[D];
   // channels of each token stored in the side-list: in the tile rows' padding
   // where it fits
-  __shared__ uint32_t omx_s[D > 128 ? TQK_MAX_G : 1][D / 32];
+  __shared__ uint32_t omx_s[D > 128 ? MG : 1][D / 32];
   // per bucket and channel (of 64 channels): X | rev4(code) << 16 | rev4(code +
   // 1) << 20; row 32: the stored outliers' code.  Channel c at column (c >> 1) +
   // 32 (c & 1): the two half-waves read columns of different halves at a time,
@@ -347,14 +358,12 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
           }
         }
         if (kout > 0 && kout < G) {
-          u16x2_t m2[TQK_MAX_G / 8];
+          u16x2_t m2[MG / 8];
 #pragma unroll
-          for (int i = 0; i < TQK_MAX_G / 8; ++i) {
+          for (int i = 0; i < MG / 8; ++i) {
             const int s = 8 * i + 2 * part;  // tokens past G count as magnitude 0
-            m2[i] = u16x2_t{0, 0};
-            if (8 * (i & ~7) < G)
-              m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
-                              (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
+            m2[i] = u16x2_t{(uint16_t)(s < G ? abs_h(kt_s[s][j]) : 0u),
+                            (uint16_t)(s + 1 < G ? abs_h(kt_s[s + 1][j]) : 0u)};
             if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);  // (the gathered halves are packed as they come)
           }
           uint32_t T = 0;
@@ -370,7 +379,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
               const u16x2_t bv = {bias, bias};
               uint32_t acc = 0;  // two 16-bit counts
 #pragma unroll
-              for (int i = 0; i < TQK_MAX_G / 8; ++i)
+              for (int i = 0; i < MG / 8; ++i)
                 acc += (__builtin_bit_cast(uint32_t, (u16x2_t)(m2[i] + bv)) >> 15) & 0x00010001u;
               const int cnt = sum_quarters((int)((acc & 0xFFFFu) + (acc >> 16)));
               if (cnt >= kout) T = cand;
@@ -391,7 +400,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
     // stored (token, channel) positions, whose codes become the grid's zero
     // level below.
     if (kout > 0) {
-      static_assert(kEncThreads >= 2 * TQK_MAX_G, "two threads per token");
+      static_assert(kEncThreads >= 2 * MG, "two threads per token");
       const bool all = kout >= G;
       constexpr int NW = D / 64;  // mask words per thread
       const int tt = tid >> 1, w0 = NW * (tid & 1);
@@ -529,7 +538,7 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
             const uint32_t e = X | (rev4((uint32_t)k) << 16) | (rev4((uint32_t)k + 1u) << 20);
             for (int i = kNf4From[k]; i < kNf4From[k + 1]; ++i) nf_s[i][col] = e;
           }
-          if (wv == 7) nf_s[32][col] = rev4(7u) << 16 | rev4(7u) << 20;
+          if (wv == kEncWaves - 1) nf_s[32][col] = rev4(7u) << 16 | rev4(7u) << 20;
         }
         __syncthreads();
         // (a hair under 16: |x - mean| = amax stays short of bucket 32)
@@ -627,14 +636,11 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   // ---- values (and PolarQuant keys) ----------------------------------------
   // kVBatch tokens at a time: their rows staged in the key tile's area, norms
   // (four threads per token, the reference's pairwise order), estimated codes
-  // (wave w: channels [16 w, 16 w + 16), then 128 further on), the flagged ones recomputed, then the
-  // rows: LE bit streams of VB-bit codes per token, or 4-token x 8-channel
-  // units (the same eight fields a thread either way)
-  constexpr int VROW = D * VB / 8, NT = 1, kVBatch = 128;
-  using Stage = PolarStage<D, kVBatch>;
-  static_assert(kVBatch * (D + 8) * 2 % 16 == 0 &&
-                kVBatch * (D + 8) * 2 + sizeof(Stage) <= sizeof(kt_s), "value staging overflows the key tile");
-  Stage& st = *reinterpret_cast<Stage*>(&kt_s[kVBatch][0]);
+  // (wave w: channels [16 w, 16 w + 16), then as many waves further on), the
+  // flagged ones recomputed, then the rows: LE bit streams of VB-bit codes per
+  // token, or 4-token x 8-channel units (the same eight fields a thread either way)
+  constexpr int VROW = D * VB / 8, NT = 1;
+  Stage& st = *reinterpret_cast<Stage*>(area_s + kBatchBytes);
   float bnd[15];
 #pragma unroll
   for (int k = 0; k < 15; ++k) bnd[k] = k < (1 << VB) - 1 ? a.p.vbnd[k] : 0.f;
@@ -755,8 +761,10 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
 __constant__ static const uint8_t kNf4Pair[32] = {0, 0, 0, 1,  1,  1,  1,  2,  2,  3,  3,  4,  4,  5,  6,  6,
                                                   7, 8, 9, 9, 10, 11, 11, 12, 12, 13, 13, 14, 14, 14, 14, 14};
 
-template <int VB, int D>
-__global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_group_f32(EncodeArgs a) {
+template <int VB, int D, int MG>
+__global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_group_f32(EncodeArgs a) {
+  constexpr int kEncThreads = enc_threads(MG), kEncWaves = kEncThreads / 64;
+  constexpr int kVBatch = enc_batch(MG);  // tokens per value batch
   const int unit = a.unit0 + (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7u);
   const bool key_side = ((blockIdx.x >> 3) & 1u) == 0u;
   if (unit >= a.n_items * a.d.n_kv_heads) return;
@@ -769,13 +777,12 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
   const int kout = d.outliers_per_channel;
   const size_t mbase = ((size_t)slot * Hkv + h) * D;
   const size_t obase = (size_t)slot * Hkv + h;
-  constexpr int kVBatch = 128;  // tokens per value batch: four threads each
   constexpr int VROW = D * VB / 8;
   constexpr int LD = 68;        // key tile row stride: eight tokens x eight channels nearly on 64 banks
 
   struct KeyLds {
-    float tile[TQK_MAX_G][LD];      // 64 channels; then a row's 32 code bytes at its start
-    uint32_t om[TQK_MAX_G][D / 32]; // side-list bits of every token
+    float tile[MG][LD];      // 64 channels; then a row's 32 code bytes at its start
+    uint32_t om[MG][D / 32]; // side-list bits of every token
     float lev[16][64];              // NF4 levels of the channels, (channel / 2) + 32 (channel % 2)
     float stat[64][2];              // (mean, amax) or (min, scale)
     float thr[64];
@@ -836,8 +843,8 @@ __global__ __launch_bounds__(kEncThreads, D <= 128 ? 4 : 2) void tqk_encode_grou
       // as the largest fp32 magnitude pattern T with #{ |x_s| >= T } >= k (NaN
       // patterns order above inf, as np.partition places NaN last): for k <= 8
       // every lane's eight largest, merged; otherwise a bitwise search.
-      {
-        const int cl = 8 * wv + (lane & 7), part = lane >> 3;
+      for (int cw = 8 * wv; cw < 64; cw += 8 * kEncWaves) {
+        const int cl = cw + (lane & 7), part = lane >> 3;
         float mn = __builtin_inff(), mx = -__builtin_inff();
         uint32_t top[8];
 #pragma unroll
@@ -1372,30 +1379,44 @@ __global__ __launch_bounds__(kThreads, 2) void tqk_dequant_tokens(DequantArgs a)
   rotate_out(vo, nrm_s[1]);
 }
 
-// one kernel instance per (value bits, head_dim); a key and a value workgroup per
+// one kernel instance per (value bits, head_dim, group size); a key and a value workgroup per
 // (item, kv head), see tqk_encode_group, as many as fewer than 2^32 threads allow
 // at a time
-template <int D>
+template <int D, int MG>
 void launch_by_vb(int vb, hipStream_t st, EncodeArgs a) {
   constexpr int kMost = 1 << 21;
+  const dim3 threads(enc_threads(MG));
   const int units = a.n_items * a.d.n_kv_heads;
   for (; a.unit0 < units; a.unit0 += kMost) {
     const dim3 grid(16 * ((min(kMost, units - a.unit0) + 7) / 8));
     if (a.d.input_f32) {
-      if (vb == 2)
-        hipLaunchKernelGGL((tqk_encode_group_f32<2, D>), grid, dim3(kEncThreads), 0, st, a);
-      else if (vb == 3)
-        hipLaunchKernelGGL((tqk_encode_group_f32<3, D>), grid, dim3(kEncThreads), 0, st, a);
-      else
-        hipLaunchKernelGGL((tqk_encode_group_f32<4, D>), grid, dim3(kEncThreads), 0, st, a);
+      if constexpr (MG != 128) {
+        if (vb == 2)
+          hipLaunchKernelGGL((tqk_encode_group_f32<2, D, MG>), grid, threads, 0, st, a);
+        else if (vb == 3)
+          hipLaunchKernelGGL((tqk_encode_group_f32<3, D, MG>), grid, threads, 0, st, a);
+        else
+          hipLaunchKernelGGL((tqk_encode_group_f32<4, D, MG>), grid, threads, 0, st, a);
+      }
     } else if (vb == 2) {
-      hipLaunchKernelGGL((tqk_encode_group<2, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group<2, D, MG>), grid, threads, 0, st, a);
     } else if (vb == 3) {
-      hipLaunchKernelGGL((tqk_encode_group<3, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group<3, D, MG>), grid, threads, 0, st, a);
     } else {
-      hipLaunchKernelGGL((tqk_encode_group<4, D>), grid, dim3(kEncThreads), 0, st, a);
+      hipLaunchKernelGGL((tqk_encode_group<4, D, MG>), grid, threads, 0, st, a);
     }
   }
+}
+// the smallest instance that takes the groups (at 128 tokens only where its key
+// tile lets four workgroups share a CU: fp16 at head_dim 64)
+template <int D>
+void launch_by_group(hipStream_t st, const EncodeArgs& a) {
+  const int G = a.d.group_tokens;
+  if (G <= 64) return launch_by_vb<D, 64>(a.d.value_bits, st, a);
+  if constexpr (D == 64) {
+    if (G <= 128 && !a.d.input_f32) return launch_by_vb<D, 128>(a.d.value_bits, st, a);
+  }
+  launch_by_vb<D, TQK_MAX_G>(a.d.value_bits, st, a);
 }
 template <int D, typename T>
 void launch_dequant(int vb, dim3 grid, hipStream_t st, const DequantArgs& a) {
@@ -1424,11 +1445,11 @@ int launch_encode(const EncodeArgs& a, void* stream) {
   if (d.key_grid == 0 && d.zero_point == 2 && !a.p.zp_mean) return TQK_EINVAL;
   if (d.key_grid == 2 && !a.p.knorm) return TQK_EINVAL;
   if (d.head_dim == 64)
-    launch_by_vb<64>(d.value_bits, st, a);
+    launch_by_group<64>(st, a);
   else if (d.head_dim == 128)
-    launch_by_vb<128>(d.value_bits, st, a);
+    launch_by_group<128>(st, a);
   else
-    launch_by_vb<256>(d.value_bits, st, a);
+    launch_by_group<256>(st, a);
   return hipGetLastError() == hipSuccess ? TQK_OK : TQK_EHIP;
 }
 
