@@ -93,6 +93,10 @@ def test_threshold_paths_agree(dtype, uniform, S):
     (64, 4, "nf4", 256, 0.02, "float16", 0, 0, 0), (64, 4, "uniform", 257, 0.02, "float32", 0, 0, 0),
     (128, 4, "nf4", 512, 0.02, "float32", 0, 0, 0), (128, 3, "uniform", 513, 0.02, "float16", 0, 0, 0),
     (256, 4, "nf4", 513, 0.02, "float16", 0, 0, 0), (256, 2, "uniform", 512, 0.02, "float32", 0, 0, 0),
+    # up to 128 tokens the threshold by counting, up to 128 of a chunk codes by pieces
+    (128, 2, "uniform", 64, 0.1, "float32", 0, 0, 0), (64, 3, "uniform", 65, 0.1, "float16", 0, 0, 0),
+    (256, 3, "uniform", 128, 0.2, "float32", 0, 0, 1), (64, 2, "uniform", 129, 0.1, "float32", 0, 0, 0),
+    (128, 3, "uniform", 384, 0.02, "float16", 0, 1, 3), (256, 2, "uniform", 385, 0.02, "float32", 0, 0, 0),
     # every element an outlier, and none
     (128, 4, "nf4", 9, 1.0, "float32", 0, 0, 0), (64, 4, "nf4", 300, 1.0, "float16", 0, 0, 0),
     (128, 4, "nf4", 300, 0.0, "float32", 0, 1, 1), (256, 2, "uniform", 40, 0.0, "float16", 0, 1, 2),

@@ -158,7 +158,10 @@ __device__ __forceinline__ float kb_load(const void* x, size_t i) {
 // amax = max |x - mu| is taken at the channel's two ends: rounding is monotone.
 // Passes 2 .. 4 refine the threshold by 8, 8 and 7 bits: the largest magnitude
 // pattern T with #{ |x| >= T } >= k is the k-th largest, so each pass picks the
-// bin, counted from the top, in which the k-th falls.
+// bin, counted from the top, in which the k-th falls.  Up to 128 tokens a wave
+// counts for its channel, a lane two tokens, how many are above them instead
+// (clearing and scanning the histograms took most of such a block: 1 x 8 x 64 x
+// 128 fp32 at 2 bits 78 us, with the codes of short blocks over all threads 31).
 template <int D, bool F32>
 __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockArgs a) {
   constexpr int NW = kKbStatThreads / 64, PER = kKbTile / (4 * NW);  // loads per thread and tile
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
   const int bh = a.bh0 + blockIdx.x / (D / 16), c0 = 16 * (blockIdx.x % (D / 16));
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, ch = lane & 15, sub = lane >> 4;
   const int S = d.tokens, kout = d.outliers_per_channel;
-  const bool select = kout > 0 && kout < S, sum = d.key_grid == 0 && d.zero_point != 2;
+  const bool small = S <= 128, select = kout > 0 && kout < S, radix = select && !small, sum = d.key_grid == 0 && d.zero_point != 2;
   const size_t base = (size_t)bh * S * D + c0 + ch;
 
   __shared__ __align__(16) float tile_s[2][16][kKbLd];
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
     pre_s[tid] = 0u;
     rem_s[tid] = kout;
   }
-  if (select) clear();
+  if (radix) clear();
   __syncthreads();
 
   // ---- pass 1
@@ -231,8 +234,8 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
       mn = fminf(mn, x[u]);  // (tokens past the end repeat the last one)
       mx = fmaxf(mx, x[u]);
       top = max(top, m);
-      if (sum) tile_s[ti & 1][ch][s] = x[u];
-      if (select && t0 + s < S) atomicAdd(&hist_s[m >> 23][lane], 1u);
+      if (sum || small) tile_s[ti & 1][ch][s] = x[u];
+      if (radix && t0 + s < S) atomicAdd(&hist_s[m >> 23][lane], 1u);
     }
     __syncthreads();
     // (the other buffer is written next; this one only after the next barrier)
@@ -265,7 +268,28 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
     red_s[2][wv][ch] = __uint_as_float(top);
   }
   if (wv == 0 && sub == 0) mean_s[ch] = acc;
-  if (select) pick(23);
+  if (radix) pick(23);
+  if (select && small) {
+    uint32_t m[2];
+    int above[2] = {0, 0}, from[2] = {0, 0};  // tokens above the lane's, and not below it
+#pragma unroll
+    for (int u = 0; u < 2; ++u) m[u] = __float_as_uint(fabsf(tile_s[0][wv][lane + 64 * u]));
+    auto count = [&](uint32_t src, int n) {
+      for (int s = 0; s < n; ++s) {
+        const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)src, s);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          above[u] += v > m[u] ? 1 : 0;
+          from[u] += v >= m[u] ? 1 : 0;
+        }
+      }
+    };
+    count(m[0], min(S, 64));
+    count(m[1], S - 64);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (lane + 64 * u < S && above[u] < kout && kout <= from[u]) pre_s[wv] = m[u];  // (ties: the same value)
+  }
   __syncthreads();
   if (tid < 16) {
     for (int w = 0; w < NW; ++w) {
@@ -297,7 +321,7 @@ __global__ __launch_bounds__(kKbStatThreads) void tqk_key_block_stats(KeyBlockAr
   if (!select) return;
 
   // ---- passes 2 .. 4 (fp16 values have no bits below the third)
-  for (int lv = 1; lv < (F32 ? 4 : 3); ++lv) {
+  for (int lv = 1; radix && lv < (F32 ? 4 : 3); ++lv) {
     const int above = 31 - 8 * lv, shift = lv == 3 ? 0 : above - 8, mask = lv == 3 ? 127 : 255;
     __syncthreads();
     clear();
@@ -431,7 +455,7 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_list(KeyBlockArgs a) {
 // order as the real ones (gaps of at least 16 ulps of the largest distance, 2
 // (|mean| + amax)) make the first argmin the number of strict decreases from
 // level to level; the others take the comparison that also orders NaN.  2- and
-// 3-bit (uniform): one token row per thread.
+// 3-bit (uniform): a token row, or 32 channels of it, per thread.
 template <int D, bool F32>
 __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) {
   constexpr int NPR = D / 2, NS = kKbChunk / NPR, PER = kKbChunk / NS;
@@ -441,16 +465,30 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) 
   const size_t base = (size_t)bh * S * D;
   const int t0 = c * kKbChunk, t1 = min(S, t0 + kKbChunk);
   if (d.bits != 4) {
-    const int bits = d.bits, s = t0 + tid;
+    // a token row per thread, or for up to 128 tokens 32 channels of it (whole
+    // dwords), so that a short block's threads all have work
+    const int bits = d.bits;
     const float qmax = (float)((1 << bits) - 1);
+    auto code = [&](size_t i, size_t j) {
+      const float r = __builtin_rintf(__fdiv_rn(__fsub_rn(kb_load<F32>(a.x, i), a.zero[j]), a.scale[j]));
+      return (uint32_t)fminf(fmaxf(r, 0.0f), qmax);
+    };
+    if (t1 - t0 <= 128) {
+      for (int i = tid; i < (t1 - t0) * (D / 32); i += kKbChunk) {
+        const int s = t0 + i / (D / 32), c32 = i % (D / 32);
+        uint32_t rw[4] = {0u, 0u, 0u, 0u};
+        for (int j = 0; j < 32; ++j)
+          put_code_ref(rw, j, bits, code(base + (size_t)s * D + 32 * c32 + j, (size_t)bh * D + 32 * c32 + j));
+        uint8_t* dst = a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8) + 4 * bits * c32;  // (at any byte)
+        for (int w = 0; w < bits; ++w) __builtin_memcpy(dst + 4 * w, &rw[w], 4);
+      }
+      return;
+    }
+    const int s = t0 + tid;
     if (s >= S) return;
     uint32_t rw[D / 8] = {0u};
-    for (int j = 0; j < D; ++j) {
-      const float xv = kb_load<F32>(a.x, base + (size_t)s * D + j);
-      const float r = __builtin_rintf(__fdiv_rn(__fsub_rn(xv, a.zero[(size_t)bh * D + j]), a.scale[(size_t)bh * D + j]));
-      put_code_ref(rw, j, bits, (uint32_t)fminf(fmaxf(r, 0.0f), qmax));
-    }
-    uint8_t* dst = a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8);  // (at any byte)
+    for (int j = 0; j < D; ++j) put_code_ref(rw, j, bits, code(base + (size_t)s * D + j, (size_t)bh * D + j));
+    uint8_t* dst = a.packed + ((size_t)bh * S + s) * (size_t)(D * bits / 8);
     for (int w = 0; w < D * bits / 32; ++w) __builtin_memcpy(dst + 4 * w, &rw[w], 4);
     return;
   }
@@ -539,7 +577,9 @@ __global__ __launch_bounds__(kKbChunk) void tqk_key_block_codes(KeyBlockArgs a) 
 }
 
 // The same in one workgroup of 2 * D threads per (b, h): blocks with outliers
-// whose packed output cannot hold KbScratch (a few tokens).
+// whose packed output cannot hold KbScratch: S D bits / 32 dwords below D + 2 + S
+// D / 32, fewer than 34 tokens at 2 bits and head_dim 64.
+constexpr int kKbFew = 36;
 template <int D>
 __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
   constexpr int T = 2 * D;  // threads
@@ -598,11 +638,15 @@ __global__ __launch_bounds__(2 * D) void tqk_key_block(KeyBlockArgs a) {
     // k-th largest |x| as the largest fp32 magnitude pattern T with
     // #{ |x_s| >= T } >= k (NaN patterns order above inf, as np.partition does)
     const int j = tid - D;
+    uint32_t m[kKbFew];  // (no tokens: magnitude 0)
+#pragma unroll
+    for (int s = 0; s < kKbFew; ++s) m[s] = s < S ? __float_as_uint(fabsf(X(s, j))) : 0u;
     uint32_t T = 0;
     for (int bit = 30; bit >= 0; --bit) {
       const uint32_t cand = T | (1u << bit);
       int cnt = 0;
-      for (int s = 0; s < S; ++s) cnt += (__float_as_uint(fabsf(X(s, j))) >= cand);
+#pragma unroll
+      for (int s = 0; s < kKbFew; ++s) cnt += m[s] >= cand ? 1 : 0;
       if (cnt >= kout) T = cand;
     }
     thr_s[j] = __uint_as_float(T);
@@ -911,8 +955,8 @@ int check_block(const tqk_block_desc* d, bool key) {
 }
 
 // Key blocks go over the chip where the packed output has room for KbScratch
-// (with no outliers nothing is handed on): 61 us at 1 x 8 x 33 x 128 (fp32), 70
-// at 64 tokens, where one workgroup per (b, h) takes 104 and 277.
+// (with no outliers nothing is handed on): 1 x 8 x 33 x 128 fp32 at 2 bits takes
+// 27 us, at 4 bits 29; 16 tokens at 2 bits, in one workgroup per (b, h), 40.
 // A launch takes fewer than 2^32 threads: as many (b, h) at a time as that allows
 // (131072 at head_dim 256).
 template <int D, bool F32>
