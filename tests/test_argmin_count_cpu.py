@@ -1,8 +1,8 @@
-"""The group encode's counting argmin, restated in NumPy fp32 and checked
+"""The block encode's counting argmin (tqk_key_block_codes), restated in NumPy fp32 and checked
 against ``np.argmin`` (the reference's nearest-level rule,
 turboquant_pro/per_channel_kv.py:377-383): for sorted NF4 levels whose every
 gap is at least (|mean| + amax) * 2^-18 -- 16 ulps of the largest distance a
-token of the group can have -- the first argmin of |x - c_l| equals the
+token of the block can have -- the first argmin of |x - c_l| equals the
 number of strict decreases d_l < d_(l-1).  Inputs: random channels over many
 scales and offsets, tokens at the levels, at fp32 midpoints between them and
 at their neighbours, and channels that fail the gap test (for which the
@@ -42,7 +42,7 @@ def test_counting_argmin_equals_first_argmin():
             n_crowded += 1
             continue
         n_spread += 1
-        # tokens of the group: |x - mu| <= amax, as fp16 inputs in the encode
+        # tokens of the block: |x - mu| <= amax, as fp16 inputs in the encode
         x = (mu + amax * rng.uniform(-1, 1, 64)).astype(np.float16).astype(np.float32)
         x = x[np.abs(x - mu) <= amax]
         mids = ((c[:-1] + c[1:]) / np.float32(2.0)).astype(np.float32)

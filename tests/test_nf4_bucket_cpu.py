@@ -4,12 +4,17 @@ key names two neighbouring levels and one comparison with an fp16 threshold
 decides.  Every fp16 number of a channel's range is checked, for channels from
 centred ones to the largest offsets whose levels count as far enough apart."""
 
+import os
+import re
+
 import numpy as np
 import pytest
 
 from turboquant_pro_amd.formats import NF4
 
-FROM = [0, 3, 7, 9, 11, 13, 14, 16, 17, 18, 20, 21, 23, 25, 27, 32]  # first bucket of every level pair
+_SOURCE = open(os.path.join(os.path.dirname(__file__), "..", "turboquant-pro_amd", "csrc", "tqk_encode.hip")).read()
+# first bucket of every level pair: the kernels' table
+FROM = [int(x) for x in re.search(r"kNf4From\[16\] = \{([^}]*)\}", _SOURCE).group(1).split(",")]
 PAIR = np.repeat(np.arange(15), np.diff(FROM))
 f32 = np.float32
 
@@ -38,6 +43,10 @@ def _thresholds(c):
             assert up[np.argmax(up):].all()  # monotone: the kernel's search relies on it
             out[k] = x[np.argmax(up)]
     return out
+
+
+def test_table_covers_the_buckets():
+    assert len(FROM) == 16 and FROM[0] == 0 and FROM[15] == 32 and np.all(np.diff(FROM) > 0)
 
 
 def test_every_bucket_holds_at_most_its_own_midpoint():

@@ -1,5 +1,5 @@
 """The VALU decode's split plan, read from the workspace size: never more splits
-than a chip with three workgroups a CU gives, and fewer only where four fit."""
+than the model's three workgroups a CU give, and fewer only where it counts four."""
 
 import ctypes
 

@@ -2475,12 +2475,15 @@ Plan make_plan(const tqk_cache_desc* d, int batch, int max_len) {
   } else {
     // VALU kernel: a workgroup pays its set-up (query, code tables, the
     // split's partial, the merge's share) once for its gps groups, about a
-    // group's time, and three of its workgroups fit a CU.  Pick gps from the
-    // bound of at most 4096 coded workgroups (which bounds the partials) up to
-    // 8x that, minimising rounds of the CUs times (gps + 1), the hot splits'
-    // workgroups counted in the rounds.  Up to head_dim 128 and 4 heads four
-    // fit (LDS; not with 4-bit value rows at 128 and 4 heads): there a larger
-    // gps is taken if it costs less with four.  16 x 8192 tokens x 8 heads in
+    // group's time.  Pick gps from the bound of at most 4096 coded workgroups
+    // (which bounds the partials) up to 8x that, minimising rounds of the CUs
+    // times (gps + 1), the hot splits' workgroups counted in the rounds.  The
+    // model counts three workgroups a CU; by LDS and registers it is two at
+    // head_dim 256 with 4-bit rows from 2 heads on and with 3-bit ones at 4
+    // (four with 2-bit rows and 1 or 2 heads; one with 4-bit rows at 8), and
+    // four, at some sizes five, up to head_dim 128 and 4 heads (three with 4-bit
+    // rows at 128 and 4 heads): there a larger gps is taken if it costs less
+    // with four.  16 x 8192 tokens x 8 heads in
     // an fp32 cache, gps 3 / 5 / 8: 121 / 116 / 148 us.  A smaller one is not:
     // its set-ups cost more than the model says (32 x 8129 tokens x 2 heads at
     // head_dim 64, gps 3 / 1: 31 / 43 us).

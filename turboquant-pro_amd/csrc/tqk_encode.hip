@@ -148,7 +148,8 @@ __device__ __forceinline__ int sum_quarters(int x) {
 // With the normalised key t = (x - mean) / amax cut into 32 buckets of 1/16 on
 // [-1, 1], every bucket widened by 0.004 on both sides holds at most one
 // midpoint of two NF4 levels (they are at least 0.080 apart), so a bucket's
-// codes are kNf4Pair[bucket] or the next one, and one comparison of x decides:
+// codes are those of its pair k (kNf4From[k] <= bucket < kNf4From[k + 1]), k and
+// k + 1, and one comparison of x decides:
 // code = pair + (x >= X), X the smallest fp16 number that argmin puts on the
 // pair's upper level.  kNf4From[k] is the first bucket of pair k.
 __constant__ static const int kNf4From[16] = {0, 3, 7, 9, 11, 13, 14, 16, 17, 18, 20, 21, 23, 25, 27, 32};
@@ -179,10 +180,11 @@ __device__ __forceinline__ uint16_t nf4_threshold(float c0, float c1) {
 // workgroups, then the eight value workgroups of the same groups, so that
 // every XCD and CU gets both kinds and a flush of one group runs them side by
 // side.  What bounds it: the keys' VALU work and LDS traffic (statistics,
-// thresholds, side-list, codes: VALU 62 % busy at four waves per SIMD).  16
-// sequences x 8192 tokens x 8 heads at head_dim 128, appended in 4096-token
-// chunks: 868 us with both sides in one 256-thread workgroup and the argmin
-// over 16 levels, 624 us like this.
+// thresholds, side-list, codes): 32 sequences x 4096 tokens x 8 heads, NF4 keys
+// with a side-list, VALU 65 % busy at four waves per SIMD, LDS 22 %, a quarter of
+// that bank conflicts, matrix cores 5 %.  16 sequences x 8192 tokens x 8 heads at
+// head_dim 128, appended in 4096-token chunks: 868 us with both sides in one
+// 256-thread workgroup and the argmin over 16 levels, 629 us like this.
 template <int VB, int D, int MG>
 __global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_group(EncodeArgs a) {
   constexpr int kEncThreads = enc_threads(MG), kEncWaves = kEncThreads / 64, kVBatch = enc_batch(MG);
@@ -758,9 +760,6 @@ __global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_
 // weights in fp32.  4 sequences x 5000 tokens x 8 heads x 128: 607 us with one
 // 256-thread workgroup per (group, head) reading the keys through L1 and L2 in
 // every phase, 226 us like this.
-__constant__ static const uint8_t kNf4Pair[32] = {0, 0, 0, 1,  1,  1,  1,  2,  2,  3,  3,  4,  4,  5,  6,  6,
-                                                  7, 8, 9, 9, 10, 11, 11, 12, 12, 13, 13, 14, 14, 14, 14, 14};
-
 template <int VB, int D, int MG>
 __global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_group_f32(EncodeArgs a) {
   constexpr int kEncThreads = enc_threads(MG), kEncWaves = kEncThreads / 64;
@@ -805,7 +804,8 @@ __global__ __launch_bounds__(enc_threads(MG), D <= 128 ? 4 : 2) void tqk_encode_
     KeyLds& L = reinterpret_cast<Lds*>(lds_s)->k;
     const int kb = d.key_bits;
     const bool all = kout >= G;
-    if (tid < 32) L.pair[tid] = kNf4Pair[tid];
+    if (tid < 15)
+      for (int i = kNf4From[tid]; i < kNf4From[tid + 1]; ++i) L.pair[i] = (uint8_t)tid;
     for (int c0 = 0; c0 < D; c0 += 64) {
       // ---- 64 channels of the group's keys
       if (tid == 0) L.crowded = 0u;
